@@ -218,7 +218,11 @@ int nvk_paged_decode_noalloc(const void* q, int64_t q_stride_tok, int64_t q_stri
  *   the (sequence, query tile) pairs by their key count into the workspace
  *   and the attention kernel runs them longest first; without the workspace
  *   they run in grid order, with the same output bits.  Two calls in flight
- *   at once need two workspaces.
+ *   at once need two workspaces.  With a workspace of
+ *   nvk_varlen_prefill_parts_workspace_size() bytes (up to 36 MB; never less
+ *   than the former) longer query ranges whose tiles fill at most half of the
+ *   GPU, e.g. one prompt's chunk after a long prefix, are split as well where
+ *   that is faster.
  * scale must be > 0.  dtype: NVK_DTYPE_BF16 or NVK_DTYPE_F16 (q, k / v and
  * out alike; f32 accumulation either way).  head_dim: 128.  G: 1, 2, 4 or 8.
  */
@@ -243,6 +247,9 @@ int nvk_varlen_prefill(const void* q, int64_t q_stride_tok, int64_t q_stride_hea
 size_t nvk_varlen_prefill_workspace_size(int32_t batch, int32_t max_seqlen_q,
                                          int32_t max_seqlen_k, int32_t num_q_heads,
                                          int32_t num_kv_heads, int32_t head_dim);
+size_t nvk_varlen_prefill_parts_workspace_size(int32_t batch, int32_t max_seqlen_q,
+                                               int32_t max_seqlen_k, int32_t num_q_heads,
+                                               int32_t num_kv_heads, int32_t head_dim);
 
 /*
  * The longest-first order of a prefill's query tiles, ranked once for every

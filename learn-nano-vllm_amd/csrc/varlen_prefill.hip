@@ -81,11 +81,12 @@ struct PrefillArgs {
   int64_t out_stride_tok, out_stride_head;
   int out_rows16;  // out 16-byte aligned, strides multiples of 8: whole-row stores
   int n_qtiles;
-  // Split-K over key tiles (short query ranges over long contexts): blockIdx.z
-  // = qtile * n_splits + split, split j owning key tiles
-  // [j*tiles_per_split, (j+1)*tiles_per_split) (the last one: to the end).
-  // With n_splits > 1 every row's partial (O unnormalised, m, l) goes to `ws`
-  // and prefill_combine_kernel writes `out`.
+  // Split-K over key tiles (steps whose query tiles alone leave workgroup
+  // slots idle): blockIdx.z = qtile * n_splits + split.  A query tile's key
+  // tiles are cut evenly into as many parts as keep tiles_per_split tiles
+  // each (at most n_splits; split_range).  A tile with one part is finished by
+  // its workgroup; the parts of the others leave records in `ws` that
+  // prefill_combine_kernel merges into `out`.
   int n_splits, tiles_per_split;
   float* ws;
   // Longest-first order of the (sequence, query tile) pairs, pair = qt * batch
@@ -94,8 +95,13 @@ struct PrefillArgs {
   const int32_t* order;
 };
 
-constexpr int kRecFloats = HD + 4;  // partial record of one row: O[HD], m, l, pad
-constexpr int kMaxSplits = 16;      // key-range splits of one query tile
+// Partial record of one (query tile, part): the unnormalised O^T accumulators
+// as the lanes hold them, then m and l of each row.  Wave w's accumulator
+// quad j = 4 db + grp (4 floats per lane) sits at float (16 w + j) * 256 + 4
+// lane, so every store and load of a record moves 1 KiB of consecutive bytes.
+constexpr int kRecO = kRows * HD;
+constexpr int kRecFloats = kRows * (HD + 4);  // O, then m and l (and a pad of 2 per row)
+constexpr int kMaxSplits = 16;      // key-range parts of one query tile
 
 // ---- longest-first order of the query tiles ----------------------------------
 // The hardware starts workgroups in blockIdx order as slots free up.  Ranking
@@ -233,6 +239,25 @@ __device__ __forceinline__ QTile qtile_info(const PrefillArgs& a, int s, int qt,
   return t;
 }
 
+// The key tiles of part `split` of a query tile with n_tiles of them.
+struct SplitRange {
+  int n_live;        // parts that hold key tiles (1 when there is no key at all)
+  int begin, end;    // this part's tiles (empty for split >= n_live)
+};
+__device__ __forceinline__ SplitRange split_range(const PrefillArgs& a, int n_tiles, int split) {
+  SplitRange r{1, 0, n_tiles};
+  if (a.n_splits > 1) {
+    int n = (n_tiles + a.tiles_per_split - 1) / a.tiles_per_split;
+    n = n < a.n_splits ? n : a.n_splits;
+    n = n > 1 ? n : 1;
+    const int per = n_tiles > 0 ? (n_tiles + n - 1) / n : 1;
+    r.n_live = n_tiles > 0 ? (n_tiles + per - 1) / per : 1;
+    r.begin = split * per;
+    r.end = r.begin + per < n_tiles ? r.begin + per : n_tiles;
+  }
+  return r;
+}
+
 // Raw buffer descriptor over [b, b + bytes) for a byte address b (stride 0,
 // dword3 0x00020000 = 32-bit data format, the gfx9 setting for untyped buffer
 // access).
@@ -318,11 +343,9 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void varlen_prefill_kernel
   const int unmasked_keys = qi.unmasked_keys;
   const int n_tiles = (n_keys + kKeys - 1) / kKeys;
   // This workgroup's key tiles [t_begin, t_end).
-  const int t_begin = split * a.tiles_per_split;
-  const int t_end = split == a.n_splits - 1 ? n_tiles
-                    : (t_begin + a.tiles_per_split < n_tiles ? t_begin + a.tiles_per_split
-                                                             : n_tiles);
-  if (a.n_splits > 1 && t_begin >= t_end) return;  // the combine skips empty splits
+  const SplitRange sr = split_range(a, n_tiles, split);
+  if (split >= sr.n_live) return;
+  const int t_begin = sr.begin, t_end = sr.end;
 
   // LDS: K stages 0/1, then V stages 0/1 (64 KB).
   __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * kTileBytes];
@@ -912,28 +935,26 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void varlen_prefill_kernel
   }
 
   // ---- epilogue: normalise and store the rows ----------------------------------
-  if (a.n_splits > 1) {  // partial record: O^T column (unnormalised), m_ref, l
+  const float l_tot = nvk_sum_xor32(l_part[0] + l_part[1]);
+  if (sr.n_live > 1) {  // partial record (O unnormalised, m_ref, l)
     if (!row_valid) return;
-    const float l_tot = nvk_sum_xor32(l_part[0] + l_part[1]);
     float* rec = a.ws + ((((int64_t)s * a.num_kv_heads + kvh) * a.n_qtiles + qt) * a.n_splits +
-                         split) * (int64_t)kRows * kRecFloats +
-                 (int64_t)row * kRecFloats;
+                         split) * (int64_t)kRecFloats;
 #pragma unroll
     for (int db = 0; db < HD / 32; ++db) {
 #pragma unroll
       for (int grp = 0; grp < 4; ++grp) {
         const nvk_f32x4 o4 = {acc_o[db][4 * grp], acc_o[db][4 * grp + 1], acc_o[db][4 * grp + 2],
                               acc_o[db][4 * grp + 3]};
-        *reinterpret_cast<nvk_f32x4*>(rec + 32 * db + 8 * grp + 4 * half) = o4;
+        *reinterpret_cast<nvk_f32x4*>(rec + (16 * wave + 4 * db + grp) * 256 + 4 * lane) = o4;
       }
     }
     if (half == 0) {
-      rec[HD] = m_ref;
-      rec[HD + 1] = l_tot;
+      rec[kRecO + 2 * row] = m_ref;
+      rec[kRecO + 2 * row + 1] = l_tot;
     }
     return;
   }
-  const float l_tot = nvk_sum_xor32(l_part[0] + l_part[1]);
   const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
   // Lane (half, l32) holds d = 32 db + 8 grp + 4 half .. +3 of its row.
   auto packed = [&](int db, int grp) {
@@ -985,35 +1006,36 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void varlen_prefill_kernel
   }
 }
 
-// Merges the split-K partial records of one (sequence, kv head, query tile):
-// thread t handles row t/8 and d range 16*(t%8) .. +15.  The m of every live
-// split is fetched in one round trip, then the splits are folded in order,
-// kFoldBatch at a time with all their loads in flight (left to itself the
-// compiler waits for each split's m in turn and keeps four of a split's
-// loads in flight).
+// Merges the partial records of one wave's 32 rows of a (sequence, kv head,
+// query tile) that was cut into parts; one workgroup of 4 waves, grid x =
+// kv head * kWaves + wave.  Wave u folds accumulator quads 4u..4u+3 of every
+// row, reading the records as the attention kernel's lanes wrote them (1 KiB
+// per load); the rows' m and l of every part are fetched in one round trip,
+// then the parts are folded in order, kFoldBatch at a time with all their
+// loads in flight.  The normalised rows go through LDS so that each store
+// writes whole 256-byte rows.
 constexpr int kFoldBatch = 4;
 template <int G, int MODE, bool F16>
-__global__ __launch_bounds__(8 * kRows) void prefill_combine_kernel(PrefillArgs a) {
+__global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a) {
   constexpr int TQ = kRows / G;
-  const int kvh = blockIdx.x, s = blockIdx.y, qt = blockIdx.z;
+  using E = NvkElt<F16>;
+  const int kvh = blockIdx.x / kWaves, w = blockIdx.x % kWaves, s = blockIdx.y, qt = blockIdx.z;
   const QTile qi = qtile_info<MODE>(a, s, qt, TQ);
   if (!qi.live) return;
-  const int r = threadIdx.x >> 3, dq = threadIdx.x & 7;
-  const int tok = qi.q0 + r / G;
-  if (tok < 0 || tok >= qi.Lq) return;
-  const int head = kvh * G + r % G;
-  const int n_tiles = (qi.n_keys + kKeys - 1) / kKeys;
-  // splits that own at least one tile (the others wrote nothing)
-  int n_live = a.tiles_per_split > 0 ? (n_tiles + a.tiles_per_split - 1) / a.tiles_per_split : 0;
-  if (n_live > a.n_splits) n_live = a.n_splits;
+  const int n_live = split_range(a, (qi.n_keys + kKeys - 1) / kKeys, 0).n_live;
+  if (n_live <= 1) return;  // finished by its workgroup
+  const int tok0 = qi.q0 + w * (32 / G);  // first token of the wave's rows
+  if (tok0 + 32 / G <= 0 || tok0 >= qi.Lq) return;  // no row of the wave holds a query
+  const int lane = threadIdx.x & 63, u = threadIdx.x >> 6;
+  const int l32 = lane & 31, half = lane >> 5;
   const float* rec0 = a.ws + (((int64_t)s * a.num_kv_heads + kvh) * a.n_qtiles + qt) *
-                                 a.n_splits * (int64_t)kRows * kRecFloats +
-                      (int64_t)r * kRecFloats;
-  const int64_t split_stride = (int64_t)kRows * kRecFloats;
+                                 a.n_splits * (int64_t)kRecFloats;
+  const float* ml0 = rec0 + kRecO + 2 * (32 * w + l32);
+  const float* o0 = rec0 + (16 * w + 4 * u) * 256 + 4 * lane;
   float mv[kMaxSplits];
 #pragma unroll
   for (int j = 0; j < kMaxSplits; ++j) {
-    const float m = rec0[(j < n_live ? j : 0) * split_stride + HD];
+    const float m = ml0[(j < n_live ? j : 0) * (int64_t)kRecFloats];
     mv[j] = j < n_live ? m : -INFINITY;
   }
   float M = -INFINITY;
@@ -1029,33 +1051,51 @@ __global__ __launch_bounds__(8 * kRows) void prefill_combine_kernel(PrefillArgs 
     float lv[kFoldBatch];
     nvk_f32x4 ov[kFoldBatch][4];
 #pragma unroll
-    for (int u = 0; u < kFoldBatch; ++u) {
-      const int j = j0 + u < n_live ? j0 + u : j0;  // past the last live split: reread j0, weight 0
-      const float* rec = rec0 + j * split_stride;
-      lv[u] = rec[HD + 1];
+    for (int v = 0; v < kFoldBatch; ++v) {
+      const int64_t j = j0 + v < n_live ? j0 + v : j0;  // past the last part: reread j0, unused
+      lv[v] = ml0[j * kRecFloats + 1];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) ov[u][i] = *reinterpret_cast<const nvk_f32x4*>(rec + 16 * dq + 4 * i);
+      for (int i = 0; i < 4; ++i)
+        ov[v][i] = *reinterpret_cast<const nvk_f32x4*>(o0 + j * kRecFloats + 256 * i);
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = 0; u < kFoldBatch; ++u) {
-      if (j0 + u >= n_live) break;
-      const float m = mv[j0 + u];
-      const float w = m == -INFINITY ? 0.f : nvk_fast_exp2(m - M);
-      L += w * lv[u];
+    for (int v = 0; v < kFoldBatch; ++v) {
+      if (j0 + v >= n_live) break;
+      const float m = mv[j0 + v];
+      const float wt = m == -INFINITY ? 0.f : nvk_fast_exp2(m - M);
+      L += wt * lv[v];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[i] += w * ov[u][i];
+      for (int i = 0; i < 4; ++i) acc[i] += wt * ov[v][i];
     }
   }
   const float inv = L > 0.f ? 1.f / L : 0.f;
-  uint16_t* op = a.out + ((int64_t)qi.q_row0 + tok) * a.out_stride_tok +
-                 (int64_t)head * a.out_stride_head + 16 * dq;
+  // quad 4u + i of a lane: d = 32 u + 8 i + 4 half .. +3 of its row
+  __shared__ __attribute__((aligned(16))) uint8_t rows[32 * HD * 2];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {  // 8-byte stores: out is only required 8-byte aligned
-    nvk_u32x2 w;
-    w.x = NvkElt<F16>::pack2(acc[i][0] * inv, acc[i][1] * inv);
-    w.y = NvkElt<F16>::pack2(acc[i][2] * inv, acc[i][3] * inv);
-    *reinterpret_cast<nvk_u32x2*>(op + 4 * i) = w;
+  for (int i = 0; i < 4; ++i) {
+    nvk_u32x2 p;
+    p.x = E::pack2(acc[i][0] * inv, acc[i][1] * inv);
+    p.y = E::pack2(acc[i][2] * inv, acc[i][3] * inv);
+    // 16-byte chunk c of row r at chunk c ^ (r & 15), as in the attention kernel
+    const int c = (4 * u + i) ^ (l32 & 15);
+    *reinterpret_cast<nvk_u32x2*>(rows + l32 * HD * 2 + 16 * c + 8 * half) = p;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int p = 0; p < 2; ++p) {
+    const int r = 16 * p + (threadIdx.x >> 4), c = threadIdx.x & 15;
+    const nvk_u32x4 v = *reinterpret_cast<const nvk_u32x4*>(rows + r * HD * 2 + 16 * (c ^ (r & 15)));
+    const int rt = tok0 + r / G;
+    if (rt < 0 || rt >= qi.Lq) continue;
+    uint16_t* op = a.out + ((int64_t)qi.q_row0 + rt) * a.out_stride_tok +
+                   (int64_t)(kvh * G + r % G) * a.out_stride_head + 8 * c;
+    if (a.out_rows16) {
+      *reinterpret_cast<nvk_u32x4*>(op) = v;
+    } else {  // out is only 8-byte aligned
+      *reinterpret_cast<nvk_u32x2*>(op) = nvk_u32x2{v.x, v.y};
+      *reinterpret_cast<nvk_u32x2*>(op + 4) = nvk_u32x2{v.z, v.w};
+    }
   }
 }
 
@@ -1067,9 +1107,8 @@ int launch_mode(const PrefillArgs& a, hipStream_t stream) {
   if (a.n_splits > 1) {
     const int st = nvk_launch_status();
     if (st != NVK_OK) return st;
-    dim3 cgrid(a.num_kv_heads, a.batch, a.n_qtiles);
-    hipLaunchKernelGGL((prefill_combine_kernel<G, MODE, F16>), cgrid, dim3(8 * kRows), 0, stream,
-                       a);
+    dim3 cgrid(a.num_kv_heads * kWaves, a.batch, a.n_qtiles);
+    hipLaunchKernelGGL((prefill_combine_kernel<G, MODE, F16>), cgrid, dim3(256), 0, stream, a);
   }
   return nvk_launch_status();
 }
@@ -1095,14 +1134,14 @@ int launch_prefill_g(const PrefillArgs& a, int G, hipStream_t s) {
 }
 
 
-// Split-K plan for a launch: split the key range when the query ranges are
-// short (at most half a query tile, so partial records stay small next to the
-// keys they summarise) and the query tiles alone give fewer than ~4
-// workgroups per CU, keeping at least 8 key tiles (512 keys) per split.
-// Deterministic in its arguments, so the workspace query and the launch agree.
+// Split-K plan for a launch.  Deterministic in its arguments, so the workspace
+// queries and the launch agree.
 struct SplitPlan {
   int n_qtiles, n_splits, tiles_per_split;
 };
+// Short query ranges (at most half a query tile, so that partial records stay
+// small next to the keys they summarise) whose query tiles alone give fewer
+// than ~4 workgroups per CU, keeping at least 8 key tiles (512 keys) per part.
 static SplitPlan plan_splits(int batch, int max_seqlen_q, int64_t max_keys, int num_q_heads,
                              int num_kv_heads) {
   SplitPlan p;
@@ -1124,25 +1163,77 @@ static SplitPlan plan_splits(int batch, int max_seqlen_q, int64_t max_keys, int 
   p.tiles_per_split = (int)((max_tiles + p.n_splits - 1) / p.n_splits);
   return p;
 }
+// Longer query ranges whose tiles fill at most half of the 512 workgroup slots
+// (256 CUs x 2), e.g. one prompt's chunk after a long prefix: without parts
+// the step takes as long as its longest tile while most CUs idle.  The number
+// of parts minimises the time of the longest part, in us, with constants
+// fitted to 60 shapes (1-8 sequences of 40-4096 new tokens after 0-16000
+// cached, 16/8, 16/2 and 4/2 heads) timed at 1 to 16 parts:
+//   no parts: 4 + tiles * r(wgs); with parts: 8.5 + 0.022 wgs' + tiles / n * r(wgs'),
+//   wgs' = wgs * n, where a key tile takes r = 1.07 us alone on its CU (1.14 us
+//   at 256 workgroups, which do not all get a CU of their own) and up to
+//   1.81 us when 512 workgroups share the CUs, and the records of a
+//   workgroup cost 0.022 us to write and merge.
+// Measured without / with parts: 1000 new after 8000 (128 workgroups, 4
+// parts) 154.7 / 82.4 us, 400 after 16000 (56, 8) 277 / 71.5 us, 100 after
+// 1000 (16, 5) 22.3 / 14.5 us, 2048 after 8000 (256, 2) 182 / 159 us.  Where
+// parts lose the rule gives none: 777 new tokens alone (104) 18.0 / 18.9 us,
+// 2048 alone (256) 35.6 / 37.9 us, 500 x 4 after 2000 (256) 54.6 / 55.3 us;
+// from 376 workgroups up no count gained more than 6 %.
+static SplitPlan plan_parts(int batch, int max_seqlen_q, int64_t max_keys, int num_q_heads,
+                            int num_kv_heads) {
+  SplitPlan p = plan_splits(batch, max_seqlen_q, max_keys, num_q_heads, num_kv_heads);
+  const int TQ = kRows / (num_q_heads / num_kv_heads);
+  const int64_t wgs = (int64_t)num_kv_heads * batch * p.n_qtiles;
+  const int64_t tiles = (max_keys + kKeys - 1) / kKeys;
+  constexpr int64_t kSlots = 512;
+  if (2 * (int64_t)max_seqlen_q <= TQ || wgs <= 0 || 2 * wgs > kSlots) return p;
+  auto tile_us = [](int64_t w) {
+    if (w <= 192) return 1.07f;
+    return w <= 256 ? 1.07f + 0.0011f * (float)(w - 192) : 1.35f + 0.0018f * (float)(w - 256);
+  };
+  const float whole = 4.f + (float)tiles * tile_us(wgs);
+  float best = 0.96f * whole;  // parts have to gain something over the fit's error
+  int best_n = 1;
+  for (int n = 2; n <= kMaxSplits && wgs * n <= kSlots && 2 * n <= tiles; ++n) {
+    const float per = (float)((tiles + n - 1) / n);
+    const float t = 8.5f + 0.022f * (float)(wgs * n) + per * tile_us(wgs * n);
+    if (t < best) {
+      best = t;
+      best_n = n;
+    }
+  }
+  if (best_n > 1) {
+    p.n_splits = best_n;
+    p.tiles_per_split = (int)((tiles + best_n - 1) / best_n);
+  }
+  return p;
+}
 static size_t split_workspace_bytes(const SplitPlan& p, int batch, int num_kv_heads) {
   if (p.n_splits <= 1) return 0;
-  return (size_t)num_kv_heads * batch * p.n_qtiles * p.n_splits * kRows * kRecFloats *
-         sizeof(float);
+  return (size_t)num_kv_heads * batch * p.n_qtiles * p.n_splits * kRecFloats * sizeof(float);
 }
 
 }  // namespace
 
-extern "C" size_t nvk_varlen_prefill_workspace_size(int32_t batch, int32_t max_seqlen_q,
-                                                    int32_t max_seqlen_k, int32_t num_q_heads,
-                                                    int32_t num_kv_heads, int32_t head_dim) {
+namespace {
+
+size_t prefill_workspace_bytes(bool parts, int32_t batch, int32_t max_seqlen_q,
+                               int32_t max_seqlen_k, int32_t num_q_heads, int32_t num_kv_heads,
+                               int32_t head_dim) {
   if (batch <= 0 || max_seqlen_q <= 0 || max_seqlen_k <= 0 || num_q_heads <= 0 ||
       num_kv_heads <= 0 || head_dim != HD || num_q_heads % num_kv_heads)
     return 0;
   const int G = num_q_heads / num_kv_heads;
   if (G != 1 && G != 2 && G != 4 && G != 8) return 0;
-  const size_t split = split_workspace_bytes(
-      plan_splits(batch, max_seqlen_q, max_seqlen_k, num_q_heads, num_kv_heads), batch,
-      num_kv_heads);
+  const SplitPlan pl = plan_splits(batch, max_seqlen_q, max_seqlen_k, num_q_heads, num_kv_heads);
+  size_t split = split_workspace_bytes(pl, batch, num_kv_heads);
+  if (parts) {
+    const size_t n = split_workspace_bytes(
+        plan_parts(batch, max_seqlen_q, max_seqlen_k, num_q_heads, num_kv_heads), batch,
+        num_kv_heads);
+    split = n > split ? n : split;
+  }
   // short query ranges over paged keys take the short-query kernels (pages of
   // a multiple of 64 keys; the size does not depend on the page size)
   const size_t sq = short_query_applies(true, 64, max_seqlen_q, num_q_heads, num_kv_heads,
@@ -1150,11 +1241,28 @@ extern "C" size_t nvk_varlen_prefill_workspace_size(int32_t batch, int32_t max_s
                         ? short_query_ws_bytes(batch, max_seqlen_k, num_q_heads, num_kv_heads)
                         : 0;
   // room for the longest-first tile order (multi-sequence prefills)
-  const SplitPlan pl = plan_splits(batch, max_seqlen_q, max_seqlen_k, num_q_heads, num_kv_heads);
   const int64_t pairs = (int64_t)batch * pl.n_qtiles;
   const size_t ord = use_order(batch, pairs, num_kv_heads) ? order_bytes(pairs) : 0;
   size_t need = split > sq ? split : sq;
   return ord > need ? ord : need;
+}
+
+}  // namespace
+
+extern "C" size_t nvk_varlen_prefill_workspace_size(int32_t batch, int32_t max_seqlen_q,
+                                                    int32_t max_seqlen_k, int32_t num_q_heads,
+                                                    int32_t num_kv_heads, int32_t head_dim) {
+  return prefill_workspace_bytes(false, batch, max_seqlen_q, max_seqlen_k, num_q_heads,
+                                 num_kv_heads, head_dim);
+}
+
+extern "C" size_t nvk_varlen_prefill_parts_workspace_size(int32_t batch, int32_t max_seqlen_q,
+                                                          int32_t max_seqlen_k,
+                                                          int32_t num_q_heads,
+                                                          int32_t num_kv_heads,
+                                                          int32_t head_dim) {
+  return prefill_workspace_bytes(true, batch, max_seqlen_q, max_seqlen_k, num_q_heads,
+                                 num_kv_heads, head_dim);
 }
 
 namespace {
@@ -1251,6 +1359,11 @@ int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_he
   }
   SplitPlan sp = plan_splits(batch, max_seqlen_q, max_keys, num_q_heads, num_kv_heads);
   if (sp.n_qtiles > 65535) return NVK_EINVAL;
+  const SplitPlan parts =
+      plan_parts(batch, max_seqlen_q, max_keys, num_q_heads, num_kv_heads);
+  if (parts.n_splits > 1 && workspace &&
+      workspace_bytes >= split_workspace_bytes(parts, batch, num_kv_heads))
+    sp = parts;
   if (sp.n_splits > 1 && (!workspace || workspace_bytes < split_workspace_bytes(sp, batch,
                                                                                 num_kv_heads))) {
     sp.n_splits = 1;  // no room for partials: one workgroup per query tile

@@ -50,6 +50,8 @@ SIGNATURES = {
                                           _c_ptr, ctypes.c_size_t, _c_i32, _c_ptr]),
     "nvk_varlen_prefill_workspace_size": (ctypes.c_size_t,
                                           [_c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32]),
+    "nvk_varlen_prefill_parts_workspace_size": (ctypes.c_size_t,
+                                                [_c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32]),
     "nvk_prefill_tile_order_size": (ctypes.c_size_t, [_c_i32, _c_i32, _c_i32, _c_i32, _c_i32,
                                                       _c_i32]),
     "nvk_prefill_tile_order": (ctypes.c_int, [_c_ptr, _c_ptr, _c_i32, _c_i32, _c_i32, _c_i32,

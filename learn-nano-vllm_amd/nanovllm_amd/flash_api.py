@@ -119,7 +119,7 @@ def varlen_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, softmax_sc
     lib = _lib.load()
     key_bound = max_blocks * block_size if bt is not None else total_k
     msk = min(int(max_seqlen_k), key_bound) if max_seqlen_k else key_bound
-    ws_bytes = lib.nvk_varlen_prefill_workspace_size(batch, int(max_seqlen_q), msk, hq, hkv, d)
+    ws_bytes = lib.nvk_varlen_prefill_parts_workspace_size(batch, int(max_seqlen_q), msk, hq, hkv, d)
     ws = _lib.workspace(dev, ws_bytes)
     order_bytes = 0
     if order is not None:
