@@ -35,6 +35,11 @@
 // non-temporal (read once).  The page of a chunk comes through a scalar load
 // when a page holds whole chunks.
 //
+// Steps with 4 or more query heads per kv head (or one, from 33 sequences up)
+// run on the MFMA kernels of short_query.hip instead (short_query.h has the
+// rule and both sides' times): the dot products and the softmax bookkeeping
+// here cost VALU time per query head.
+//
 // Finishing: a group that ends inside a wave's range is normalised in
 // registers and written as bf16.  A group cut between waves leaves one
 // partial (o, m, l) record per wave and head; every wave also writes the
@@ -48,6 +53,7 @@
 
 #include "nvk_common.h"
 #include "qk_math.h"
+#include "short_query.h"
 
 namespace {
 
@@ -786,10 +792,14 @@ size_t decode_ws_bytes(int batch, int num_q_heads, int num_kv_heads, int head_di
 template <int HD, int G, bool FUSED, bool F16>
 int launch_decode(const DecodeArgs& a, bool aligned, hipStream_t stream) {
   const dim3 grid(a.n_waves / kWavesPerWG);
-  if (aligned)
-    hipLaunchKernelGGL((paged_decode_kernel<HD, G, true, FUSED, F16>), grid, dim3(256), 0, stream,
-                       a);
-  else
+  // HD 128 with 4 or 8 heads per kv head and pages of whole chunks: the
+  // short-query kernels' (an empty pool, num_blocks 0, takes the general form)
+  constexpr bool kWholePages = FUSED || HD != 128 || G <= kDecodeKernelGroup;
+  if constexpr (kWholePages)
+    if (aligned)
+      hipLaunchKernelGGL((paged_decode_kernel<HD, G, true, FUSED, F16>), grid, dim3(256), 0,
+                         stream, a);
+  if (!kWholePages || !aligned)
     hipLaunchKernelGGL((paged_decode_kernel<HD, G, false, FUSED, F16>), grid, dim3(256), 0,
                        stream, a);
   int st = nvk_launch_status();
@@ -881,8 +891,36 @@ int decode_setup(const void* q, int64_t q_stride_tok, int64_t q_stride_head, con
   return NVK_OK;
 }
 
+// The decode on the short-query MFMA kernels.
+int decode_short_query(const DecodeArgs& a, float scale, void* workspace, hipStream_t s) {
+  ShortQueryParams p{};
+  p.q = a.q;
+  p.q_stride_tok = a.q_stride_tok;
+  p.q_stride_head = a.q_stride_head;
+  p.k_cache = a.k_cache;
+  p.v_cache = a.v_cache;
+  p.context_lens = a.context_lens;
+  p.batch = a.batch;
+  p.block_tables = a.block_tables;
+  p.bt_stride = a.bt_stride;
+  p.max_blocks = a.max_blocks;
+  p.block_size = a.block_size;
+  p.num_blocks = a.num_blocks;
+  p.num_q_heads = a.num_q_heads;
+  p.num_kv_heads = a.num_kv_heads;
+  p.scale = scale;
+  p.out = a.out;
+  p.out_stride_tok = a.out_stride_tok;
+  p.out_stride_head = a.out_stride_head;
+  p.f16 = a.f16;
+  return short_query_launch(p, (int64_t)a.block_size * a.max_blocks, workspace, s);
+}
+
 // Points the descriptors and records of `a` into `workspace` and launches.
-int decode_run(DecodeArgs& a, int head_dim, void* workspace, hipStream_t s) {
+int decode_run(DecodeArgs& a, int head_dim, float scale, void* workspace, hipStream_t s) {
+  if (short_query_decode_applies(a.block_size, a.num_blocks, a.num_q_heads, a.num_kv_heads,
+                                 head_dim, a.batch))
+    return decode_short_query(a, scale, workspace, s);
   const size_t desc = ((size_t)a.batch * (a.num_kv_heads / a.hpi) * 8 + 255) / 256 * 256;
   a.ws_desc = static_cast<int32_t*>(workspace);
   a.ws_rec = reinterpret_cast<float*>(static_cast<char*>(workspace) + desc);
@@ -969,7 +1007,7 @@ extern "C" int nvk_paged_decode(const void* q, int64_t q_stride_tok, int64_t q_s
   if (st != NVK_OK || batch == 0) return st;
   if (workspace == nullptr || workspace_bytes < need) return NVK_EWORKSPACE;
   if ((uintptr_t)workspace % 256) return NVK_EALIGN;
-  return decode_run(a, head_dim, workspace, reinterpret_cast<hipStream_t>(stream));
+  return decode_run(a, head_dim, scale, workspace, reinterpret_cast<hipStream_t>(stream));
 }
 
 extern "C" int nvk_paged_decode_noalloc(const void* q, int64_t q_stride_tok,
@@ -996,7 +1034,7 @@ extern "C" int nvk_paged_decode_noalloc(const void* q, int64_t q_stride_tok,
   if (sst != NVK_OK) return sst;
   // Every descriptor and record the kernels read is written earlier in the
   // same call, so the scratch needs no clearing between calls.
-  return decode_run(a, head_dim, ws, s);
+  return decode_run(a, head_dim, scale, ws, s);
 }
 
 extern "C" int nvk_paged_decode_noalloc_init(void) {
@@ -1087,6 +1125,24 @@ extern "C" int nvk_paged_decode_prologue(
   const bool aligned = (block_size % tc) == 0;
   a.f16 = dtype == NVK_DTYPE_F16;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  // Group sizes whose decode runs on the short-query kernels: the prologue
+  // kernel writes q into `out` (whose rows a wave overwrites only when it has
+  // finished the whole group it read them for; the rows of cut groups are
+  // written by the combine), then that decode.
+  if (short_query_decode_applies(block_size, num_blocks, num_q_heads, num_kv_heads, head_dim,
+                                 batch) &&
+      out_stride_head >= head_dim && out_stride_tok >= (int64_t)num_q_heads * out_stride_head) {
+    const int st = nvk_qk_norm_rope_store(
+        qkv, qkv_row_stride, batch, positions, q_norm_weight, k_norm_weight, eps, cos_sin_cache,
+        cos_sin_row_stride, max_position, num_q_heads, num_kv_heads, head_dim, out,
+        out_stride_tok, out_stride_head, nullptr, 0, 0, k_cache, v_cache, slot_mapping,
+        cache_slots, dtype, stream);
+    if (st != NVK_OK) return st;
+    a.q = a.out;
+    a.q_stride_tok = out_stride_tok;
+    a.q_stride_head = out_stride_head;
+    return decode_short_query(a, scale, workspace, s);
+  }
   if (a.f16) return dispatch_group<128, true, true>(a, G, aligned, s);
   return dispatch_group<128, true>(a, G, aligned, s);
 }

@@ -32,10 +32,14 @@
 //     order comes from the wave's LDS copy of the chunk by two
 //     ds_read_b64_tr_b16 per operand (16-byte chunks of each 256-byte row
 //     XOR-swizzled by 2*(row & 7): conflict-free);
+//   * (decode form) a decode of 4 or 8 query heads per kv head is such a step
+//     with one query per sequence: the stream costs no VALU time per head;
 //   * online softmax per chunk in log2 units; groups cut between waves leave
 //     (O, m, l) records that a combine kernel merges, as in the decode (with
 //     16 waves folding interleaved slices of the parts when groups are cut
 //     into many).
+#include <type_traits>
+
 #include "nvk_common.h"
 #include "short_query.h"
 
@@ -75,25 +79,42 @@ struct SqArgs {
   int64_t row_elems;   // Hkv * HD
   uint32_t row_bytes;  // row_elems * 2
   int32_t* desc;       // [batch][Hkv] x 2: first and last wave of the group, -1 if empty
-  float* rec;          // [n_waves][2][kR][kRec]
+  float* rec;          // [n_waves][2][rec_rows][kRec]
+  int rec_rows;        // kR; decode: G
   int n_waves;
 };
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
+// DECODE: one query per sequence, row s of q, over context_lens[s] keys.
+template <bool DECODE>
+__device__ __forceinline__ int raw_keys(const SqArgs& a, int s) {
+  if constexpr (DECODE) return ((sq_const_i32*)a.p.context_lens)[s];
+  return ((sq_const_i32*)a.p.cu_k)[s + 1] - ((sq_const_i32*)a.p.cu_k)[s];
+}
+template <bool DECODE>
 __device__ __forceinline__ int seq_keys(const SqArgs& a, int s) {
-  int lk = ((sq_const_i32*)a.p.cu_k)[s + 1] - ((sq_const_i32*)a.p.cu_k)[s];
+  int lk = raw_keys<DECODE>(a, s);
   lk = lk < 0 ? 0 : lk;
   return lk > a.cap ? a.cap : lk;
 }
+template <bool DECODE>
 __device__ __forceinline__ int seq_queries(const SqArgs& a, int s) {
+  if constexpr (DECODE) return 1;
   return ((sq_const_i32*)a.p.cu_q)[s + 1] - ((sq_const_i32*)a.p.cu_q)[s];
 }
+template <bool DECODE>
+__device__ __forceinline__ int first_row(const SqArgs& a, int s) {
+  if constexpr (DECODE) return s;
+  return ((sq_const_i32*)a.p.cu_q)[s];
+}
+template <bool DECODE>
 __device__ __forceinline__ int seq_chunks(const SqArgs& a, int s) {
-  return seq_queries(a, s) > 0 ? (seq_keys(a, s) + kCK - 1) / kCK : 0;
+  return seq_queries<DECODE>(a, s) > 0 ? (seq_keys<DECODE>(a, s) + kCK - 1) / kCK : 0;
 }
 
 // Exclusive prefix of chunks per sequence into s_cs[0..B]; returns the total.
+template <bool DECODE>
 __device__ int chunk_prefix(const SqArgs& a, int* s_cs, int* s_wsum) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int B = a.p.batch;
@@ -101,7 +122,7 @@ __device__ int chunk_prefix(const SqArgs& a, int* s_cs, int* s_wsum) {
   const int b0 = tid * per;
   int local = 0;
   for (int i = 0; i < per; ++i)
-    if (b0 + i < B) local += seq_chunks(a, b0 + i);
+    if (b0 + i < B) local += seq_chunks<DECODE>(a, b0 + i);
   const int x = nvk_wave_scan_add(local);  // inclusive over the wave
   if (lane == 63) s_wsum[wave] = x;
   __syncthreads();
@@ -110,7 +131,7 @@ __device__ int chunk_prefix(const SqArgs& a, int* s_cs, int* s_wsum) {
   for (int i = 0; i < per; ++i) {
     if (b0 + i < B) {
       s_cs[b0 + i] = run;
-      run += seq_chunks(a, b0 + i);
+      run += seq_chunks<DECODE>(a, b0 + i);
     }
   }
   const int total = s_wsum[0] + s_wsum[1] + s_wsum[2] + s_wsum[3];
@@ -157,7 +178,7 @@ __device__ __forceinline__ float max_xor16(float x) {
 
 // KLDS: K staged in LDS by full-row DMA loads like V (then read in the MFMA
 // operand layout), instead of loaded straight into the operand layout.
-template <bool F16, bool KLDS>
+template <bool F16, bool KLDS, bool DECODE>
 __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs a) {
   using E = NvkElt<F16>;
   typedef typename E::vec8 vec8;
@@ -169,7 +190,7 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
   const int r = lane & 15, g = lane >> 4;
   const int Hkv = a.p.num_kv_heads;
 
-  const int S = chunk_prefix(a, s_cs, s_wsum);
+  const int S = chunk_prefix<DECODE>(a, s_cs, s_wsum);
   if (blockIdx.x == 0) {  // groups no wave visits (no query or no key)
     for (int e = tid; e < a.p.batch * Hkv; e += 256) {
       const int b = e / Hkv;
@@ -227,11 +248,10 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
   const int32_t* bt_row = nullptr;
 
   auto start_group = [&]() {
-    q_row0 = ((sq_const_i32*)a.p.cu_q)[s];
-    Lq = seq_queries(a, s);
-    const int lk_raw = ((sq_const_i32*)a.p.cu_k)[s + 1] - ((sq_const_i32*)a.p.cu_k)[s];
-    nkeys = seq_keys(a, s);
-    diag = lk_raw - Lq;
+    q_row0 = first_row<DECODE>(a, s);
+    Lq = seq_queries<DECODE>(a, s);
+    nkeys = seq_keys<DECODE>(a, s);
+    diag = raw_keys<DECODE>(a, s) - Lq;
     tok = r / a.G;
     head = kvh * a.G + r % a.G;
     row_valid = tok < Lq;
@@ -353,7 +373,7 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
     ChunkSrc nsrc;
     if (!last) {
       const int32_t* nbt = a.p.block_tables + (int64_t)ns * a.p.bt_stride;
-      const int nkeys_n = ns == s ? nkeys : seq_keys(a, ns);
+      const int nkeys_n = ns == s ? nkeys : seq_keys<DECODE>(a, ns);
       nsrc = chunk_src(ns, nkvh, nk, nbt, nkeys_n);
       // KLDS: this chunk's K reads are done before its buffer is refilled
       if constexpr (KLDS) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -437,7 +457,7 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
           }
         }
       } else if (row_valid) {  // the combine reads the valid rows only
-        float* rec = a.rec + ((w * 2 + (started_here ? 0 : 1)) * kR + r) * (int64_t)kRec;
+        float* rec = a.rec + ((w * 2 + (started_here ? 0 : 1)) * a.rec_rows + r) * (int64_t)kRec;
 #pragma unroll
         for (int db = 0; db < HD / 16; ++db) *reinterpret_cast<nvk_f32x4*>(rec + 16 * db + 4 * g) = acc_o[db];
         if (g == 0) {
@@ -484,7 +504,7 @@ __device__ __forceinline__ void sq_merge_parts(const SqArgs& a, int row, int d0,
       const int p = base + u * S;
       const bool ok = p <= p2;
       const int pr = ok ? p : p1;
-      const float* rec = a.rec + (((int64_t)pr * 2 + (pr == p1 ? 0 : 1)) * kR + row) * kRec;
+      const float* rec = a.rec + (((int64_t)pr * 2 + (pr == p1 ? 0 : 1)) * a.rec_rows + row) * kRec;
       mv[u] = ok ? rec[HD] : -INFINITY;
       lv[u] = rec[HD + 1];
       ov[u] = *reinterpret_cast<const nvk_f32x4*>(rec + d0);
@@ -517,15 +537,15 @@ __device__ __forceinline__ void sq_write_row(uint16_t* op, float L, const nvk_f3
 
 // grid = (Hkv, batch), 512 threads: thread t owns row t / 32 and
 // d = 4 (t % 32) .. +3.
-template <bool F16>
+template <bool F16, bool DECODE>
 __global__ __launch_bounds__(512) void short_query_combine_kernel(SqArgs a) {
   const int kvh = blockIdx.x, s = blockIdx.y;
   const int row = threadIdx.x >> 5, d0 = 4 * (threadIdx.x & 31);
-  const int Lq = seq_queries(a, s);
+  const int Lq = seq_queries<DECODE>(a, s);
   const int tok = row / a.G;
   if (tok >= Lq) return;
   const int head = kvh * a.G + row % a.G;
-  uint16_t* op = a.p.out + (int64_t)(a.p.cu_q[s] + tok) * a.p.out_stride_tok +
+  uint16_t* op = a.p.out + (int64_t)(first_row<DECODE>(a, s) + tok) * a.p.out_stride_tok +
                  (int64_t)head * a.p.out_stride_head + d0;
   const int2 desc = *reinterpret_cast<const int2*>(a.desc + 2 * (s * a.p.num_kv_heads + kvh));
   if (desc.x < 0) {
@@ -555,17 +575,19 @@ __global__ __launch_bounds__(512) void short_query_combine_kernel(SqArgs a) {
 // a wave per row, 4 columns per lane), and wave 0 merges the waves' states
 // through LDS.
 constexpr int kSqSlices = 16;
-template <bool F16>
+template <bool F16, bool DECODE>
 __global__ __launch_bounds__(64 * kSqSlices) void short_query_combine_sliced_kernel(SqArgs a) {
   const int kvh = blockIdx.x / (kR / 2), s = blockIdx.y;
   const int lane = threadIdx.x & 63, slice = threadIdx.x >> 6;
-  const int row = 2 * (blockIdx.x % (kR / 2)) + (lane >> 5), d0 = 4 * (lane & 31);
-  const int Lq = seq_queries(a, s);
+  int row = 2 * (blockIdx.x % (kR / 2)) + (lane >> 5);
+  const int d0 = 4 * (lane & 31);
+  const int Lq = seq_queries<DECODE>(a, s);
   if (2 * (blockIdx.x % (kR / 2)) >= Lq * a.G) return;  // both rows empty (uniform)
   const bool row_ok = row < Lq * a.G;
+  if (!row_ok) --row;  // an odd row count: the spare half wave rereads the last row
   const int tok = row / a.G;
   const int head = kvh * a.G + row % a.G;
-  uint16_t* op = a.p.out + (int64_t)(a.p.cu_q[s] + tok) * a.p.out_stride_tok +
+  uint16_t* op = a.p.out + (int64_t)(first_row<DECODE>(a, s) + tok) * a.p.out_stride_tok +
                  (int64_t)head * a.p.out_stride_head + d0;
   const int2 desc = *reinterpret_cast<const int2*>(a.desc + 2 * (s * a.p.num_kv_heads + kvh));
   if (desc.x < 0) {  // uniform over the workgroup
@@ -628,6 +650,15 @@ bool short_query_applies(bool paged, int block_size, int max_seqlen_q, int num_q
   return max_seqlen_q > 0 && (int64_t)max_seqlen_q * G <= kR && batch > 0 && batch <= kMaxBatch;
 }
 
+bool short_query_decode_applies(int block_size, int num_blocks, int num_q_heads, int num_kv_heads,
+                                int head_dim, int batch) {
+  if (head_dim != HD || block_size <= 0 || block_size % kCK || num_blocks <= 0) return false;
+  if (num_kv_heads <= 0 || num_q_heads % num_kv_heads || batch <= 0 || batch > kMaxBatch)
+    return false;
+  const int G = num_q_heads / num_kv_heads;
+  return G <= kR && (G > kDecodeKernelGroup || (G == 1 && batch > kDecodeKernelBatch));
+}
+
 size_t short_query_ws_bytes(int batch, int64_t max_keys, int num_q_heads, int num_kv_heads) {
   (void)num_q_heads;
   if (batch <= 0 || num_kv_heads <= 0 || max_keys <= 0) return 0;
@@ -652,29 +683,30 @@ int short_query_launch(const ShortQueryParams& p, int64_t max_keys, void* ws, hi
   // trip less per chunk).  Bound from the static sizes.
   const int64_t chunks_bound = (max_keys + kCK - 1) / kCK * p.batch * p.num_kv_heads;
   const bool klds = chunks_bound >= (int64_t)kKldsMinChunks * a.n_waves;
-  const dim3 grid(a.n_waves / kWavesPerWG), block(64 * kWavesPerWG);
-  if (p.f16) {
-    if (klds) hipLaunchKernelGGL((short_query_kernel<true, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((short_query_kernel<true, false>), grid, block, 0, s, a);
-  } else {
-    if (klds) hipLaunchKernelGGL((short_query_kernel<false, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((short_query_kernel<false, false>), grid, block, 0, s, a);
-  }
-  int st = nvk_launch_status();
-  if (st != NVK_OK) return st;
+  const bool decode = p.context_lens != nullptr;
+  a.rec_rows = decode ? a.G : kR;
   // At least 32 waves per (sequence, kv head) group: its parts are folded in
   // slices.
   const bool sliced = a.n_waves >= 32 * (int64_t)p.batch * p.num_kv_heads;
-  const dim3 sgrid(p.num_kv_heads * (kR / 2), p.batch), cgrid(p.num_kv_heads, p.batch);
-  if (sliced && p.f16)
-    hipLaunchKernelGGL(short_query_combine_sliced_kernel<true>, sgrid, dim3(64 * kSqSlices), 0, s,
-                       a);
-  else if (sliced)
-    hipLaunchKernelGGL(short_query_combine_sliced_kernel<false>, sgrid, dim3(64 * kSqSlices), 0,
-                       s, a);
-  else if (p.f16)
-    hipLaunchKernelGGL(short_query_combine_kernel<true>, cgrid, dim3(32 * kR), 0, s, a);
-  else
-    hipLaunchKernelGGL(short_query_combine_kernel<false>, cgrid, dim3(32 * kR), 0, s, a);
-  return nvk_launch_status();
+  auto launch = [&](auto f16, auto dec) {
+    constexpr bool F16 = decltype(f16)::value, DECODE = decltype(dec)::value;
+    const dim3 grid(a.n_waves / kWavesPerWG), block(64 * kWavesPerWG);
+    if (klds) hipLaunchKernelGGL((short_query_kernel<F16, true, DECODE>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((short_query_kernel<F16, false, DECODE>), grid, block, 0, s, a);
+    const int st = nvk_launch_status();
+    if (st != NVK_OK) return st;
+    // thread / row ranges: rows of the records only (decode: G of kR)
+    const int rows = a.rec_rows;
+    if (sliced)
+      hipLaunchKernelGGL((short_query_combine_sliced_kernel<F16, DECODE>),
+                         dim3(p.num_kv_heads * (kR / 2), p.batch), dim3(64 * kSqSlices), 0, s, a);
+    else
+      hipLaunchKernelGGL((short_query_combine_kernel<F16, DECODE>), dim3(p.num_kv_heads, p.batch),
+                         dim3(32 * rows), 0, s, a);
+    return nvk_launch_status();
+  };
+  if (p.f16) return decode ? launch(std::true_type{}, std::true_type{})
+                           : launch(std::true_type{}, std::false_type{});
+  return decode ? launch(std::false_type{}, std::true_type{})
+                : launch(std::false_type{}, std::false_type{});
 }

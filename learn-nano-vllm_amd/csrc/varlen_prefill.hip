@@ -1334,7 +1334,7 @@ int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_he
                           num_kv_heads, head_dim, batch) &&
       workspace && workspace_bytes >= short_query_ws_bytes(batch, max_keys, num_q_heads,
                                                            num_kv_heads)) {
-    ShortQueryParams sp;
+    ShortQueryParams sp{};  // context_lens null: the varlen form
     sp.q = static_cast<const uint16_t*>(q);
     sp.q_stride_tok = q_stride_tok;
     sp.q_stride_head = q_stride_head;

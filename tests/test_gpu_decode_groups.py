@@ -1,0 +1,73 @@
+"""Decodes that run on the short-query MFMA kernels (4 and 8 query heads per kv
+head; one from 33 sequences up) against the oracle: contexts at the edges of
+chunks and pages, empty contexts, cut groups, strided q and out, both dtypes,
+and the prologue form, whose prologue writes q into the output rows."""
+import pytest
+import torch
+
+from gpu_utils import assert_attn_close, oracle_decode, say
+from nanovllm_amd import (paged_decode, paged_decode_with_prologue, qk_norm_rope_store,
+                          rope_cos_sin_cache)
+from nanovllm_amd.workloads import decode_case
+
+pytestmark = pytest.mark.gpu
+
+EDGES = [1, 0, 31, 32, 33, 255, 256, 257, 0, 1500, 4097]
+
+
+@pytest.mark.parametrize("hq,hkv,ctx,bs", [
+    (16, 4, EDGES, 256),
+    (16, 2, EDGES, 32),
+    (8, 1, [9000], 256),                          # one group over many waves: sliced combine
+    (16, 2, [0, 0, 0], 256),                      # nothing to read
+    (16, 2, [300 + 7 * i for i in range(150)], 64),   # K through LDS
+    (4, 4, [1 + 37 * i for i in range(33)], 256),     # one head, first batch on these kernels
+    (4, 4, [1 + 37 * i for i in range(32)], 256),     # the last on the decode kernel
+    (4, 1, EDGES, 48),                            # pages of 48 keys: the decode kernel
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_decode_groups_match_oracle(hq, hkv, ctx, bs, dtype):
+    pages = sum(-(-c // bs) for c in ctx)
+    case = decode_case(seed=7, hq=hq, hkv=hkv, ctx=ctx, block_size=bs, pool_blocks=pages + 2,
+                       width=max(1, max(-(-c // bs) for c in ctx)))
+    q, kc, vc = (t.to(dtype) for t in (case.q, case.k_cache, case.v_cache))
+    ref = oracle_decode(q, kc, vc, case.block_tables, case.context_lens, bs, case.scale)
+    say(f"decode {hq}/{hkv} heads, {len(ctx)} sequences, page {bs}, {dtype}")
+    b = len(ctx)
+    wide = torch.zeros(b, hq, 160, dtype=dtype, device="cuda")
+    wide[..., 16:144] = q.cuda()
+    out = torch.full((b, hq, 136), float("nan"), dtype=dtype, device="cuda")
+    kc, vc, lens, bt = (t.cuda() for t in (kc, vc, case.context_lens, case.block_tables))
+    paged_decode(wide[..., 16:144], kc, vc, lens, bt, case.scale, out=out[..., :128])
+    plain = paged_decode(q.cuda(), kc, vc, lens, bt, case.scale)
+    torch.cuda.synchronize()
+    assert_attn_close(plain, ref, "contiguous")
+    assert torch.equal(out[..., :128], plain), "strided rows give the same bits"
+    assert out[..., 128:].isnan().all(), "nothing outside the rows is written"
+
+
+@pytest.mark.parametrize("strided", [False, True])
+def test_prologue_form_with_q_in_the_output_rows(strided):
+    hq, hkv, bs = 16, 2, 256
+    ctx = [1, 32, 33, 257, 1700, 2900]
+    case = decode_case(seed=8, hq=hq, hkv=hkv, ctx=ctx, pool_blocks=30)
+    g = torch.Generator().manual_seed(9)
+    qkv = (torch.randn(len(ctx), (hq + 2 * hkv) * 128, generator=g) * 2).to(torch.bfloat16).cuda()
+    w = (1 + 0.2 * torch.randn(2, 128, generator=g)).to(torch.bfloat16).cuda()
+    cs = rope_cos_sin_cache(128, 4096, 1e6).cuda()
+    lens, bt = case.context_lens.cuda(), case.block_tables.cuda()
+    pos = (lens - 1).long()
+    slots = (bt.gather(1, (pos // bs)[:, None]).squeeze(1) * bs + pos % bs).to(torch.int32)
+    caches = [[case.k_cache.cuda(), case.v_cache.cuda()] for _ in range(2)]
+    say(f"prologue form, strided out {strided}")
+    q, _, _ = qk_norm_rope_store(pos, qkv, hq, hkv, 128, w[0], w[1], 1e-6, cs, *caches[0], slots,
+                                 return_k=False)
+    ref = paged_decode(q, *caches[0], lens, bt, 128 ** -0.5)
+    out = torch.empty(len(ctx), hq, 136 if strided else 128, dtype=torch.bfloat16, device="cuda")
+    out = out[..., :128]
+    for _ in range(2):      # the second call finds the first one's outputs in out
+        paged_decode_with_prologue(pos, qkv, hq, hkv, 128, w[0], w[1], 1e-6, cs, *caches[1], slots,
+                                   lens, bt, 128 ** -0.5, out=out)
+    torch.cuda.synchronize()
+    assert torch.equal(out, ref)
+    assert all(torch.equal(a, b) for a, b in zip(*caches))
