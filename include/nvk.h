@@ -252,6 +252,34 @@ size_t nvk_varlen_prefill_parts_workspace_size(int32_t batch, int32_t max_seqlen
                                                int32_t num_kv_heads, int32_t head_dim);
 
 /*
+ * A prefill layer's prologue and attention in one call: what
+ * nvk_qk_norm_rope_store (storing the new k and v at slot_mapping; NULL: no
+ * store) followed by nvk_varlen_prefill_ordered on its q give, bit for bit;
+ * q needs no memory of its own, it goes through out's rows.
+ *
+ * qkv, positions, the norm weights and the cos/sin cache: as in
+ * nvk_qk_norm_rope_store, n_tokens = total_q.
+ * Paged (block_tables != NULL): the keys are the caches', which then must be
+ *   given; k_new is unused.
+ * Dense: the keys are the new tokens' own, rotated into k_new
+ *   [total_q][num_kv_heads][head_dim] (contiguous, 16-byte aligned), the values
+ *   the v part of qkv.
+ * out: 16-byte aligned, strides multiples of 8, out_stride_tok >=
+ *   num_q_heads * out_stride_head >= num_q_heads * head_dim.
+ * workspace, order, max_seqlen_q / k: as in nvk_varlen_prefill_ordered.
+ */
+int nvk_varlen_prefill_prologue(
+    const void* qkv, int64_t qkv_row_stride, int64_t total_q, const int64_t* positions,
+    const void* q_norm_weight, const void* k_norm_weight, float eps, const float* cos_sin_cache,
+    int64_t cos_sin_row_stride, int64_t max_position, void* k_cache, void* v_cache,
+    const int32_t* slot_mapping, int64_t cache_slots, void* k_new, const int32_t* cu_seqlens_q,
+    const int32_t* cu_seqlens_k, int32_t batch, int32_t max_seqlen_q, int32_t max_seqlen_k,
+    const int32_t* block_tables, int64_t bt_stride, int32_t max_blocks, int32_t block_size,
+    int32_t num_blocks, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, float scale,
+    void* out, int64_t out_stride_tok, int64_t out_stride_head, void* workspace,
+    size_t workspace_bytes, const int32_t* order, size_t order_bytes, int32_t dtype, void* stream);
+
+/*
  * The longest-first order of a prefill's query tiles, ranked once for every
  * layer of a step.  Every decoder layer of a model step calls the prefill
  * with the same cu_seqlens (nanovllm/layers/attention.py:67-70, once per

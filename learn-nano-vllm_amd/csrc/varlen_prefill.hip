@@ -93,6 +93,10 @@ struct PrefillArgs {
   // + s, written by prefill_tile_order_kernel; null: the grid order.  Only
   // with n_splits == 1.
   const int32_t* order;
+  // Finite rows that no workgroup writes, row stride dummy_stride: q itself, or
+  // the packed qkv rows when q shares out's rows.
+  const uint16_t* dummy;
+  int64_t dummy_stride;
 };
 
 // Partial record of one (query tile, part): the unnormalised O^T accumulators
@@ -396,9 +400,9 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void varlen_prefill_kernel
   const uint64_t head_k = (uint64_t)(uintptr_t)(a.k + kvh * HD);
   const uint64_t head_v = (uint64_t)(uintptr_t)(a.v + kvh * HD);
   const uint32_t page_bytes = (uint32_t)a.block_size * k_row_bytes;
-  // kPagedAny: a key that does not exist reads the sequence's first q row
-  // (finite); its score is masked to -inf and its probability is 0.
-  const uint16_t* dummy = a.q + (int64_t)q_row0 * a.q_stride_tok;
+  // kPagedAny: a key that does not exist reads a row of the sequence's first
+  // query (finite); its score is masked to -inf and its probability is 0.
+  const uint16_t* dummy = a.dummy + (int64_t)q_row0 * a.dummy_stride;
 
   // A K or V tile load into one LDS stage, planned once per tile and issued as
   // kLoadsPerWave instructions per wave (load j: 4 rows), so the issues can be
@@ -1283,6 +1287,22 @@ size_t order_bytes_for(int32_t batch, int32_t max_seqlen_q, int64_t max_keys, in
   return order_bytes(pairs);
 }
 
+// The prologue of nvk_varlen_prefill_prologue: the arguments of
+// nvk_qk_norm_rope_store that its attention call does not have.
+struct Prologue {
+  const void* qkv;
+  int64_t qkv_row_stride;
+  const int64_t* positions;
+  const void *q_norm_weight, *k_norm_weight;
+  float eps;
+  const float* cos_sin;
+  int64_t cos_sin_stride, max_position;
+  void* k_new;  // dense: the new keys, normed and rotated
+  void *k_store, *v_store;
+  const int32_t* slot_mapping;
+  int64_t cache_slots;
+};
+
 int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
                         int64_t total_q, const void* k, const void* v, int64_t k_stride_tok,
                         int64_t v_stride_tok, int64_t kv_stride_head, int64_t total_k,
@@ -1293,7 +1313,7 @@ int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_he
                         int32_t head_dim, float scale, void* out, int64_t out_stride_tok,
                         int64_t out_stride_head, void* workspace, size_t workspace_bytes,
                         int32_t dtype, void* stream, const int32_t* given_order,
-                        size_t given_order_bytes) {
+                        size_t given_order_bytes, const Prologue* pro = nullptr) {
   if (batch < 0 || max_seqlen_q < 0 || max_seqlen_k < 0 || num_q_heads <= 0 ||
       num_kv_heads <= 0 || total_q < 0 || total_k < 0)
     return NVK_EINVAL;
@@ -1327,38 +1347,14 @@ int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_he
   int64_t max_keys = block_tables ? (int64_t)max_blocks * block_size : total_k;
   if (max_seqlen_k > 0 && max_seqlen_k < max_keys) max_keys = max_seqlen_k;
 
-  // Short query ranges (<= 16 rows per kv head) over paged keys: the stream-K
-  // short-query kernels, when the workspace holds their records.
-  if (num_blocks > 0 && max_keys > 0 &&
+  SplitPlan sp = plan_splits(batch, max_seqlen_q, max_keys, num_q_heads, num_kv_heads);
+  const bool short_q =
+      num_blocks > 0 && max_keys > 0 &&
       short_query_applies(block_tables != nullptr, block_size, max_seqlen_q, num_q_heads,
                           num_kv_heads, head_dim, batch) &&
       workspace && workspace_bytes >= short_query_ws_bytes(batch, max_keys, num_q_heads,
-                                                           num_kv_heads)) {
-    ShortQueryParams sp{};  // context_lens null: the varlen form
-    sp.q = static_cast<const uint16_t*>(q);
-    sp.q_stride_tok = q_stride_tok;
-    sp.q_stride_head = q_stride_head;
-    sp.k_cache = static_cast<const uint16_t*>(k);
-    sp.v_cache = static_cast<const uint16_t*>(v);
-    sp.cu_q = cu_seqlens_q;
-    sp.cu_k = cu_seqlens_k;
-    sp.batch = batch;
-    sp.block_tables = block_tables;
-    sp.bt_stride = bt_stride;
-    sp.max_blocks = max_blocks;
-    sp.block_size = block_size;
-    sp.num_blocks = num_blocks;
-    sp.num_q_heads = num_q_heads;
-    sp.num_kv_heads = num_kv_heads;
-    sp.scale = scale;
-    sp.out = static_cast<uint16_t*>(out);
-    sp.out_stride_tok = out_stride_tok;
-    sp.out_stride_head = out_stride_head;
-    sp.f16 = dtype == NVK_DTYPE_F16;
-    return short_query_launch(sp, max_keys, workspace, reinterpret_cast<hipStream_t>(stream));
-  }
-  SplitPlan sp = plan_splits(batch, max_seqlen_q, max_keys, num_q_heads, num_kv_heads);
-  if (sp.n_qtiles > 65535) return NVK_EINVAL;
+                                                           num_kv_heads);
+  if (sp.n_qtiles > 65535 && !short_q) return NVK_EINVAL;
   const SplitPlan parts =
       plan_parts(batch, max_seqlen_q, max_keys, num_q_heads, num_kv_heads);
   if (parts.n_splits > 1 && workspace &&
@@ -1369,11 +1365,59 @@ int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_he
     sp.n_splits = 1;  // no room for partials: one workgroup per query tile
     sp.tiles_per_split = (int)((max_keys + kKeys - 1) / kKeys);
   }
+  const int64_t pairs = (int64_t)batch * sp.n_qtiles;
+  const bool ranked = sp.n_splits == 1 && !short_q && use_order(batch, pairs, num_kv_heads);
+  if (ranked && given_order) {
+    if (given_order_bytes < order_bytes(pairs)) return NVK_EWORKSPACE;
+    if ((uintptr_t)given_order % 4) return NVK_EALIGN;
+  }
 
-  PrefillArgs a;
+  if (pro) {
+    // q goes through out's rows: a workgroup (or, in the short-query kernels, a
+    // wave) overwrites only rows whose q it alone has read, and the rows of
+    // tiles and groups that several of them share are written by the merging
+    // kernel, after all of them.
+    const int st = nvk_qk_norm_rope_store(
+        pro->qkv, pro->qkv_row_stride, total_q, pro->positions, pro->q_norm_weight,
+        pro->k_norm_weight, pro->eps, pro->cos_sin, pro->cos_sin_stride, pro->max_position,
+        num_q_heads, num_kv_heads, head_dim, out, out_stride_tok, out_stride_head, pro->k_new,
+        (int64_t)num_kv_heads * head_dim, head_dim, pro->k_store, pro->v_store, pro->slot_mapping,
+        pro->cache_slots, dtype, stream);
+    if (st != NVK_OK) return st;
+  }
+
+  // Short query ranges (<= 16 rows per kv head) over paged keys: the stream-K
+  // short-query kernels, when the workspace holds their records.
+  if (short_q) {
+    ShortQueryParams sq{};  // context_lens null: the varlen form
+    sq.q = static_cast<const uint16_t*>(q);
+    sq.q_stride_tok = q_stride_tok;
+    sq.q_stride_head = q_stride_head;
+    sq.k_cache = static_cast<const uint16_t*>(k);
+    sq.v_cache = static_cast<const uint16_t*>(v);
+    sq.cu_q = cu_seqlens_q;
+    sq.cu_k = cu_seqlens_k;
+    sq.batch = batch;
+    sq.block_tables = block_tables;
+    sq.bt_stride = bt_stride;
+    sq.max_blocks = max_blocks;
+    sq.block_size = block_size;
+    sq.num_blocks = num_blocks;
+    sq.num_q_heads = num_q_heads;
+    sq.num_kv_heads = num_kv_heads;
+    sq.scale = scale;
+    sq.out = static_cast<uint16_t*>(out);
+    sq.out_stride_tok = out_stride_tok;
+    sq.out_stride_head = out_stride_head;
+    sq.f16 = dtype == NVK_DTYPE_F16;
+    return short_query_launch(sq, max_keys, workspace, reinterpret_cast<hipStream_t>(stream));
+  }
+  PrefillArgs a{};
   a.q = static_cast<const uint16_t*>(q);
   a.q_stride_tok = q_stride_tok;
   a.q_stride_head = q_stride_head;
+  a.dummy = pro ? static_cast<const uint16_t*>(pro->qkv) : a.q;
+  a.dummy_stride = pro ? pro->qkv_row_stride : q_stride_tok;
   a.total_q = total_q;
   a.k = static_cast<const uint16_t*>(k);
   a.v = static_cast<const uint16_t*>(v);
@@ -1405,12 +1449,8 @@ int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_he
   // One query tile per workgroup, a grid of several rounds and room in the
   // workspace: rank the tiles longest first (one more small kernel).  One
   // sequence: the grid order (last query tile first) already is.
-  a.order = nullptr;
-  const int64_t pairs = (int64_t)batch * sp.n_qtiles;
-  if (sp.n_splits == 1 && use_order(batch, pairs, num_kv_heads)) {
+  if (ranked) {
     if (given_order) {
-      if (given_order_bytes < order_bytes(pairs)) return NVK_EWORKSPACE;
-      if ((uintptr_t)given_order % 4) return NVK_EALIGN;
       a.order = given_order;  // ranked once for every layer of the step
     } else if (workspace && workspace_bytes >= order_bytes(pairs)) {
       int32_t* order = static_cast<int32_t*>(workspace);
@@ -1461,6 +1501,33 @@ extern "C" int nvk_varlen_prefill_ordered(
                              max_blocks, block_size, num_blocks, num_q_heads, num_kv_heads,
                              head_dim, scale, out, out_stride_tok, out_stride_head, workspace,
                              workspace_bytes, dtype, stream, order, order_bytes_);
+}
+
+extern "C" int nvk_varlen_prefill_prologue(
+    const void* qkv, int64_t qkv_row_stride, int64_t total_q, const int64_t* positions,
+    const void* q_norm_weight, const void* k_norm_weight, float eps, const float* cos_sin_cache,
+    int64_t cos_sin_row_stride, int64_t max_position, void* k_cache, void* v_cache,
+    const int32_t* slot_mapping, int64_t cache_slots, void* k_new, const int32_t* cu_seqlens_q,
+    const int32_t* cu_seqlens_k, int32_t batch, int32_t max_seqlen_q, int32_t max_seqlen_k,
+    const int32_t* block_tables, int64_t bt_stride, int32_t max_blocks, int32_t block_size,
+    int32_t num_blocks, int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim, float scale,
+    void* out, int64_t out_stride_tok, int64_t out_stride_head, void* workspace,
+    size_t workspace_bytes, const int32_t* order, size_t order_bytes_, int32_t dtype,
+    void* stream) {
+  if (num_q_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0) return NVK_EINVAL;
+  if (!qkv || (block_tables ? (!k_cache || !v_cache) : !k_new)) return NVK_EINVAL;
+  const Prologue p = {qkv, qkv_row_stride, positions, q_norm_weight, k_norm_weight, eps,
+                      cos_sin_cache, cos_sin_row_stride, max_position,
+                      block_tables ? nullptr : k_new, k_cache, v_cache, slot_mapping, cache_slots};
+  // dense: the step's own keys and the v part of qkv
+  const int64_t k_row = (int64_t)num_kv_heads * head_dim;
+  const uint16_t* v = static_cast<const uint16_t*>(qkv) + (int64_t)num_q_heads * head_dim + k_row;
+  return varlen_prefill_impl(
+      out, out_stride_tok, out_stride_head, total_q, block_tables ? k_cache : k_new,
+      block_tables ? v_cache : v, k_row, qkv_row_stride, head_dim, total_q, cu_seqlens_q,
+      cu_seqlens_k, batch, max_seqlen_q, max_seqlen_k, block_tables, bt_stride, max_blocks,
+      block_size, num_blocks, num_q_heads, num_kv_heads, head_dim, scale, out, out_stride_tok,
+      out_stride_head, workspace, workspace_bytes, dtype, stream, order, order_bytes_, &p);
 }
 
 extern "C" size_t nvk_prefill_tile_order_size(int32_t batch, int32_t max_seqlen_q,

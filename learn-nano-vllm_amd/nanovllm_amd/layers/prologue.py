@@ -24,6 +24,8 @@ from __future__ import annotations
 import torch
 
 from nanovllm_amd import _lib
+from nanovllm_amd.flash_api import _int32, _key_bound
+from nanovllm_amd.layers.attention import Attention, _prefill_order
 from nanovllm_amd.utils.context import get_context
 
 # Largest decode batch routed to the decode kernel with the prologue inside.
@@ -58,6 +60,35 @@ def _same_dtype(*ts: torch.Tensor) -> None:
                                 f"{dt} and {t.dtype}")
 
 
+def _check_prologue(positions, qkv, num_heads, num_kv_heads, head_dim, q_norm_weight,
+                    k_norm_weight, cos_sin_cache, k_cache, v_cache, slot_mapping):
+    """The prologue's argument checks; returns (cos/sin rows, int64 positions,
+    int32 slots or None, rows of the caches)."""
+    T = qkv.shape[0]
+    q_size, kv_size = num_heads * head_dim, num_kv_heads * head_dim
+    assert qkv.dim() == 2 and qkv.shape[1] == q_size + 2 * kv_size and qkv.stride(-1) == 1
+    assert positions.numel() == T
+    assert q_norm_weight.numel() == head_dim and k_norm_weight.numel() == head_dim
+    cs = cos_sin_cache.reshape(cos_sin_cache.shape[0], -1)
+    assert cs.shape[1] == head_dim and cs.stride(-1) == 1 and cs.dtype == torch.float32
+    _same_dtype(qkv, q_norm_weight, k_norm_weight)
+    slots, cache_slots = None, 0
+    if slot_mapping is not None:
+        D = kv_size
+        assert k_cache is not None and v_cache is not None
+        assert k_cache.stride(1) == D and v_cache.stride(1) == D      # attention.py:38
+        assert slot_mapping.numel() == T                               # attention.py:39
+        assert k_cache.stride(0) == k_cache.shape[1] * D and v_cache.stride(0) == v_cache.shape[1] * D
+        assert k_cache.shape == v_cache.shape
+        _same_dtype(qkv, k_cache, v_cache)
+        _lib.require_gpu(slot_mapping)
+        slots = slot_mapping if slot_mapping.dtype == torch.int32 else slot_mapping.to(torch.int32)
+        slots = slots.contiguous()
+        cache_slots = k_cache.shape[0] * k_cache.shape[1]
+    pos = positions if positions.dtype == torch.int64 else positions.to(torch.int64)
+    return cs, pos.contiguous(), slots, cache_slots
+
+
 def qk_norm_rope_store(positions: torch.Tensor, qkv: torch.Tensor, num_heads: int,
                        num_kv_heads: int, head_dim: int, q_norm_weight: torch.Tensor,
                        k_norm_weight: torch.Tensor, eps: float, cos_sin_cache: torch.Tensor,
@@ -74,36 +105,16 @@ def qk_norm_rope_store(positions: torch.Tensor, qkv: torch.Tensor, num_heads: in
     store_kvcache does; without it nothing is stored.
     """
     T = qkv.shape[0]
-    q_size, kv_size = num_heads * head_dim, num_kv_heads * head_dim
-    assert qkv.dim() == 2 and qkv.shape[1] == q_size + 2 * kv_size and qkv.stride(-1) == 1
-    assert positions.numel() == T
-    assert q_norm_weight.numel() == head_dim and k_norm_weight.numel() == head_dim
-    cs = cos_sin_cache.reshape(cos_sin_cache.shape[0], -1)
-    assert cs.shape[1] == head_dim and cs.stride(-1) == 1 and cs.dtype == torch.float32
-    _same_dtype(qkv, q_norm_weight, k_norm_weight)
-    v = qkv[:, q_size + kv_size:].view(-1, num_kv_heads, head_dim)
-    store = slot_mapping is not None
-    if store:
-        D = kv_size
-        assert k_cache is not None and v_cache is not None
-        assert k_cache.stride(1) == D and v_cache.stride(1) == D      # attention.py:38
-        assert slot_mapping.numel() == T                               # attention.py:39
-        assert k_cache.stride(0) == k_cache.shape[1] * D and v_cache.stride(0) == v_cache.shape[1] * D
-        assert k_cache.shape == v_cache.shape
-        _same_dtype(qkv, k_cache, v_cache)
-    dev = _lib.require_gpu(qkv, positions, q_norm_weight, k_norm_weight, cs,
-                           k_cache if store else None, v_cache if store else None, slot_mapping)
+    cs, pos, slots, cache_slots = _check_prologue(
+        positions, qkv, num_heads, num_kv_heads, head_dim, q_norm_weight, k_norm_weight,
+        cos_sin_cache, k_cache, v_cache, slot_mapping)
+    store = slots is not None
+    v = qkv[:, (num_heads + num_kv_heads) * head_dim:].view(-1, num_kv_heads, head_dim)
+    dev = _lib.require_gpu(qkv, pos, q_norm_weight, k_norm_weight, cs,
+                           k_cache if store else None, v_cache if store else None, slots)
     q = torch.empty(T, num_heads, head_dim, dtype=qkv.dtype, device=dev)
     k = torch.empty(T, num_kv_heads, head_dim, dtype=qkv.dtype, device=dev) if return_k else None
-    pos = positions if positions.dtype == torch.int64 else positions.to(torch.int64)
-    pos = pos.contiguous()
     qw, kw = q_norm_weight.contiguous(), k_norm_weight.contiguous()
-    slots = None
-    cache_slots = 0
-    if store:
-        slots = slot_mapping if slot_mapping.dtype == torch.int32 else slot_mapping.to(torch.int32)
-        slots = slots.contiguous()
-        cache_slots = k_cache.shape[0] * k_cache.shape[1]
     lib = _lib.load()
     with torch.cuda.device(dev):
         code = lib.nvk_qk_norm_rope_store(
@@ -175,6 +186,65 @@ def paged_decode_with_prologue(positions: torch.Tensor, qkv: torch.Tensor, num_h
     return out
 
 
+def _hooked(m: torch.nn.Module) -> bool:
+    """Whether calling the module runs more than its forward."""
+    mod = torch.nn.modules.module
+    return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                or m._backward_pre_hooks or mod._global_forward_hooks
+                or mod._global_forward_pre_hooks or mod._global_backward_hooks
+                or mod._global_backward_pre_hooks)
+
+
+def _prefill_with_prologue(attn, context, positions, qkv, qw, kw, eps, cos_sin_cache, store):
+    """A prefill step's prologue and attention in one library call
+    (``nvk_varlen_prefill_prologue``): the results of ``qk_norm_rope_store``
+    followed by ``attn(q, k, v, kv_stored=True)``, bit for bit."""
+    T, hq, hkv, d = qkv.shape[0], attn.num_heads, attn.num_kv_heads, attn.head_dim
+    cs, pos, slots, cache_slots = _check_prologue(
+        positions, qkv, hq, hkv, d, qw, kw, cos_sin_cache, attn.k_cache if store else None,
+        attn.v_cache if store else None, context.slot_mapping if store else None)
+    bt = context.block_tables
+    dev = _lib.require_gpu(qkv, pos, qw, kw, cs, slots, attn.k_cache if store else None,
+                           attn.v_cache if store else None, context.cu_seqlens_q,
+                           context.cu_seqlens_k, bt)
+    qw, kw = qw.contiguous(), kw.contiguous()
+    cu_q, cu_k = _int32(context.cu_seqlens_q), _int32(context.cu_seqlens_k)
+    batch = cu_q.numel() - 1
+    if cu_k.numel() != batch + 1:
+        raise _lib.NvkError("cu_seqlens_q and cu_seqlens_k disagree on the batch size")
+    mq = int(context.max_seqlen_q)
+    out = torch.empty((T, hq, d), dtype=qkv.dtype, device=dev)
+    if bt is not None:
+        keys, k_new = attn.k_cache, None
+        if not (keys.is_contiguous() and attn.v_cache.is_contiguous()):
+            raise _lib.NvkError("paged k/v must be contiguous [num_blocks, block_size, Hkv, D] caches")
+        bt = _int32(bt)
+        if bt.dim() != 2 or bt.shape[0] != batch:
+            raise _lib.NvkError("block_table must be [batch, max_blocks]")
+        num_blocks, block_size = keys.shape[:2]
+        max_blocks, bt_stride = bt.shape[1], bt.stride(0)
+    else:
+        keys = k_new = torch.empty((T, hkv, d), dtype=qkv.dtype, device=dev)
+        num_blocks = block_size = max_blocks = bt_stride = 0
+    mk = _key_bound(keys, bt, context.max_seqlen_k)
+    order = _prefill_order(context, out, keys, bt)
+    lib = _lib.load()
+    ws_bytes = lib.nvk_varlen_prefill_parts_workspace_size(batch, mq, mk, hq, hkv, d)
+    ws = _lib.workspace(dev, ws_bytes)
+    with torch.cuda.device(dev):
+        code = lib.nvk_varlen_prefill_prologue(
+            qkv.data_ptr(), qkv.stride(0), T, pos.data_ptr(), qw.data_ptr(), kw.data_ptr(),
+            float(eps), cs.data_ptr(), cs.stride(0), cs.shape[0],
+            attn.k_cache.data_ptr() if store else None, attn.v_cache.data_ptr() if store else None,
+            _lib.ptr(slots), cache_slots, _lib.ptr(k_new), cu_q.data_ptr(), cu_k.data_ptr(), batch,
+            mq, mk, _lib.ptr(bt), bt_stride, max_blocks, block_size, num_blocks, hq, hkv, d,
+            float(attn.scale), out.data_ptr(), out.stride(0), out.stride(1), _lib.ptr(ws),
+            ws_bytes, _lib.ptr(order), order.numel() * 4 if order is not None else 0,
+            _lib.dtype_code(qkv), _lib.stream_ptr(dev))
+    _lib.check(code)
+    return out
+
+
 def attention_with_prologue(attn, positions: torch.Tensor, qkv: torch.Tensor, q_norm, k_norm,
                             rotary_emb) -> torch.Tensor:
     """Qwen3Attention.forward up to and including ``self.attn(q, k, v)``
@@ -193,6 +263,10 @@ def attention_with_prologue(attn, positions: torch.Tensor, qkv: torch.Tensor, q_
             k_norm.weight, q_norm.eps, rotary_emb.cos_sin_cache, attn.k_cache, attn.v_cache,
             context.slot_mapping, context.context_lens, context.block_tables,
             attn.scale).unsqueeze(1)
+    if (context.is_prefill and context.max_seqlen_q > 0 and type(attn) is Attention
+            and (store or context.block_tables is None) and not _hooked(attn)):
+        return _prefill_with_prologue(attn, context, positions, qkv, q_norm.weight, k_norm.weight,
+                                      q_norm.eps, rotary_emb.cos_sin_cache, store)
     # k itself is read only by the dense (no block table) prefill
     need_k = context.is_prefill and context.block_tables is None
     q, k, v = qk_norm_rope_store(
