@@ -27,7 +27,7 @@
 // are ordered b-major, head block next, and the T chunks of the step are cut
 // into equal contiguous ranges, one per wave of a persistent grid of at most
 // 512 workgroups x 4 waves (static, so the launch can be captured in a graph;
-// when T is small only T/2 waves take part).  Every wave streams the same
+// when T is small only T or T/2 waves take part).  Every wave streams the same
 // number of bytes whatever the mix of context lengths.  Measured on MI355X, a
 // wave that issues one chunk, waits and computes it, with 8 waves per CU,
 // streams this access pattern at the rate of a plain read probe; deeper
@@ -61,10 +61,18 @@ constexpr int kLoads = 8;          // load instructions per tensor per chunk
 constexpr int kWavesPerWG = 4;
 constexpr int kMaxWGs = 512;       // 256 CUs x 2 workgroups (8 waves per CU)
 constexpr int kMaxBatch = 2048;    // sequences per call (LDS prefix table)
-// A wave streams at least this many chunks.  Measured on MI355X: 2 against 8
-// takes a 4-sequence decode from 30 to 17 us and a 16-sequence one from 34 to
-// 27 us (more waves share a small step), and changes nothing from 64 up.
+// Chunks a wave streams at least.  One where every chunk of the step gets a
+// wave of its own and no group is cut into very many parts: the second chunk's
+// page id, K/V round trip and arithmetic follow the first's, ~2 us of a step
+// that takes ~10.  Two otherwise: uneven ranges of one and two chunks take as
+// long as two, with more parts to merge.  Measured on MI355X, two / one, 16/8
+// heads: 1 x 100 keys 9.4 / 8.1 us, 1 x 1000 11.9 / 10.0, 16 x U{100..300}
+// 12.6 / 10.6, 4 x U{100..2048} 13.7 / 13.1 (a 28-layer graph step of one
+// sequence 391 / 309 us); 16 x U{100..2048} (1.8 chunks a wave) 20.1 / 21.8;
+// 8/4 heads, 1 x 16000 (500 chunks per group) 16.9 / 19.2, 2 x U{4000..8000}
+// 15.1 / 16.0.
 constexpr int kMinChunks = 2;
+constexpr int kOneChunkGroup = 128;  // chunks per group, on average, up to which one is taken
 #ifndef NVK_DECODE_SLICE_MIN_WAVES
 #define NVK_DECODE_SLICE_MIN_WAVES 32
 #endif
@@ -120,9 +128,11 @@ __device__ __forceinline__ int clamp_ctx(const DecodeArgs& a, int b) {
   return ctx;
 }
 
-// Waves that take part for T chunks: at most P, and few enough that each
-// range holds kMinChunks chunks (bounds how finely a context is split).
-__device__ __forceinline__ int64_t active_waves(int64_t T, int64_t P) {
+// Waves that take part for T chunks of `groups` groups: at most P, and few
+// enough that each range holds kMinChunks chunks (bounds how finely a context
+// is split), or one per chunk (kOneChunkGroup).
+__device__ __forceinline__ int64_t active_waves(int64_t T, int64_t P, int64_t groups) {
+  if (T <= P && T <= kOneChunkGroup * groups) return T < 1 ? 1 : T;
   int64_t p = T / kMinChunks;
   if (p > P) p = P;
   return p < 1 ? 1 : p;
@@ -516,7 +526,7 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(DecodeArgs a) {
     }
   }
   const int64_t T = (int64_t)n_blk * S;
-  const int64_t P = active_waves(T, a.n_waves);
+  const int64_t P = active_waves(T, a.n_waves, (int64_t)a.batch * n_blk);
   // the wave index is wave-uniform; say so, so that the range bookkeeping and
   // the page-table reads stay scalar
   const int64_t w = (int64_t)blockIdx.x * kWavesPerWG + uniform(tid >> 6);
@@ -774,7 +784,7 @@ int decode_waves(int batch, int num_kv_heads, int head_dim, int block_size, int 
   const int tc = decode_tc(num_kv_heads, head_dim);
   const int64_t max_chunks_seq = ((int64_t)block_size * max_blocks + tc - 1) / tc;
   const int64_t t_max = max_chunks_seq * batch * (num_kv_heads / decode_hpi(num_kv_heads, head_dim));
-  int64_t wgs = (t_max / kMinChunks + kWavesPerWG - 1) / kWavesPerWG;
+  int64_t wgs = (t_max + kWavesPerWG - 1) / kWavesPerWG;
   if (wgs > kMaxWGs) wgs = kMaxWGs;
   if (wgs < 1) wgs = 1;
   return (int)wgs * kWavesPerWG;

@@ -58,7 +58,15 @@ constexpr int kKB = kCK / 16;                 // 16-key blocks of a chunk
 constexpr int kPairs = kCK / 32;              // 32-key pairs (one P.V k-step each)
 constexpr int kWavesPerWG = 4;
 constexpr int kMaxWGs = 256;                  // one workgroup per CU
-constexpr int kMinChunks = 2;                 // a wave streams at least this many chunks
+// Chunks a wave streams at least: two, or one in steps of up to kOneChunkMax
+// chunks with at most kOneChunkGroup per group (a second chunk's round trip and
+// arithmetic follow the first's; more waves and parts cost more from there
+// on).  Measured on MI355X, decodes of 16/2 heads, two / one: 1 x 100 keys 9.0 /
+// 7.8 us, 4 x U{100..2048} 12.4 / 11.4, 16 x U{100..300} 12.0 / 10.9; 16 x
+// U{100..2048} (940 chunks) 13.6 / 14.0, 1 x 16000 (500 per group) 16.2 / 20.0.
+constexpr int kMinChunks = 2;
+constexpr int64_t kOneChunkMax = 768;
+constexpr int kOneChunkGroup = 128;
 #ifndef NVK_SQ_KLDS_MIN
 #define NVK_SQ_KLDS_MIN 32
 #endif
@@ -140,7 +148,8 @@ __device__ int chunk_prefix(const SqArgs& a, int* s_cs, int* s_wsum) {
   return total;
 }
 
-__device__ __forceinline__ int64_t active_waves(int64_t T, int64_t P) {
+__device__ __forceinline__ int64_t active_waves(int64_t T, int64_t P, int64_t groups) {
+  if (T <= P && T <= kOneChunkMax && T <= kOneChunkGroup * groups) return T < 1 ? 1 : T;
   int64_t p = T / kMinChunks;
   if (p > P) p = P;
   return p < 1 ? 1 : p;
@@ -198,7 +207,7 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
     }
   }
   const int64_t T = (int64_t)Hkv * S;
-  const int64_t P = active_waves(T, a.n_waves);
+  const int64_t P = active_waves(T, a.n_waves, (int64_t)a.p.batch * Hkv);
   const int wave = uniform(tid >> 6);
   const int64_t w = (int64_t)blockIdx.x * kWavesPerWG + wave;
   if (w >= P || T == 0) return;
@@ -627,10 +636,12 @@ __global__ __launch_bounds__(64 * kSqSlices) void short_query_combine_sliced_ker
   sq_write_row<F16>(op, L, O);
 }
 
-int sq_waves(int batch, int64_t max_keys, int num_kv_heads) {
+// Waves of the grid: as many as the step's chunks can use, by its static bound
+// (decode form: one chunk each, the varlen form's workspace holds two).
+int sq_waves(int batch, int64_t max_keys, int num_kv_heads, bool decode) {
   const int64_t chunks = (max_keys + kCK - 1) / kCK;
   const int64_t t_max = chunks * batch * num_kv_heads;
-  int64_t wgs = (t_max / kMinChunks + kWavesPerWG - 1) / kWavesPerWG;
+  int64_t wgs = (t_max / (decode ? 1 : kMinChunks) + kWavesPerWG - 1) / kWavesPerWG;
   if (wgs > kMaxWGs) wgs = kMaxWGs;
   if (wgs < 1) wgs = 1;
   return (int)wgs * kWavesPerWG;
@@ -663,7 +674,7 @@ size_t short_query_ws_bytes(int batch, int64_t max_keys, int num_q_heads, int nu
   (void)num_q_heads;
   if (batch <= 0 || num_kv_heads <= 0 || max_keys <= 0) return 0;
   return sq_desc_bytes(batch, num_kv_heads) +
-         (size_t)sq_waves(batch, max_keys, num_kv_heads) * 2 * kR * kRec * sizeof(float);
+         (size_t)sq_waves(batch, max_keys, num_kv_heads, false) * 2 * kR * kRec * sizeof(float);
 }
 
 int short_query_launch(const ShortQueryParams& p, int64_t max_keys, void* ws, hipStream_t s) {
@@ -677,7 +688,7 @@ int short_query_launch(const ShortQueryParams& p, int64_t max_keys, void* ws, hi
   a.row_bytes = (uint32_t)(a.row_elems * 2);
   a.desc = static_cast<int32_t*>(ws);
   a.rec = reinterpret_cast<float*>(static_cast<char*>(ws) + sq_desc_bytes(p.batch, p.num_kv_heads));
-  a.n_waves = sq_waves(p.batch, max_keys, p.num_kv_heads);
+  a.n_waves = sq_waves(p.batch, max_keys, p.num_kv_heads, p.context_lens != nullptr);
   // K through LDS when a wave may stream many chunks (its full-row loads
   // stream faster); straight into registers for short ranges (one LDS round
   // trip less per chunk).  Bound from the static sizes.

@@ -71,3 +71,25 @@ def test_prologue_form_with_q_in_the_output_rows(strided):
     torch.cuda.synchronize()
     assert torch.equal(out, ref)
     assert all(torch.equal(a, b) for a, b in zip(*caches))
+
+
+@pytest.mark.parametrize("hq,hkv,ctx", [
+    (16, 8, [1]), (16, 8, [1000]),                 # one chunk per wave
+    (4, 2, [4096]), (4, 2, [4097]),                # 128 and 129 chunks per group
+    (16, 8, [2048] * 4), (16, 8, [2048] * 4 + [1]),    # 2048 chunks (all waves) and more
+    (16, 2, [3072] * 4), (16, 2, [3073] * 4),      # 768 chunks, and more, on the MFMA kernels
+    (8, 1, [4096, 1]), (8, 1, [9000, 0, 1]),
+])
+def test_one_and_two_chunks_per_wave(hq, hkv, ctx):
+    case = decode_case(seed=17, hq=hq, hkv=hkv, ctx=ctx, pool_blocks=sum(-(-c // 256) for c in ctx))
+    ref = oracle_decode(case.q, case.k_cache, case.v_cache, case.block_tables, case.context_lens,
+                        256, case.scale)
+    c = case.to("cuda")
+    say(f"decode {hq}/{hkv} over {ctx}")
+    # a wider table than the contexts need: more waves in the grid than chunks
+    wide = torch.full((len(ctx), c.block_tables.shape[1] + 40), -1, dtype=torch.int32, device="cuda")
+    wide[:, :c.block_tables.shape[1]] = c.block_tables
+    for bt in (c.block_tables, wide):
+        out = paged_decode(c.q, c.k_cache, c.v_cache, c.context_lens, bt, case.scale)
+        torch.cuda.synchronize()
+        assert_attn_close(out, ref, f"{hq}/{hkv} {ctx}")
