@@ -227,20 +227,38 @@ __device__ __forceinline__ float mass_x(float l, float scale) {
   return (x == x && x != INFINITY) ? x : -INFINITY;
 }
 
+// Maximum and inclusive prefix over the 64 lanes in VALU steps (DPP moves
+// inside the 16-lane rows, lane swaps and row broadcasts across them) instead
+// of six dependent LDS permutes each: a wave's chain from its last logit to its
+// stores has one of each.
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-  for (int m = 32; m >= 1; m >>= 1) v = fmaxf(v, __shfl_xor(v, m));
-  return v;
+  v = fmaxf(v, nvk_dpp<NVK_DPP_QP_XOR1>(v));
+  v = fmaxf(v, nvk_dpp<NVK_DPP_QP_XOR2>(v));
+  v = fmaxf(v, nvk_dpp<NVK_DPP_HALF_MIRROR>(v));
+  v = fmaxf(v, nvk_dpp<NVK_DPP_MIRROR>(v));
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false,
+                                                  false);
+  return nvk_max_xor32(fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])));
+}
+// v of the lane that CTRL names, 0 where it names none or the row is not in
+// ROWS.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ float dpp_or_zero(float v) {
+  return __int_as_float(
+      __builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, ROWS, 0xF, false));
 }
 // Inclusive prefix of v over the 64 lanes of a wave (in lane order).
 __device__ __forceinline__ float wave_incl(float v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const float y = __shfl_up(v, o);
-    if (lane >= o) v += y;
-  }
+  v += dpp_or_zero<0x111, 0xF>(v);  // row_shr:1
+  v += dpp_or_zero<0x112, 0xF>(v);  // row_shr:2
+  v += dpp_or_zero<0x114, 0xF>(v);  // row_shr:4
+  v += dpp_or_zero<0x118, 0xF>(v);  // row_shr:8
+  v += dpp_or_zero<0x142, 0xA>(v);  // row_bcast:15 -> rows 1, 3
+  v += dpp_or_zero<0x143, 0xC>(v);  // row_bcast:31 -> rows 2, 3
   return v;
+}
+__device__ __forceinline__ float lane_value(float v, int lane) {  // lane wave-uniform
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
 
 // two uniforms in (0, 1] from Philox4x32-10 at counter (offset, row, word),
@@ -353,7 +371,7 @@ __global__ __launch_bounds__(kPartThreads) void sample_draw_kernel(SampleArgs a)
   }
   // the lane, then the element of the lane
   const float incl = wave_incl(run);
-  const float total = __shfl(incl, 63);
+  const float total = lane_value(incl, 63);
   float u1, u2;
   row_uniforms(a, (uint32_t)row, 2u + (uint32_t)(c * (kPartThreads / 64) + wave), &u1, &u2);
   const uint64_t pos = __ballot(run > 0.f);
@@ -362,7 +380,7 @@ __global__ __launch_bounds__(kPartThreads) void sample_draw_kernel(SampleArgs a)
   const int pick = hit ? __builtin_ctzll(hit) : (pos ? 63 - __builtin_clzll(pos) : 0);
   const int k = first_reaching(cum, fmaxf(u2 * run, 1.401298464e-45f));
   const int tok = first + (k >> 3) * (kPartThreads * 8) + (k & 7);
-  const int tok_pick = __shfl(tok, pick);
+  const int tok_pick = __builtin_amdgcn_readlane(tok, __builtin_amdgcn_readfirstlane(pick));
   if (lane == 0) {
     const int64_t slot = (int64_t)row * (a.chunks * (kPartThreads / 64)) + c * (kPartThreads / 64) + wave;
     a.part_score[slot] = pos ? M : -INFINITY;
@@ -406,7 +424,7 @@ __global__ __launch_bounds__(256) void sample_choose_kernel(SampleArgs a, int ba
   for (int j = 0; j < kCached; ++j) {
     w[j] = weight(m[j], sm[j]);
     incl[j] = wave_incl(w[j]);
-    total += __shfl(incl[j], 63);
+    total += lane_value(incl[j], 63);
   }
   for (int base = 64 * kCached; base < n; base += 64) {
     const int e = base + lane;
@@ -424,7 +442,7 @@ __global__ __launch_bounds__(256) void sample_choose_kernel(SampleArgs a, int ba
     const uint64_t hit = __ballot(w[j] > 0.f && run + incl[j] >= t);
     if (pos) last = __shfl(tk[j], 63 - __builtin_clzll(pos));
     if (tok < 0 && hit) tok = __shfl(tk[j], __builtin_ctzll(hit));
-    run += __shfl(incl[j], 63);
+    run += lane_value(incl[j], 63);
   }
   for (int base = 64 * kCached; tok < 0 && base < n; base += 64) {
     const int e = base + lane;
