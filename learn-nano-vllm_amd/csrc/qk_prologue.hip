@@ -157,28 +157,34 @@ __global__ __launch_bounds__(16 * kMaxRowGroups) void qk_prologue_kernel(Prologu
     prologue_row<F16>(a, t, g, j, slot, raw, w, w, cs);
     return;
   }
-  nvk_u32x4 cs[4];
-  load_cs(cs);
-  const nvk_u32x4 wq = *reinterpret_cast<const nvk_u32x4*>(a.q_weight + 8 * j);
-  const nvk_u32x4 wk = *reinterpret_cast<const nvk_u32x4*>(a.k_weight + 8 * j);
-  auto pass = [&](int r0) {
-    nvk_u32x4 raw[kRowsPerPass];
+  nvk_u32x4 cs[4], wq, wk, raw[kRowsPerPass];
+  auto load_rows = [&](int r0) {
 #pragma unroll
     for (int i = 0; i < kRowsPerPass; ++i) {
       const int r = r0 + i * groups;  // a row past R loads row r0 (< R) unused
       raw[i] = load_nt(row0 + (int64_t)(r < R ? r : r0) * kHD);
     }
-    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto finish_rows = [&](int r0) {
 #pragma unroll
     for (int i = 0; i < kRowsPerPass; ++i) {
       const int r = r0 + i * groups;
       if (r < R) prologue_row<F16>(a, t, r, j, slot, raw[i], wq, wk, cs);
     }
   };
-  if (R <= kRowsPerPass * groups) {  // one pass (Qwen3: 32 rows, 16 groups): no loop
-    pass(g);
-  } else {
-    for (int r0 = g; r0 < R; r0 += kRowsPerPass * groups) pass(r0);
+  // The rows' loads leave first: the cos / sin addresses wait for the position.
+  // Measured (graph replays past the Infinity Cache, 16/8 heads): 600 tokens
+  // 4.95 -> 4.54 us, 2048 8.96 -> 8.62, 16384 45.5 -> 45.4 (5.9 TB/s).
+  load_rows(g);
+  wq = *reinterpret_cast<const nvk_u32x4*>(a.q_weight + 8 * j);
+  wk = *reinterpret_cast<const nvk_u32x4*>(a.k_weight + 8 * j);
+  load_cs(cs);
+  __builtin_amdgcn_sched_barrier(0);
+  finish_rows(g);
+  for (int r0 = g + kRowsPerPass * groups; r0 < R; r0 += kRowsPerPass * groups) {
+    load_rows(r0);
+    __builtin_amdgcn_sched_barrier(0);
+    finish_rows(r0);
   }
 }
 
