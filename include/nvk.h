@@ -252,6 +252,27 @@ size_t nvk_varlen_prefill_parts_workspace_size(int32_t batch, int32_t max_seqlen
                                                int32_t num_kv_heads, int32_t head_dim);
 
 /*
+ * n_query queries per sequence at the end of its context_lens[s] cached keys
+ * (speculative-decode verification): nvk_uniform_cu_seqlens +
+ * nvk_varlen_prefill in one launch less, without cu_seqlens in memory.  q and
+ * out: [batch * n_query] rows.  Only where the short-query kernels apply
+ * (n_query * num_q_heads / num_kv_heads <= 16, head_dim 128, pages of a
+ * multiple of 32 keys, batch <= 2048): elsewhere the workspace size is 0 and
+ * the call returns NVK_EUNSUPPORTED.
+ */
+size_t nvk_paged_verify_workspace_size(int32_t batch, int32_t n_query, int32_t num_q_heads,
+                                       int32_t num_kv_heads, int32_t head_dim,
+                                       int32_t block_size, int32_t max_blocks);
+int nvk_paged_verify(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
+                     const void* k_cache, const void* v_cache, const int32_t* block_tables,
+                     int64_t bt_stride, const int32_t* context_lens, int32_t batch,
+                     int32_t n_query, int32_t num_q_heads, int32_t num_kv_heads,
+                     int32_t head_dim, int32_t block_size, int32_t max_blocks,
+                     int32_t num_blocks, float scale, void* out, int64_t out_stride_tok,
+                     int64_t out_stride_head, void* workspace, size_t workspace_bytes,
+                     int32_t dtype, void* stream);
+
+/*
  * A prefill layer's prologue and attention in one call: what
  * nvk_qk_norm_rope_store (storing the new k and v at slot_mapping; NULL: no
  * store) followed by nvk_varlen_prefill_ordered on its q give, bit for bit;

@@ -910,6 +910,7 @@ int decode_short_query(const DecodeArgs& a, float scale, void* workspace, hipStr
   p.k_cache = a.k_cache;
   p.v_cache = a.v_cache;
   p.context_lens = a.context_lens;
+  p.n_query = 1;
   p.batch = a.batch;
   p.block_tables = a.block_tables;
   p.bt_stride = a.bt_stride;

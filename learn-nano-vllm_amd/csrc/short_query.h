@@ -15,8 +15,10 @@ struct ShortQueryParams {
   const uint16_t* v_cache;
   const int32_t* cu_q;
   const int32_t* cu_k;
-  // decode form: one query per sequence (row s of q), cu_q / cu_k unused; else null
+  // uniform form: n_query queries per sequence (rows s * n_query .. of q) at the
+  // end of its context_lens[s] keys, cu_q / cu_k unused; else null
   const int32_t* context_lens = nullptr;
+  int n_query = 1;
   int batch;
   const int32_t* block_tables;
   int64_t bt_stride;
@@ -55,10 +57,12 @@ constexpr int kDecodeKernelBatch = 32;
 bool short_query_decode_applies(int block_size, int num_blocks, int num_q_heads, int num_kv_heads,
                                 int head_dim, int batch);
 
-// Workspace bytes (descriptors + partial records) for these static sizes (the
-// decode form needs no more than nvk_paged_decode_workspace_size: at most as
-// many waves, the same records).
-size_t short_query_ws_bytes(int batch, int64_t max_keys, int num_q_heads, int num_kv_heads);
+// Workspace bytes (descriptors + partial records) for these static sizes.
+// n_query 0: the varlen form; else the uniform form (of which a decode needs
+// no more than nvk_paged_decode_workspace_size: at most as many waves, the same
+// records).
+size_t short_query_ws_bytes(int batch, int64_t max_keys, int num_q_heads, int num_kv_heads,
+                            int n_query = 0);
 
 // Enqueues the two kernels (stream-K pass, combine).  ws: 256-byte aligned,
 // short_query_ws_bytes() bytes.  Returns NVK_OK or a hipError_t.

@@ -88,41 +88,41 @@ struct SqArgs {
   uint32_t row_bytes;  // row_elems * 2
   int32_t* desc;       // [batch][Hkv] x 2: first and last wave of the group, -1 if empty
   float* rec;          // [n_waves][2][rec_rows][kRec]
-  int rec_rows;        // kR; decode: G
+  int rec_rows;        // kR; uniform form: n_query * G
   int n_waves;
 };
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
-// DECODE: one query per sequence, row s of q, over context_lens[s] keys.
-template <bool DECODE>
+// UNIFORM: n_query queries per sequence at the end of its context_lens[s] keys.
+template <bool UNIFORM>
 __device__ __forceinline__ int raw_keys(const SqArgs& a, int s) {
-  if constexpr (DECODE) return ((sq_const_i32*)a.p.context_lens)[s];
+  if constexpr (UNIFORM) return ((sq_const_i32*)a.p.context_lens)[s];
   return ((sq_const_i32*)a.p.cu_k)[s + 1] - ((sq_const_i32*)a.p.cu_k)[s];
 }
-template <bool DECODE>
+template <bool UNIFORM>
 __device__ __forceinline__ int seq_keys(const SqArgs& a, int s) {
-  int lk = raw_keys<DECODE>(a, s);
+  int lk = raw_keys<UNIFORM>(a, s);
   lk = lk < 0 ? 0 : lk;
   return lk > a.cap ? a.cap : lk;
 }
-template <bool DECODE>
+template <bool UNIFORM>
 __device__ __forceinline__ int seq_queries(const SqArgs& a, int s) {
-  if constexpr (DECODE) return 1;
+  if constexpr (UNIFORM) return a.p.n_query;
   return ((sq_const_i32*)a.p.cu_q)[s + 1] - ((sq_const_i32*)a.p.cu_q)[s];
 }
-template <bool DECODE>
+template <bool UNIFORM>
 __device__ __forceinline__ int first_row(const SqArgs& a, int s) {
-  if constexpr (DECODE) return s;
+  if constexpr (UNIFORM) return s * a.p.n_query;
   return ((sq_const_i32*)a.p.cu_q)[s];
 }
-template <bool DECODE>
+template <bool UNIFORM>
 __device__ __forceinline__ int seq_chunks(const SqArgs& a, int s) {
-  return seq_queries<DECODE>(a, s) > 0 ? (seq_keys<DECODE>(a, s) + kCK - 1) / kCK : 0;
+  return seq_queries<UNIFORM>(a, s) > 0 ? (seq_keys<UNIFORM>(a, s) + kCK - 1) / kCK : 0;
 }
 
 // Exclusive prefix of chunks per sequence into s_cs[0..B]; returns the total.
-template <bool DECODE>
+template <bool UNIFORM>
 __device__ int chunk_prefix(const SqArgs& a, int* s_cs, int* s_wsum) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int B = a.p.batch;
@@ -130,7 +130,7 @@ __device__ int chunk_prefix(const SqArgs& a, int* s_cs, int* s_wsum) {
   const int b0 = tid * per;
   int local = 0;
   for (int i = 0; i < per; ++i)
-    if (b0 + i < B) local += seq_chunks<DECODE>(a, b0 + i);
+    if (b0 + i < B) local += seq_chunks<UNIFORM>(a, b0 + i);
   const int x = nvk_wave_scan_add(local);  // inclusive over the wave
   if (lane == 63) s_wsum[wave] = x;
   __syncthreads();
@@ -139,7 +139,7 @@ __device__ int chunk_prefix(const SqArgs& a, int* s_cs, int* s_wsum) {
   for (int i = 0; i < per; ++i) {
     if (b0 + i < B) {
       s_cs[b0 + i] = run;
-      run += seq_chunks<DECODE>(a, b0 + i);
+      run += seq_chunks<UNIFORM>(a, b0 + i);
     }
   }
   const int total = s_wsum[0] + s_wsum[1] + s_wsum[2] + s_wsum[3];
@@ -187,7 +187,7 @@ __device__ __forceinline__ float max_xor16(float x) {
 
 // KLDS: K staged in LDS by full-row DMA loads like V (then read in the MFMA
 // operand layout), instead of loaded straight into the operand layout.
-template <bool F16, bool KLDS, bool DECODE>
+template <bool F16, bool KLDS, bool UNIFORM>
 __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs a) {
   using E = NvkElt<F16>;
   typedef typename E::vec8 vec8;
@@ -199,7 +199,7 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
   const int r = lane & 15, g = lane >> 4;
   const int Hkv = a.p.num_kv_heads;
 
-  const int S = chunk_prefix<DECODE>(a, s_cs, s_wsum);
+  const int S = chunk_prefix<UNIFORM>(a, s_cs, s_wsum);
   if (blockIdx.x == 0) {  // groups no wave visits (no query or no key)
     for (int e = tid; e < a.p.batch * Hkv; e += 256) {
       const int b = e / Hkv;
@@ -257,10 +257,10 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
   const int32_t* bt_row = nullptr;
 
   auto start_group = [&]() {
-    q_row0 = first_row<DECODE>(a, s);
-    Lq = seq_queries<DECODE>(a, s);
-    nkeys = seq_keys<DECODE>(a, s);
-    diag = raw_keys<DECODE>(a, s) - Lq;
+    q_row0 = first_row<UNIFORM>(a, s);
+    Lq = seq_queries<UNIFORM>(a, s);
+    nkeys = seq_keys<UNIFORM>(a, s);
+    diag = raw_keys<UNIFORM>(a, s) - Lq;
     tok = r / a.G;
     head = kvh * a.G + r % a.G;
     row_valid = tok < Lq;
@@ -382,7 +382,7 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
     ChunkSrc nsrc;
     if (!last) {
       const int32_t* nbt = a.p.block_tables + (int64_t)ns * a.p.bt_stride;
-      const int nkeys_n = ns == s ? nkeys : seq_keys<DECODE>(a, ns);
+      const int nkeys_n = ns == s ? nkeys : seq_keys<UNIFORM>(a, ns);
       nsrc = chunk_src(ns, nkvh, nk, nbt, nkeys_n);
       // KLDS: this chunk's K reads are done before its buffer is refilled
       if constexpr (KLDS) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -546,15 +546,15 @@ __device__ __forceinline__ void sq_write_row(uint16_t* op, float L, const nvk_f3
 
 // grid = (Hkv, batch), 512 threads: thread t owns row t / 32 and
 // d = 4 (t % 32) .. +3.
-template <bool F16, bool DECODE>
+template <bool F16, bool UNIFORM>
 __global__ __launch_bounds__(512) void short_query_combine_kernel(SqArgs a) {
   const int kvh = blockIdx.x, s = blockIdx.y;
   const int row = threadIdx.x >> 5, d0 = 4 * (threadIdx.x & 31);
-  const int Lq = seq_queries<DECODE>(a, s);
+  const int Lq = seq_queries<UNIFORM>(a, s);
   const int tok = row / a.G;
   if (tok >= Lq) return;
   const int head = kvh * a.G + row % a.G;
-  uint16_t* op = a.p.out + (int64_t)(first_row<DECODE>(a, s) + tok) * a.p.out_stride_tok +
+  uint16_t* op = a.p.out + (int64_t)(first_row<UNIFORM>(a, s) + tok) * a.p.out_stride_tok +
                  (int64_t)head * a.p.out_stride_head + d0;
   const int2 desc = *reinterpret_cast<const int2*>(a.desc + 2 * (s * a.p.num_kv_heads + kvh));
   if (desc.x < 0) {
@@ -584,19 +584,19 @@ __global__ __launch_bounds__(512) void short_query_combine_kernel(SqArgs a) {
 // a wave per row, 4 columns per lane), and wave 0 merges the waves' states
 // through LDS.
 constexpr int kSqSlices = 16;
-template <bool F16, bool DECODE>
+template <bool F16, bool UNIFORM>
 __global__ __launch_bounds__(64 * kSqSlices) void short_query_combine_sliced_kernel(SqArgs a) {
   const int kvh = blockIdx.x / (kR / 2), s = blockIdx.y;
   const int lane = threadIdx.x & 63, slice = threadIdx.x >> 6;
   int row = 2 * (blockIdx.x % (kR / 2)) + (lane >> 5);
   const int d0 = 4 * (lane & 31);
-  const int Lq = seq_queries<DECODE>(a, s);
+  const int Lq = seq_queries<UNIFORM>(a, s);
   if (2 * (blockIdx.x % (kR / 2)) >= Lq * a.G) return;  // both rows empty (uniform)
   const bool row_ok = row < Lq * a.G;
   if (!row_ok) --row;  // an odd row count: the spare half wave rereads the last row
   const int tok = row / a.G;
   const int head = kvh * a.G + row % a.G;
-  uint16_t* op = a.p.out + (int64_t)(first_row<DECODE>(a, s) + tok) * a.p.out_stride_tok +
+  uint16_t* op = a.p.out + (int64_t)(first_row<UNIFORM>(a, s) + tok) * a.p.out_stride_tok +
                  (int64_t)head * a.p.out_stride_head + d0;
   const int2 desc = *reinterpret_cast<const int2*>(a.desc + 2 * (s * a.p.num_kv_heads + kvh));
   if (desc.x < 0) {  // uniform over the workgroup
@@ -637,11 +637,11 @@ __global__ __launch_bounds__(64 * kSqSlices) void short_query_combine_sliced_ker
 }
 
 // Waves of the grid: as many as the step's chunks can use, by its static bound
-// (decode form: one chunk each, the varlen form's workspace holds two).
-int sq_waves(int batch, int64_t max_keys, int num_kv_heads, bool decode) {
+// (uniform form: one chunk each, the varlen form's workspace holds two).
+int sq_waves(int batch, int64_t max_keys, int num_kv_heads, bool uniform_q) {
   const int64_t chunks = (max_keys + kCK - 1) / kCK;
   const int64_t t_max = chunks * batch * num_kv_heads;
-  int64_t wgs = (t_max / (decode ? 1 : kMinChunks) + kWavesPerWG - 1) / kWavesPerWG;
+  int64_t wgs = (t_max / (uniform_q ? 1 : kMinChunks) + kWavesPerWG - 1) / kWavesPerWG;
   if (wgs > kMaxWGs) wgs = kMaxWGs;
   if (wgs < 1) wgs = 1;
   return (int)wgs * kWavesPerWG;
@@ -670,11 +670,13 @@ bool short_query_decode_applies(int block_size, int num_blocks, int num_q_heads,
   return G <= kR && (G > kDecodeKernelGroup || (G == 1 && batch > kDecodeKernelBatch));
 }
 
-size_t short_query_ws_bytes(int batch, int64_t max_keys, int num_q_heads, int num_kv_heads) {
-  (void)num_q_heads;
+size_t short_query_ws_bytes(int batch, int64_t max_keys, int num_q_heads, int num_kv_heads,
+                            int n_query) {
   if (batch <= 0 || num_kv_heads <= 0 || max_keys <= 0) return 0;
+  const int rows = n_query > 0 ? n_query * (num_q_heads / num_kv_heads) : kR;
   return sq_desc_bytes(batch, num_kv_heads) +
-         (size_t)sq_waves(batch, max_keys, num_kv_heads, false) * 2 * kR * kRec * sizeof(float);
+         (size_t)sq_waves(batch, max_keys, num_kv_heads, n_query > 0) * 2 * rows * kRec *
+             sizeof(float);
 }
 
 int short_query_launch(const ShortQueryParams& p, int64_t max_keys, void* ws, hipStream_t s) {
@@ -694,30 +696,95 @@ int short_query_launch(const ShortQueryParams& p, int64_t max_keys, void* ws, hi
   // trip less per chunk).  Bound from the static sizes.
   const int64_t chunks_bound = (max_keys + kCK - 1) / kCK * p.batch * p.num_kv_heads;
   const bool klds = chunks_bound >= (int64_t)kKldsMinChunks * a.n_waves;
-  const bool decode = p.context_lens != nullptr;
-  a.rec_rows = decode ? a.G : kR;
+  const bool uniform_q = p.context_lens != nullptr;
+  a.rec_rows = uniform_q ? p.n_query * a.G : kR;
   // At least 32 waves per (sequence, kv head) group: its parts are folded in
   // slices.
   const bool sliced = a.n_waves >= 32 * (int64_t)p.batch * p.num_kv_heads;
-  auto launch = [&](auto f16, auto dec) {
-    constexpr bool F16 = decltype(f16)::value, DECODE = decltype(dec)::value;
+  auto launch = [&](auto f16, auto uni) {
+    constexpr bool F16 = decltype(f16)::value, UNIFORM = decltype(uni)::value;
     const dim3 grid(a.n_waves / kWavesPerWG), block(64 * kWavesPerWG);
-    if (klds) hipLaunchKernelGGL((short_query_kernel<F16, true, DECODE>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((short_query_kernel<F16, false, DECODE>), grid, block, 0, s, a);
+    if (klds) hipLaunchKernelGGL((short_query_kernel<F16, true, UNIFORM>), grid, block, 0, s, a);
+    else hipLaunchKernelGGL((short_query_kernel<F16, false, UNIFORM>), grid, block, 0, s, a);
     const int st = nvk_launch_status();
     if (st != NVK_OK) return st;
-    // thread / row ranges: rows of the records only (decode: G of kR)
+    // rows of the records only
     const int rows = a.rec_rows;
     if (sliced)
-      hipLaunchKernelGGL((short_query_combine_sliced_kernel<F16, DECODE>),
+      hipLaunchKernelGGL((short_query_combine_sliced_kernel<F16, UNIFORM>),
                          dim3(p.num_kv_heads * (kR / 2), p.batch), dim3(64 * kSqSlices), 0, s, a);
     else
-      hipLaunchKernelGGL((short_query_combine_kernel<F16, DECODE>), dim3(p.num_kv_heads, p.batch),
+      hipLaunchKernelGGL((short_query_combine_kernel<F16, UNIFORM>), dim3(p.num_kv_heads, p.batch),
                          dim3(32 * rows), 0, s, a);
     return nvk_launch_status();
   };
-  if (p.f16) return decode ? launch(std::true_type{}, std::true_type{})
-                           : launch(std::true_type{}, std::false_type{});
-  return decode ? launch(std::false_type{}, std::true_type{})
-                : launch(std::false_type{}, std::false_type{});
+  if (p.f16) return uniform_q ? launch(std::true_type{}, std::true_type{})
+                              : launch(std::true_type{}, std::false_type{});
+  return uniform_q ? launch(std::false_type{}, std::true_type{})
+                   : launch(std::false_type{}, std::false_type{});
+}
+
+extern "C" size_t nvk_paged_verify_workspace_size(int32_t batch, int32_t n_query,
+                                                  int32_t num_q_heads, int32_t num_kv_heads,
+                                                  int32_t head_dim, int32_t block_size,
+                                                  int32_t max_blocks) {
+  if (n_query <= 0 || max_blocks <= 0 ||
+      !short_query_applies(true, block_size, n_query, num_q_heads, num_kv_heads, head_dim, batch))
+    return 0;
+  const int G = num_q_heads / num_kv_heads;
+  if (G != 1 && G != 2 && G != 4 && G != 8) return 0;
+  return short_query_ws_bytes(batch, (int64_t)block_size * max_blocks, num_q_heads, num_kv_heads,
+                              n_query);
+}
+
+extern "C" int nvk_paged_verify(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
+                                const void* k_cache, const void* v_cache,
+                                const int32_t* block_tables, int64_t bt_stride,
+                                const int32_t* context_lens, int32_t batch, int32_t n_query,
+                                int32_t num_q_heads, int32_t num_kv_heads, int32_t head_dim,
+                                int32_t block_size, int32_t max_blocks, int32_t num_blocks,
+                                float scale, void* out, int64_t out_stride_tok,
+                                int64_t out_stride_head, void* workspace,
+                                size_t workspace_bytes, int32_t dtype, void* stream) {
+  if (batch < 0 || n_query <= 0 || num_q_heads <= 0 || num_kv_heads <= 0 || block_size <= 0 ||
+      max_blocks <= 0 || num_blocks < 0)
+    return NVK_EINVAL;
+  if (!(scale > 0.f)) return NVK_EINVAL;
+  if (dtype != NVK_DTYPE_BF16 && dtype != NVK_DTYPE_F16) return NVK_EUNSUPPORTED;
+  if (num_q_heads % num_kv_heads) return NVK_EINVAL;
+  if (batch == 0) return NVK_OK;
+  const size_t need = nvk_paged_verify_workspace_size(batch, n_query, num_q_heads, num_kv_heads,
+                                                      head_dim, block_size, max_blocks);
+  if (need == 0 || num_blocks == 0) return NVK_EUNSUPPORTED;
+  if (!q || !k_cache || !v_cache || !block_tables || !context_lens || !out) return NVK_EINVAL;
+  if (bt_stride < max_blocks || (int64_t)num_kv_heads * HD >= (1 << 23)) return NVK_EINVAL;
+  if ((int64_t)batch * n_query > INT32_MAX) return NVK_EINVAL;
+  if (((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16) return NVK_EALIGN;
+  if ((q_stride_tok % 8) || (q_stride_head % 8)) return NVK_EALIGN;
+  if (((uintptr_t)out % 8) || (out_stride_tok % 4) || (out_stride_head % 4)) return NVK_EALIGN;
+  if (!workspace || workspace_bytes < need) return NVK_EWORKSPACE;
+  if ((uintptr_t)workspace % 256) return NVK_EALIGN;
+  ShortQueryParams p{};
+  p.q = static_cast<const uint16_t*>(q);
+  p.q_stride_tok = q_stride_tok;
+  p.q_stride_head = q_stride_head;
+  p.k_cache = static_cast<const uint16_t*>(k_cache);
+  p.v_cache = static_cast<const uint16_t*>(v_cache);
+  p.context_lens = context_lens;
+  p.n_query = n_query;
+  p.batch = batch;
+  p.block_tables = block_tables;
+  p.bt_stride = bt_stride;
+  p.max_blocks = max_blocks;
+  p.block_size = block_size;
+  p.num_blocks = num_blocks;
+  p.num_q_heads = num_q_heads;
+  p.num_kv_heads = num_kv_heads;
+  p.scale = scale;
+  p.out = static_cast<uint16_t*>(out);
+  p.out_stride_tok = out_stride_tok;
+  p.out_stride_head = out_stride_head;
+  p.f16 = dtype == NVK_DTYPE_F16;
+  return short_query_launch(p, (int64_t)block_size * max_blocks, workspace,
+                            reinterpret_cast<hipStream_t>(stream));
 }

@@ -68,6 +68,12 @@ SIGNATURES = {
                                               _c_i32, _c_i32, _c_ptr, _c_i64, _c_i64, _c_ptr,
                                               _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64,
                                               _c_i32, _c_ptr]),
+    "nvk_paged_verify_workspace_size": (ctypes.c_size_t, [_c_i32, _c_i32, _c_i32, _c_i32, _c_i32,
+                                                          _c_i32, _c_i32]),
+    "nvk_paged_verify": (ctypes.c_int, [_c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i64,
+                                        _c_ptr, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32, _c_i32,
+                                        _c_i32, _c_i32, ctypes.c_float, _c_ptr, _c_i64, _c_i64,
+                                        _c_ptr, ctypes.c_size_t, _c_i32, _c_ptr]),
     "nvk_varlen_prefill_prologue": (ctypes.c_int, [
         _c_ptr, _c_i64, _c_i64, _c_ptr, _c_ptr, _c_ptr, ctypes.c_float, _c_ptr, _c_i64, _c_i64,
         _c_ptr, _c_ptr, _c_ptr, _c_i64, _c_ptr, _c_ptr, _c_ptr, _c_i32, _c_i32, _c_i32, _c_ptr,

@@ -181,6 +181,39 @@ def paged_decode(q, k_cache, v_cache, context_lens, block_table, softmax_scale, 
     return out
 
 
+def _verify(q, k_cache, v_cache, lens, block_table, softmax_scale):
+    """nvk_paged_verify where it applies (few query rows per kv head over paged
+    keys), else None: the caller's general path then runs, and raises what it
+    raises."""
+    b, sq, hq, d = q.shape
+    if (k_cache.dim() != 4 or k_cache.shape != v_cache.shape or not k_cache.is_contiguous()
+            or not v_cache.is_contiguous() or block_table.dim() != 2 or block_table.shape[0] != b
+            or lens.numel() != b or q.stride(-1) != 1):
+        return None
+    num_blocks, block_size, hkv, dk = k_cache.shape
+    if dk != d or num_blocks == 0 or hkv == 0 or hq % hkv:
+        return None
+    dev = _lib.require_gpu(q, k_cache, v_cache, lens, block_table)
+    dtype = _attn_dtype(q, k_cache, v_cache)
+    bt = _int32(block_table)
+    lib = _lib.load()
+    ws_bytes = lib.nvk_paged_verify_workspace_size(b, sq, hq, hkv, d, block_size, bt.shape[1])
+    if ws_bytes == 0:
+        return None
+    qf = q.reshape(b * sq, hq, d)
+    out = torch.empty((b, sq, hq, d), dtype=q.dtype, device=dev)
+    scale = float(softmax_scale) if softmax_scale is not None else d ** -0.5
+    ws = _lib.workspace(dev, ws_bytes)
+    with torch.cuda.device(dev):
+        code = lib.nvk_paged_verify(
+            qf.data_ptr(), qf.stride(0), qf.stride(1), k_cache.data_ptr(), v_cache.data_ptr(),
+            bt.data_ptr(), bt.stride(0), lens.data_ptr(), b, sq, hq, hkv, d, block_size,
+            bt.shape[1], num_blocks, scale, out.data_ptr(), out.stride(1), out.stride(2),
+            _lib.ptr(ws), ws_bytes, dtype, _lib.stream_ptr(dev))
+    _lib.check(code)
+    return out
+
+
 def flash_attn_varlen_func(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, max_seqlen_k,
                            dropout_p=0.0, softmax_scale=None, causal=False, window_size=(-1, -1),
                            softcap=0.0, alibi_slopes=None, deterministic=False,
@@ -229,6 +262,9 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=None
     if not causal:
         raise NotImplementedError("nanovllm_amd: seqlen_q > 1 needs causal=True")
     lens = _int32(cache_seqlens)
+    out = _verify(q, k_cache, v_cache, lens, block_table, softmax_scale)
+    if out is not None:
+        return out
     cu = torch.empty(2, b + 1, dtype=torch.int32, device=dev)   # cu_seqlens_q, cu_seqlens_k
     with torch.cuda.device(dev):
         code = _lib.load().nvk_uniform_cu_seqlens(lens.data_ptr(), b, sq, cu[0].data_ptr(),
