@@ -12,6 +12,7 @@ valid inside the library.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 
@@ -159,7 +160,16 @@ def require_gpu(*tensors: torch.Tensor) -> torch.device:
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle on `device` (without building a Stream object)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
+
+
+_NO_SWITCH = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """``torch.cuda.device(device)``, or nothing where it is current already."""
+    return _NO_SWITCH if torch.cuda.current_device() == device.index else torch.cuda.device(device)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -190,10 +200,10 @@ def workspace(device: torch.device, nbytes: int) -> torch.Tensor | None:
     blocks."""
     if nbytes <= 0:
         return None
-    with torch.cuda.device(device):
+    with on_device(device):
         if torch.cuda.is_current_stream_capturing():
             return torch.empty(nbytes, dtype=torch.uint8, device=device)
-    key = (device.index, torch.cuda.current_stream(device).cuda_stream)
+    key = (device.index, stream_ptr(device))
     buf = _workspaces.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = torch.empty(nbytes, dtype=torch.uint8, device=device)

@@ -63,7 +63,7 @@ def prefill_tile_order(cu_seqlens_q, cu_seqlens_k, max_seqlen_q, k, num_q_heads,
     if nbytes == 0:
         return None
     order = torch.empty(nbytes // 4, dtype=torch.int32, device=dev)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         code = lib.nvk_prefill_tile_order(cu_q.data_ptr(), cu_k.data_ptr(), batch,
                                           int(max_seqlen_q), mk, num_q_heads, hkv, bs,
                                           order.data_ptr(), nbytes, _lib.stream_ptr(dev))
@@ -133,7 +133,7 @@ def varlen_prefill(q, k, v, cu_seqlens_q, cu_seqlens_k, max_seqlen_q, softmax_sc
         elif order_bytes < need:
             raise _lib.NvkError(f"order holds {order_bytes} bytes; a prefill of these sizes "
                                 f"needs {need} (rank it with this call's sizes and head counts)")
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         code = lib.nvk_varlen_prefill_ordered(
             q.data_ptr(), q.stride(0), q.stride(1), tq,
             k.data_ptr(), v.data_ptr(), k_st, v_st, kv_sh, total_k,
@@ -171,7 +171,7 @@ def paged_decode(q, k_cache, v_cache, context_lens, block_table, softmax_scale, 
     max_blocks = bt.shape[1]
     ws_bytes = lib.nvk_paged_decode_workspace_size(b, hq, hkv, d, block_size, max_blocks)
     ws = _lib.workspace(dev, ws_bytes)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         code = lib.nvk_paged_decode(
             q.data_ptr(), q.stride(0), q.stride(1), k_cache.data_ptr(), v_cache.data_ptr(),
             bt.data_ptr(), bt.stride(0), lens.data_ptr(), b, hq, hkv, d, block_size, max_blocks,
@@ -204,7 +204,7 @@ def _verify(q, k_cache, v_cache, lens, block_table, softmax_scale):
     out = torch.empty((b, sq, hq, d), dtype=q.dtype, device=dev)
     scale = float(softmax_scale) if softmax_scale is not None else d ** -0.5
     ws = _lib.workspace(dev, ws_bytes)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         code = lib.nvk_paged_verify(
             qf.data_ptr(), qf.stride(0), qf.stride(1), k_cache.data_ptr(), v_cache.data_ptr(),
             bt.data_ptr(), bt.stride(0), lens.data_ptr(), b, sq, hq, hkv, d, block_size,
@@ -266,7 +266,7 @@ def flash_attn_with_kvcache(q, k_cache, v_cache, k=None, v=None, rotary_cos=None
     if out is not None:
         return out
     cu = torch.empty(2, b + 1, dtype=torch.int32, device=dev)   # cu_seqlens_q, cu_seqlens_k
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         code = _lib.load().nvk_uniform_cu_seqlens(lens.data_ptr(), b, sq, cu[0].data_ptr(),
                                                   cu[1].data_ptr(), _lib.stream_ptr(dev))
     _lib.check(code)

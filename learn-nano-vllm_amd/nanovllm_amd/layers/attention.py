@@ -38,7 +38,7 @@ def store_kvcache(key: torch.Tensor, value: torch.Tensor, k_cache: torch.Tensor,
     slots = slots.contiguous()
     cache_slots = k_cache.shape[0] * k_cache.shape[1]
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         code = lib.nvk_kv_store(key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0),
                                 k_cache.data_ptr(), v_cache.data_ptr(), slots.data_ptr(), N, D,
                                 key.element_size(), cache_slots, _lib.stream_ptr(dev))

@@ -116,7 +116,7 @@ def qk_norm_rope_store(positions: torch.Tensor, qkv: torch.Tensor, num_heads: in
     k = torch.empty(T, num_kv_heads, head_dim, dtype=qkv.dtype, device=dev) if return_k else None
     qw, kw = q_norm_weight.contiguous(), k_norm_weight.contiguous()
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         code = lib.nvk_qk_norm_rope_store(
             qkv.data_ptr(), qkv.stride(0), T, pos.data_ptr(), qw.data_ptr(), kw.data_ptr(),
             float(eps), cs.data_ptr(), cs.stride(0), cs.shape[0], num_heads, num_kv_heads, head_dim,
@@ -174,7 +174,7 @@ def paged_decode_with_prologue(positions: torch.Tensor, qkv: torch.Tensor, num_h
     ws_bytes = lib.nvk_paged_decode_workspace_size(B, num_heads, num_kv_heads, head_dim,
                                                    block_size, max_blocks)
     ws = _lib.workspace(dev, ws_bytes)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         code = lib.nvk_paged_decode_prologue(
             qkv.data_ptr(), qkv.stride(0), pos.data_ptr(), qw.data_ptr(), kw.data_ptr(),
             float(eps), cs.data_ptr(), cs.stride(0), cs.shape[0], k_cache.data_ptr(),
@@ -231,7 +231,7 @@ def _prefill_with_prologue(attn, context, positions, qkv, qw, kw, eps, cos_sin_c
     lib = _lib.load()
     ws_bytes = lib.nvk_varlen_prefill_parts_workspace_size(batch, mq, mk, hq, hkv, d)
     ws = _lib.workspace(dev, ws_bytes)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         code = lib.nvk_varlen_prefill_prologue(
             qkv.data_ptr(), qkv.stride(0), T, pos.data_ptr(), qw.data_ptr(), kw.data_ptr(),
             float(eps), cs.data_ptr(), cs.stride(0), cs.shape[0],

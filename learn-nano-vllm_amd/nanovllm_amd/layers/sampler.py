@@ -46,7 +46,7 @@ class Sampler(nn.Module):
         lib = _lib.load()
         ws_bytes = lib.nvk_sample_workspace_size(b, v)
         ws = torch.empty(max(ws_bytes, 1), dtype=torch.uint8, device=dev)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             code = lib.nvk_sample(logits.data_ptr(), logits.stride(0), b, v, _lib.dtype_code(logits),
                                   temps.data_ptr(), _lib.ptr(noise),
                                   noise.stride(0) if noise is not None else 0, seed, offset,
@@ -64,7 +64,7 @@ def last_token_hidden(x: torch.Tensor, cu_seqlens_q: torch.Tensor) -> torch.Tens
     cu = cu.contiguous()
     out = torch.empty(b, x.shape[1], dtype=x.dtype, device=dev)
     lib = _lib.load()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         code = lib.nvk_gather_last_tokens(x.data_ptr(), x.stride(0), cu.data_ptr(), b, x.shape[1],
                                           _lib.dtype_code(x), out.data_ptr(), out.stride(0),
                                           _lib.stream_ptr(dev))
