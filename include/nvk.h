@@ -276,7 +276,8 @@ int nvk_paged_verify(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
  * A prefill layer's prologue and attention in one call: what
  * nvk_qk_norm_rope_store (storing the new k and v at slot_mapping; NULL: no
  * store) followed by nvk_varlen_prefill_ordered on its q give, bit for bit;
- * q needs no memory of its own, it goes through out's rows.
+ * q needs no memory of its own: it goes through out's rows, or (large steps)
+ * every attention workgroup norms and rotates the q rows that it reads.
  *
  * qkv, positions, the norm weights and the cos/sin cache: as in
  * nvk_qk_norm_rope_store, n_tokens = total_q.

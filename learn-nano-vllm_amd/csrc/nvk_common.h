@@ -92,7 +92,12 @@ struct NvkElt<true> {  // f16
   static NVK_DEVICE float hi(uint32_t w) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
   }
-  static NVK_DEVICE float round(float x) { return (float)(_Float16)x; }
+  static NVK_DEVICE float round(float x) {
+    // x is a value rounded to f32: folding its product into v_fma_mixlo_f16
+    // would round once, and differently from one kernel to the next
+    asm("" : "+v"(x));
+    return (float)(_Float16)x;
+  }
   static NVK_DEVICE nvk_f32x16 mfma32x32x16(vec8 a, vec8 b, nvk_f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
   }

@@ -99,4 +99,60 @@ __device__ __forceinline__ nvk_u32x4 norm_rope8(nvk_u32x4 raw, nvk_u32x4 wraw, f
   return norm_rope8_cs<F16>(raw, wraw, eps, v, j);
 }
 
+// One head row in the MFMA operand layout of the prefill kernel: a lane holds
+// chunks 2 ks + half (ks = 0..7, 8 elements each), its partner lane ^ 32 the
+// others.  raw: those chunks, replaced by the normed and rotated ones; w: the
+// norm weights of the same chunks; cs[p]: cos (2) and sin (2) of the 8 dims
+// of chunk 2 p + half, p < 4 (chunk 2 (p + 4) + half, 64 dims further, shares
+// them).  The sums and products are norm_rope8_cs's in the same order, so the
+// bits are the same.  live: false gives zeros.  All 64 lanes must be active.
+template <bool F16>
+__device__ __forceinline__ void norm_rope_frag(nvk_u32x4 (&raw)[8], const nvk_u32x4 (&w)[8],
+                                               const nvk_u32x4 (&cs)[4][4], float eps, bool live) {
+#pragma clang fp contract(off)
+  using E = NvkElt<F16>;
+  float p[8];
+#pragma unroll
+  for (int ks = 0; ks < 8; ++ks) {
+    const uint32_t r4[4] = {raw[ks].x, raw[ks].y, raw[ks].z, raw[ks].w};
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float a = E::lo(r4[i]), b = E::hi(r4[i]);
+      ss += a * a;
+      ss += b * b;
+    }
+    p[ks] = nvk_sum_xor32(ss);  // chunks 2 ks and 2 ks + 1
+  }
+  const float ss = ((p[0] + p[1]) + (p[2] + p[3])) + ((p[4] + p[5]) + (p[6] + p[7]));
+  const float rstd = live ? rsqrtf(ss / (float)kHD + eps) : 0.f;
+  auto normed = [&](int ks, float (&x)[8]) {
+    const uint32_t r4[4] = {raw[ks].x, raw[ks].y, raw[ks].z, raw[ks].w};
+    const uint32_t w4[4] = {w[ks].x, w[ks].y, w[ks].z, w[ks].w};
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float n0 = E::round(E::lo(r4[i]) * rstd), n1 = E::round(E::hi(r4[i]) * rstd);
+      x[2 * i] = E::round(n0 * E::lo(w4[i]));
+      x[2 * i + 1] = E::round(n1 * E::hi(w4[i]));
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    float x1[8], x2[8], y1[8], y2[8];
+    normed(q, x1);
+    normed(q + 4, x2);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float c = __uint_as_float(cs[q][e >> 2][e & 3]);
+      const float s = __uint_as_float(cs[q][2 + (e >> 2)][e & 3]);
+      y1[e] = x1[e] * c - x2[e] * s;
+      y2[e] = x2[e] * c + x1[e] * s;
+    }
+    raw[q] = nvk_u32x4{E::pack2(y1[0], y1[1]), E::pack2(y1[2], y1[3]), E::pack2(y1[4], y1[5]),
+                       E::pack2(y1[6], y1[7])};
+    raw[q + 4] = nvk_u32x4{E::pack2(y2[0], y2[1]), E::pack2(y2[2], y2[3]),
+                           E::pack2(y2[4], y2[5]), E::pack2(y2[6], y2[7])};
+  }
+}
+
 }  // namespace nvk_qk

@@ -27,6 +27,7 @@
 // measured ~10 % faster than 16-row workgroups over the flattened row space,
 // which read the position, slot and cos/sin row once per row group.
 #include "qk_math.h"
+#include "qk_prologue.h"
 
 namespace {
 
@@ -57,6 +58,7 @@ struct PrologueArgs {
   int64_t cos_sin_stride;
   int64_t max_position;
   int num_q_heads, num_kv_heads;
+  int first_row;  // head rows [first_row, Hq + 2 Hkv) are this launch's (0, or Hq: k and v only)
   uint16_t* q_out;
   int64_t q_out_stride_tok, q_out_stride_head;
   uint16_t* k_out;  // may be null
@@ -131,7 +133,7 @@ __global__ __launch_bounds__(16 * kMaxRowGroups) void qk_prologue_kernel(Prologu
   const int64_t t = blockIdx.x;
   const int j = threadIdx.x & (kLanesPerRow - 1);
   const int groups = blockDim.x / kLanesPerRow;
-  const int R = a.num_q_heads + 2 * a.num_kv_heads;
+  const int R = a.num_q_heads + 2 * a.num_kv_heads;  // rows first_row .. R - 1
   int64_t pos = a.positions[t];
   pos = pos < 0 ? 0 : (pos >= a.max_position ? a.max_position - 1 : pos);
   int32_t slot = a.slot_mapping != nullptr ? a.slot_mapping[t] : -1;
@@ -144,8 +146,8 @@ __global__ __launch_bounds__(16 * kMaxRowGroups) void qk_prologue_kernel(Prologu
     cs[3] = *reinterpret_cast<const nvk_u32x4*>(c + kHD / 2 + 4);
   };
   const uint16_t* row0 = a.qkv + t * a.qkv_row_stride + 8 * j;
-  const int g = threadIdx.x / kLanesPerRow;
-  if (groups >= R) {  // one row per row group (small steps): only the loads it needs
+  const int g = a.first_row + threadIdx.x / kLanesPerRow;
+  if (a.first_row + groups >= R) {  // one row per row group (small steps): only the loads it needs
     if (g >= R) return;
     const nvk_u32x4 raw = load_nt(row0 + (int64_t)g * kHD);
     const bool is_q = g < a.num_q_heads, is_k = !is_q && g < a.num_q_heads + a.num_kv_heads;
@@ -190,6 +192,77 @@ __global__ __launch_bounds__(16 * kMaxRowGroups) void qk_prologue_kernel(Prologu
 
 }  // namespace
 
+int qk_prologue_launch(const QkPrologue& p, bool with_q, void* stream) {
+  if (p.n_tokens < 0 || p.num_q_heads <= 0 || p.num_kv_heads <= 0 || !(p.eps >= 0.f))
+    return NVK_EINVAL;
+  if ((p.dtype != NVK_DTYPE_BF16 && p.dtype != NVK_DTYPE_F16) || p.head_dim != kHD)
+    return NVK_EUNSUPPORTED;
+  if (p.n_tokens == 0) return NVK_OK;
+  void* q_out = with_q ? p.q_out : nullptr;
+  if (!p.qkv || !p.positions || !p.q_norm_weight || !p.k_norm_weight || !p.cos_sin ||
+      (with_q && !q_out))
+    return NVK_EINVAL;
+  if (p.max_position <= 0 || p.cos_sin_stride < p.head_dim) return NVK_EINVAL;
+  const int64_t R = (int64_t)p.num_q_heads + 2 * p.num_kv_heads;
+  if (p.qkv_row_stride < R * p.head_dim) return NVK_EINVAL;
+  if (with_q && (p.q_out_stride_head < p.head_dim ||
+                 p.q_out_stride_tok < (int64_t)p.num_q_heads * p.q_out_stride_head))
+    return NVK_EINVAL;
+  if (p.k_out && (p.k_out_stride_head < p.head_dim ||
+                  p.k_out_stride_tok < (int64_t)p.num_kv_heads * p.k_out_stride_head))
+    return NVK_EINVAL;
+  const bool store = p.slot_mapping != nullptr;
+  if (store && (!p.k_cache || !p.v_cache || p.cache_slots < 0)) return NVK_EINVAL;
+  // 16-byte vector access of every row and of the cos/sin rows.
+  if (((uintptr_t)p.qkv | (uintptr_t)q_out | (uintptr_t)p.k_out | (uintptr_t)p.q_norm_weight |
+       (uintptr_t)p.k_norm_weight | (uintptr_t)p.cos_sin | (uintptr_t)p.k_cache |
+       (uintptr_t)p.v_cache) % 16)
+    return NVK_EALIGN;
+  if ((p.qkv_row_stride % 8) ||
+      (with_q && ((p.q_out_stride_tok % 8) || (p.q_out_stride_head % 8))) ||
+      (p.k_out && ((p.k_out_stride_tok % 8) || (p.k_out_stride_head % 8))) ||
+      (p.cos_sin_stride % 4))
+    return NVK_EALIGN;
+  if (p.n_tokens > INT32_MAX || R > 65535) return NVK_EINVAL;
+  if (!with_q && !p.k_out && !store) return NVK_OK;
+  const int rows = (int)R - (with_q ? 0 : p.num_q_heads);
+  const int max_groups = p.n_tokens <= kSmallTokens ? kMaxRowGroups : kMaxGroups;
+  const int groups = rows < max_groups ? rows : max_groups;
+
+  PrologueArgs a;
+  a.qkv = static_cast<const uint16_t*>(p.qkv);
+  a.qkv_row_stride = p.qkv_row_stride;
+  a.n_tokens = p.n_tokens;
+  a.positions = p.positions;
+  a.q_weight = static_cast<const uint16_t*>(p.q_norm_weight);
+  a.k_weight = static_cast<const uint16_t*>(p.k_norm_weight);
+  a.eps = p.eps;
+  a.cos_sin = p.cos_sin;
+  a.cos_sin_stride = p.cos_sin_stride;
+  a.max_position = p.max_position;
+  a.num_q_heads = p.num_q_heads;
+  a.num_kv_heads = p.num_kv_heads;
+  a.first_row = with_q ? 0 : p.num_q_heads;
+  a.q_out = static_cast<uint16_t*>(q_out);
+  a.q_out_stride_tok = p.q_out_stride_tok;
+  a.q_out_stride_head = p.q_out_stride_head;
+  a.k_out = static_cast<uint16_t*>(p.k_out);
+  a.k_out_stride_tok = p.k_out_stride_tok;
+  a.k_out_stride_head = p.k_out_stride_head;
+  a.k_cache = store ? static_cast<uint16_t*>(p.k_cache) : nullptr;
+  a.v_cache = store ? static_cast<uint16_t*>(p.v_cache) : nullptr;
+  a.slot_mapping = store ? p.slot_mapping : nullptr;
+  a.cache_slots = p.cache_slots;
+  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+  if (p.dtype == NVK_DTYPE_F16)
+    hipLaunchKernelGGL(qk_prologue_kernel<true>, dim3((unsigned)p.n_tokens),
+                       dim3(groups * kLanesPerRow), 0, st, a);
+  else
+    hipLaunchKernelGGL(qk_prologue_kernel<false>, dim3((unsigned)p.n_tokens),
+                       dim3(groups * kLanesPerRow), 0, st, a);
+  return nvk_launch_status();
+}
+
 extern "C" int nvk_qk_norm_rope_store(
     const void* qkv, int64_t qkv_row_stride, int64_t n_tokens, const int64_t* positions,
     const void* q_norm_weight, const void* k_norm_weight, float eps, const float* cos_sin_cache,
@@ -197,63 +270,10 @@ extern "C" int nvk_qk_norm_rope_store(
     int32_t head_dim, void* q_out, int64_t q_out_stride_tok, int64_t q_out_stride_head, void* k_out,
     int64_t k_out_stride_tok, int64_t k_out_stride_head, void* k_cache, void* v_cache,
     const int32_t* slot_mapping, int64_t cache_slots, int32_t dtype, void* stream) {
-  if (n_tokens < 0 || num_q_heads <= 0 || num_kv_heads <= 0 || !(eps >= 0.f)) return NVK_EINVAL;
-  if ((dtype != NVK_DTYPE_BF16 && dtype != NVK_DTYPE_F16) || head_dim != kHD)
-    return NVK_EUNSUPPORTED;
-  if (n_tokens == 0) return NVK_OK;
-  if (!qkv || !positions || !q_norm_weight || !k_norm_weight || !cos_sin_cache || !q_out)
-    return NVK_EINVAL;
-  if (max_position <= 0 || cos_sin_row_stride < head_dim) return NVK_EINVAL;
-  const int64_t R = (int64_t)num_q_heads + 2 * num_kv_heads;
-  if (qkv_row_stride < R * head_dim) return NVK_EINVAL;
-  if (q_out_stride_head < head_dim || q_out_stride_tok < (int64_t)num_q_heads * q_out_stride_head)
-    return NVK_EINVAL;
-  if (k_out && (k_out_stride_head < head_dim ||
-                k_out_stride_tok < (int64_t)num_kv_heads * k_out_stride_head))
-    return NVK_EINVAL;
-  const bool store = slot_mapping != nullptr;
-  if (store && (!k_cache || !v_cache || cache_slots < 0)) return NVK_EINVAL;
-  // 16-byte vector access of every row and of the cos/sin rows.
-  if (((uintptr_t)qkv | (uintptr_t)q_out | (uintptr_t)k_out | (uintptr_t)q_norm_weight |
-       (uintptr_t)k_norm_weight | (uintptr_t)cos_sin_cache | (uintptr_t)k_cache |
-       (uintptr_t)v_cache) % 16)
-    return NVK_EALIGN;
-  if ((qkv_row_stride % 8) || (q_out_stride_tok % 8) || (q_out_stride_head % 8) ||
-      (k_out && ((k_out_stride_tok % 8) || (k_out_stride_head % 8))) || (cos_sin_row_stride % 4))
-    return NVK_EALIGN;
-  if (n_tokens > INT32_MAX || R > 65535) return NVK_EINVAL;
-  const int max_groups = n_tokens <= kSmallTokens ? kMaxRowGroups : kMaxGroups;
-  const int groups = R < max_groups ? (int)R : max_groups;
-
-  PrologueArgs a;
-  a.qkv = static_cast<const uint16_t*>(qkv);
-  a.qkv_row_stride = qkv_row_stride;
-  a.n_tokens = n_tokens;
-  a.positions = positions;
-  a.q_weight = static_cast<const uint16_t*>(q_norm_weight);
-  a.k_weight = static_cast<const uint16_t*>(k_norm_weight);
-  a.eps = eps;
-  a.cos_sin = cos_sin_cache;
-  a.cos_sin_stride = cos_sin_row_stride;
-  a.max_position = max_position;
-  a.num_q_heads = num_q_heads;
-  a.num_kv_heads = num_kv_heads;
-  a.q_out = static_cast<uint16_t*>(q_out);
-  a.q_out_stride_tok = q_out_stride_tok;
-  a.q_out_stride_head = q_out_stride_head;
-  a.k_out = static_cast<uint16_t*>(k_out);
-  a.k_out_stride_tok = k_out_stride_tok;
-  a.k_out_stride_head = k_out_stride_head;
-  a.k_cache = store ? static_cast<uint16_t*>(k_cache) : nullptr;
-  a.v_cache = store ? static_cast<uint16_t*>(v_cache) : nullptr;
-  a.slot_mapping = store ? slot_mapping : nullptr;
-  a.cache_slots = cache_slots;
-  hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-  if (dtype == NVK_DTYPE_F16)
-    hipLaunchKernelGGL(qk_prologue_kernel<true>, dim3((unsigned)n_tokens),
-                       dim3(groups * kLanesPerRow), 0, st, a);
-  else
-    hipLaunchKernelGGL(qk_prologue_kernel<false>, dim3((unsigned)n_tokens),
-                       dim3(groups * kLanesPerRow), 0, st, a);
-  return nvk_launch_status();
+  const QkPrologue p = {qkv, qkv_row_stride, n_tokens, positions, q_norm_weight, k_norm_weight, eps,
+                        cos_sin_cache, cos_sin_row_stride, max_position, num_q_heads, num_kv_heads,
+                        head_dim, q_out, q_out_stride_tok, q_out_stride_head, k_out,
+                        k_out_stride_tok, k_out_stride_head, k_cache, v_cache, slot_mapping,
+                        cache_slots, dtype};
+  return qk_prologue_launch(p, true, stream);
 }

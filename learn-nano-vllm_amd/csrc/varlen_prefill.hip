@@ -42,6 +42,8 @@
 #include <type_traits>
 
 #include "nvk_common.h"
+#include "qk_math.h"
+#include "qk_prologue.h"
 #include "short_query.h"
 
 namespace {
@@ -97,6 +99,13 @@ struct PrefillArgs {
   // the packed qkv rows when q shares out's rows.
   const uint16_t* dummy;
   int64_t dummy_stride;
+  // QN: q holds the raw query part of the packed qkv rows; a workgroup norms and
+  // rotates its own rows at the tokens' positions.
+  const int64_t* positions;
+  const uint16_t* q_weight;
+  float eps;
+  const float* cos_sin;
+  int64_t cos_sin_stride, max_position;
 };
 
 // Partial record of one (query tile, part): the unnormalised O^T accumulators
@@ -313,7 +322,7 @@ __device__ __forceinline__ void wait_lds_loads() {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
-template <int G, int MODE, bool F16>
+template <int G, int MODE, bool F16, bool QN>
 __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void varlen_prefill_kernel(PrefillArgs a) {
   constexpr int TQ = kRows / G;  // query tokens per workgroup
   using E = NvkElt<F16>;
@@ -367,15 +376,40 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void varlen_prefill_kernel
   const int head = kvh * G + row % G;
   const bool row_valid = tok >= 0 && tok < Lq;
   vec8 qf[HD / 16];
+  // QN: the raw rows, the norm weights and the cos / sin, loaded here and
+  // applied once the first key tiles are under way
+  nvk_u32x4 q_raw[HD / 16], q_w[HD / 16], q_cs[4][4];
+  bool q_live = false;
   {
     const int64_t qrow = (int64_t)q_row0 + tok;
     const bool ok = row_valid && qrow < a.total_q;
     const uint16_t* qp = a.q + qrow * a.q_stride_tok + (int64_t)head * a.q_stride_head + 8 * half;
+    if constexpr (QN) {
+      int64_t pos = 0;
+      if (ok) pos = a.positions[qrow];
 #pragma unroll
-    for (int ks = 0; ks < HD / 16; ++ks) {
-      nvk_u32x4 w = {0, 0, 0, 0};
-      if (ok) w = *reinterpret_cast<const nvk_u32x4*>(qp + 16 * ks);
-      qf[ks] = __builtin_bit_cast(vec8, w);
+      for (int ks = 0; ks < HD / 16; ++ks) {
+        q_raw[ks] = nvk_u32x4{0, 0, 0, 0};
+        if (ok) q_raw[ks] = *reinterpret_cast<const nvk_u32x4*>(qp + 16 * ks);
+        q_w[ks] = *reinterpret_cast<const nvk_u32x4*>(a.q_weight + 16 * ks + 8 * half);
+      }
+      pos = pos < 0 ? 0 : (pos >= a.max_position ? a.max_position - 1 : pos);
+      const float* c = a.cos_sin + pos * a.cos_sin_stride + 8 * half;
+#pragma unroll
+      for (int p = 0; p < 4; ++p) {
+        q_cs[p][0] = *reinterpret_cast<const nvk_u32x4*>(c + 16 * p);
+        q_cs[p][1] = *reinterpret_cast<const nvk_u32x4*>(c + 16 * p + 4);
+        q_cs[p][2] = *reinterpret_cast<const nvk_u32x4*>(c + 16 * p + HD / 2);
+        q_cs[p][3] = *reinterpret_cast<const nvk_u32x4*>(c + 16 * p + HD / 2 + 4);
+      }
+      q_live = ok;
+    } else {
+#pragma unroll
+      for (int ks = 0; ks < HD / 16; ++ks) {
+        nvk_u32x4 w = {0, 0, 0, 0};
+        if (ok) w = *reinterpret_cast<const nvk_u32x4*>(qp + 16 * ks);
+        qf[ks] = __builtin_bit_cast(vec8, w);
+      }
     }
   }
   const int row_limit = tok + diag;  // last visible key of this row
@@ -864,6 +898,11 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void varlen_prefill_kernel
         issue_load(k1, j, false);
       }
     }
+    if constexpr (QN) {
+      nvk_qk::norm_rope_frag<F16>(q_raw, q_w, q_cs, a.eps, q_live);
+#pragma unroll
+      for (int ks = 0; ks < HD / 16; ++ks) qf[ks] = __builtin_bit_cast(vec8, q_raw[ks]);
+    }
     DmaPlan plan_v = plan_tile(tb + 1, v_stage(1), true, pg[1], ip[1]);
     TileOff toff = tile_off(tb + 2, pg[2], ip[2]);  // aligned paged: tile kt+2 of the step
     DmaPlan plan_k = MODE == kPagedAligned ? plan_at(toff, k_stage(0), false)
@@ -1106,8 +1145,12 @@ __global__ __launch_bounds__(256) void prefill_combine_kernel(PrefillArgs a) {
 template <int G, int MODE, bool F16>
 int launch_mode(const PrefillArgs& a, hipStream_t stream) {
   dim3 grid(a.num_kv_heads, a.batch, a.n_qtiles * a.n_splits);
-  hipLaunchKernelGGL((varlen_prefill_kernel<G, MODE, F16>), grid, dim3(64 * kWaves), 0, stream,
-                     a);
+  if (a.positions)
+    hipLaunchKernelGGL((varlen_prefill_kernel<G, MODE, F16, true>), grid, dim3(64 * kWaves), 0,
+                       stream, a);
+  else
+    hipLaunchKernelGGL((varlen_prefill_kernel<G, MODE, F16, false>), grid, dim3(64 * kWaves), 0,
+                       stream, a);
   if (a.n_splits > 1) {
     const int st = nvk_launch_status();
     if (st != NVK_OK) return st;
@@ -1287,21 +1330,19 @@ size_t order_bytes_for(int32_t batch, int32_t max_seqlen_q, int64_t max_keys, in
   return order_bytes(pairs);
 }
 
-// The prologue of nvk_varlen_prefill_prologue: the arguments of
-// nvk_qk_norm_rope_store that its attention call does not have.
-struct Prologue {
-  const void* qkv;
-  int64_t qkv_row_stride;
-  const int64_t* positions;
-  const void *q_norm_weight, *k_norm_weight;
-  float eps;
-  const float* cos_sin;
-  int64_t cos_sin_stride, max_position;
-  void* k_new;  // dense: the new keys, normed and rotated
-  void *k_store, *v_store;
-  const int32_t* slot_mapping;
-  int64_t cache_slots;
-};
+// Whether the attention workgroups norm and rotate their own q rows, so that
+// q is neither written by the prologue kernel nor read back (8 KiB per token of
+// 16 heads), at ~800 VALU instructions and a round trip for the rotation rows
+// at each workgroup's start.  Measured per pass, q through out's rows / here
+// (eager calls, two layers): 28 prompts of 100-1024 tokens 263.5 / 255.8 us, 32
+// x 100-1024 after a shared 512 402.5 / 390.0, 4 x 4096 (one layer) 335.0 /
+// 329.1, 1 x 4096 230.0 / 223.3, 8 x 100-1024 after 512 145.8 / 143.9; 8
+// prompts of 100-1024 82.1 / 82.6.  Below one round of the workgroup slots the
+// start is exposed, and parts of one tile would repeat the work.
+constexpr int64_t kNormQMinWgs = 512, kNormQMinTokens = 4096;
+bool prefill_norms_q(const SplitPlan& p, int64_t wgs, int64_t tokens) {
+  return p.n_splits == 1 && wgs >= kNormQMinWgs && tokens >= kNormQMinTokens;
+}
 
 int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
                         int64_t total_q, const void* k, const void* v, int64_t k_stride_tok,
@@ -1313,7 +1354,7 @@ int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_he
                         int32_t head_dim, float scale, void* out, int64_t out_stride_tok,
                         int64_t out_stride_head, void* workspace, size_t workspace_bytes,
                         int32_t dtype, void* stream, const int32_t* given_order,
-                        size_t given_order_bytes, const Prologue* pro = nullptr) {
+                        size_t given_order_bytes, const QkPrologue* pro = nullptr) {
   if (batch < 0 || max_seqlen_q < 0 || max_seqlen_k < 0 || num_q_heads <= 0 ||
       num_kv_heads <= 0 || total_q < 0 || total_k < 0)
     return NVK_EINVAL;
@@ -1372,18 +1413,19 @@ int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_he
     if ((uintptr_t)given_order % 4) return NVK_EALIGN;
   }
 
+  const bool norm_q = pro && !short_q && prefill_norms_q(sp, pairs * num_kv_heads, total_q);
   if (pro) {
-    // q goes through out's rows: a workgroup (or, in the short-query kernels, a
-    // wave) overwrites only rows whose q it alone has read, and the rows of
-    // tiles and groups that several of them share are written by the merging
-    // kernel, after all of them.
-    const int st = nvk_qk_norm_rope_store(
-        pro->qkv, pro->qkv_row_stride, total_q, pro->positions, pro->q_norm_weight,
-        pro->k_norm_weight, pro->eps, pro->cos_sin, pro->cos_sin_stride, pro->max_position,
-        num_q_heads, num_kv_heads, head_dim, out, out_stride_tok, out_stride_head, pro->k_new,
-        (int64_t)num_kv_heads * head_dim, head_dim, pro->k_store, pro->v_store, pro->slot_mapping,
-        pro->cache_slots, dtype, stream);
+    // Without norm_q, q goes through out's rows: a workgroup (or, in the
+    // short-query kernels, a wave) overwrites only rows whose q it alone has
+    // read, and the rows of tiles and groups that several of them share are
+    // written by the merging kernel, after all of them.
+    const int st = qk_prologue_launch(*pro, !norm_q, stream);
     if (st != NVK_OK) return st;
+    if (norm_q) {
+      q = pro->qkv;
+      q_stride_tok = pro->qkv_row_stride;
+      q_stride_head = head_dim;
+    }
   }
 
   // Short query ranges (<= 16 rows per kv head) over paged keys: the stream-K
@@ -1461,6 +1503,14 @@ int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_he
       a.order = order;
     }
   }
+  if (norm_q) {
+    a.positions = pro->positions;
+    a.q_weight = static_cast<const uint16_t*>(pro->q_norm_weight);
+    a.eps = pro->eps;
+    a.cos_sin = pro->cos_sin;
+    a.cos_sin_stride = pro->cos_sin_stride;
+    a.max_position = pro->max_position;
+  }
   return dtype == NVK_DTYPE_F16 ? launch_prefill_g<true>(a, G, s) : launch_prefill_g<false>(a, G, s);
 }
 
@@ -1516,11 +1566,19 @@ extern "C" int nvk_varlen_prefill_prologue(
     void* stream) {
   if (num_q_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0) return NVK_EINVAL;
   if (!qkv || (block_tables ? (!k_cache || !v_cache) : !k_new)) return NVK_EINVAL;
-  const Prologue p = {qkv, qkv_row_stride, positions, q_norm_weight, k_norm_weight, eps,
-                      cos_sin_cache, cos_sin_row_stride, max_position,
-                      block_tables ? nullptr : k_new, k_cache, v_cache, slot_mapping, cache_slots};
-  // dense: the step's own keys and the v part of qkv
   const int64_t k_row = (int64_t)num_kv_heads * head_dim;
+  const QkPrologue p = {qkv, qkv_row_stride, total_q, positions, q_norm_weight, k_norm_weight, eps,
+                        cos_sin_cache, cos_sin_row_stride, max_position, num_q_heads, num_kv_heads,
+                        head_dim, out, out_stride_tok, out_stride_head,
+                        block_tables ? nullptr : k_new, k_row, head_dim, k_cache, v_cache,
+                        slot_mapping, cache_slots, dtype};
+  // as the step's q would be checked, whichever way it goes
+  if (((uintptr_t)qkv | (uintptr_t)out) % 16 || qkv_row_stride % 8 || out_stride_tok % 8 ||
+      out_stride_head % 8)
+    return NVK_EALIGN;
+  if (out_stride_head < head_dim || out_stride_tok < (int64_t)num_q_heads * out_stride_head)
+    return NVK_EINVAL;
+  // dense: the step's own keys and the v part of qkv
   const uint16_t* v = static_cast<const uint16_t*>(qkv) + (int64_t)num_q_heads * head_dim + k_row;
   return varlen_prefill_impl(
       out, out_stride_tok, out_stride_head, total_q, block_tables ? k_cache : k_new,

@@ -1,6 +1,7 @@
 """A prefill layer's prologue and attention in one call
 (nvk_varlen_prefill_prologue, the prefill route of attention_with_prologue)
-against the two calls it replaces, bit for bit (q shares the output's rows):
+against the two calls it replaces, bit for bit: large steps, whose workgroups
+norm and rotate their own q rows, and others, whose q shares the output's rows;
 dense, paged, split, ranked and short-query forms, every group size, both
 dtypes, positions outside the rotation table, padding slots, an empty cache and
 a hooked module."""
@@ -48,6 +49,9 @@ CASES = [  # lens_q, cached, hq, hkv, bs
     ([1, 63, 64, 65, 300] * 4 + [40] * 6, [0] * 26, 16, 8, 256),     # ranked tiles
     ([700] * 7 + [1, 33], [256 * i + 7 for i in range(9)], 16, 8, 256),
     ([700] * 7 + [1, 33], [100] * 9, 16, 8, 48),                     # per-row page lookups
+    ([700] * 7, [64] * 7, 16, 4, 64),
+    ([700] * 7, [64 * i for i in range(7)], 16, 2, 128),
+    ([1400] * 3 + [1], [0] * 4, 16, 4, 256),
     ([500] * 5, [300] * 5, 16, 4, 64),
     ([300] * 4, [64] * 4, 16, 2, 128),
     ([600] * 8, [128] * 8, 16, 16, 256),
