@@ -313,12 +313,15 @@ __global__ __launch_bounds__(kPartThreads) void sample_draw_kernel(SampleArgs a)
   float l[32];
   const int first = c * kChunk + tid * 8;
   if (sizeof(T) == 2 && a.vec_ok && (int64_t)(c + 1) * kChunk <= a.vocab) {
-    // a whole chunk of bf16: the kIters 16-byte loads all leave before the first wait
+    // a whole chunk of bf16: the kIters 16-byte loads all leave before the first
+    // wait.  Read once: non-temporal (512 rows 32.2 -> 29.3 us, 64 rows 9.8 ->
+    // 8.9 against cached loads).
     const uint16_t* p = static_cast<const uint16_t*>(a.logits) + (int64_t)row * a.row_stride + first;
     nvk_u32x4 w[kIters];
 #pragma unroll
     for (int it = 0; it < kIters; ++it)
-      w[it] = *reinterpret_cast<const nvk_u32x4*>(p + it * kPartThreads * 8);
+      w[it] = __builtin_nontemporal_load(
+          reinterpret_cast<const nvk_u32x4*>(p + it * kPartThreads * 8));
 #pragma unroll
     for (int it = 0; it < kIters; ++it) {
       const uint32_t ww[4] = {w[it].x, w[it].y, w[it].z, w[it].w};
