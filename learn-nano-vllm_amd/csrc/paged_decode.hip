@@ -628,7 +628,7 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(DecodeArgs a) {
 // output of empty contexts.
 // Merge of one output element over the parts of a cut group: wave p1's head
 // record (slot 0) and the continuation records (slot 1) of waves p1+1 .. p2
-// (every active wave's range holds at least kMinChunks chunks, so each of
+// (every active wave's range holds a chunk at least, so each of
 // them wrote one).  A slice s of S folds parts p1+s, p1+s+S, ...; kBatch
 // parts are fetched per round trip (3 kBatch loads in flight), then folded
 // into (M, L, O).  rec0: the record of wave 0, slot 0, for this thread's kv

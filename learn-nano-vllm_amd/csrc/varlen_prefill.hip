@@ -33,6 +33,10 @@
 //     v_dot2_f32_bf16 over the packed probabilities.
 //   * The grid runs the query tiles nearest the end of each sequence (the
 //     ones with most keys) first.
+//   * Steps whose tiles fill at most half of the workgroup slots are cut along
+//     the keys as well (plan_parts), and merged by a second kernel.
+//   * In large steps the workgroup applies the q norm and rotation of the layer's
+//     prologue to its own rows (QN, prefill_norms_q).
 //   * The normalised output rows go back through LDS (each wave's 32 rows in
 //     the K stages, free in a range's last step), so each store writes four
 //     whole 256-byte rows.  Stored straight from the accumulator layout, a
@@ -1181,7 +1185,7 @@ int launch_prefill_g(const PrefillArgs& a, int G, hipStream_t s) {
 }
 
 
-// Split-K plan for a launch.  Deterministic in its arguments, so the workspace
+// Split-K plan of a launch.  Deterministic in its arguments, so the workspace
 // queries and the launch agree.
 struct SplitPlan {
   int n_qtiles, n_splits, tiles_per_split;

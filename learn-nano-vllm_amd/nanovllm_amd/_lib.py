@@ -161,7 +161,8 @@ def require_gpu(*tensors: torch.Tensor) -> torch.device:
 
 def stream_ptr(device: torch.device) -> int:
     """The current stream's handle on `device` (without building a Stream object)."""
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    index = torch.cuda.current_device() if device.index is None else device.index
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 _NO_SWITCH = contextlib.nullcontext()
@@ -169,7 +170,8 @@ _NO_SWITCH = contextlib.nullcontext()
 
 def on_device(device: torch.device):
     """``torch.cuda.device(device)``, or nothing where it is current already."""
-    return _NO_SWITCH if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+    current = device.index is None or device.index == torch.cuda.current_device()
+    return _NO_SWITCH if current else torch.cuda.device(device)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
