@@ -406,7 +406,10 @@ int nvk_qk_norm_rope_store(const void* qkv, int64_t qkv_row_stride, int64_t n_to
  * registers for key context_lens[b] - 1, which must be that cache row (as
  * model_runner.prepare_decode builds it: slot = the row of position
  * len - 1, context_lens = len); a sequence of context length 0 (a graph
- * padding row) stores nothing.  Output, caches, block tables, context
+ * padding row) stores nothing.  With 4 or 8 query heads per kv head (and, from
+ * 33 sequences up, with one) the prologue runs as a kernel of its own, q passing
+ * through out's rows, and key context_lens[b] - 1 is read back from the cache.
+ * Output, caches, block tables, context
  * lengths, workspace (nvk_paged_decode_workspace_size) and empty contexts as
  * in nvk_paged_decode; norm weights, eps, cos_sin_cache and positions as in
  * nvk_qk_norm_rope_store.  The result equals the two calls' bit for bit.

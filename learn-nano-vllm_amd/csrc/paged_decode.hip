@@ -53,6 +53,7 @@
 
 #include "nvk_common.h"
 #include "qk_math.h"
+#include "qk_prologue.h"
 #include "short_query.h"
 
 namespace {
@@ -1143,11 +1144,11 @@ extern "C" int nvk_paged_decode_prologue(
   if (short_query_decode_applies(block_size, num_blocks, num_q_heads, num_kv_heads, head_dim,
                                  batch) &&
       out_stride_head >= head_dim && out_stride_tok >= (int64_t)num_q_heads * out_stride_head) {
-    const int st = nvk_qk_norm_rope_store(
-        qkv, qkv_row_stride, batch, positions, q_norm_weight, k_norm_weight, eps, cos_sin_cache,
-        cos_sin_row_stride, max_position, num_q_heads, num_kv_heads, head_dim, out,
-        out_stride_tok, out_stride_head, nullptr, 0, 0, k_cache, v_cache, slot_mapping,
-        cache_slots, dtype, stream);
+    const QkPrologue p = {qkv, qkv_row_stride, batch, positions, q_norm_weight, k_norm_weight, eps,
+                          cos_sin_cache, cos_sin_row_stride, max_position, num_q_heads,
+                          num_kv_heads, head_dim, out, out_stride_tok, out_stride_head, nullptr, 0,
+                          0, k_cache, v_cache, slot_mapping, cache_slots, dtype, context_lens};
+    const int st = qk_prologue_launch(p, true, stream);
     if (st != NVK_OK) return st;
     a.q = a.out;
     a.q_stride_tok = out_stride_tok;

@@ -22,6 +22,8 @@ struct QkPrologue {
   const int32_t* slot_mapping;  // null: no store
   int64_t cache_slots;
   int32_t dtype;
+  // decode steps: tokens whose context length is 0 (graph padding) store nothing; null: unused
+  const int32_t* context_lens = nullptr;
 };
 
 // Checks the arguments and launches.  with_q false: the q rows are left to the

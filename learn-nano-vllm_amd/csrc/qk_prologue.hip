@@ -67,6 +67,7 @@ struct PrologueArgs {
   uint16_t* v_cache;
   const int32_t* slot_mapping;
   int64_t cache_slots;
+  const int32_t* context_lens;  // null, or: a token of context length <= 0 stores nothing
 };
 
 // The qkv rows are read once and every output row (q, k, cache rows) written
@@ -138,6 +139,7 @@ __global__ __launch_bounds__(16 * kMaxRowGroups) void qk_prologue_kernel(Prologu
   pos = pos < 0 ? 0 : (pos >= a.max_position ? a.max_position - 1 : pos);
   int32_t slot = a.slot_mapping != nullptr ? a.slot_mapping[t] : -1;
   if ((int64_t)slot >= a.cache_slots) slot = -1;
+  if (a.context_lens != nullptr && a.context_lens[t] <= 0) slot = -1;
   const float* c = a.cos_sin + pos * a.cos_sin_stride + 8 * (j & 7);
   auto load_cs = [&](nvk_u32x4 (&cs)[4]) {
     cs[0] = *reinterpret_cast<const nvk_u32x4*>(c);
@@ -253,6 +255,7 @@ int qk_prologue_launch(const QkPrologue& p, bool with_q, void* stream) {
   a.v_cache = store ? static_cast<uint16_t*>(p.v_cache) : nullptr;
   a.slot_mapping = store ? p.slot_mapping : nullptr;
   a.cache_slots = p.cache_slots;
+  a.context_lens = p.context_lens;
   hipStream_t st = reinterpret_cast<hipStream_t>(stream);
   if (p.dtype == NVK_DTYPE_F16)
     hipLaunchKernelGGL(qk_prologue_kernel<true>, dim3((unsigned)p.n_tokens),
