@@ -16,8 +16,9 @@ further: the decode kernel itself norms and rotates q and the new k, stores
 the new k and v and attends (``nvk_paged_decode_prologue``), one launch
 fewer and q never written.  ``attention_with_prologue`` is the matching
 replacement for the body of ``Qwen3Attention.forward`` up to
-``self.attn(q, k, v)`` and takes the decode-step form for batches of up to
-``FUSED_DECODE_MAX_BATCH`` sequences.
+``self.attn(q, k, v)``: it takes the decode-step form for batches of up to
+``FUSED_DECODE_MAX_BATCH`` sequences, and in prefill steps one call that runs
+prologue and attention (``nvk_varlen_prefill_prologue``).
 """
 from __future__ import annotations
 

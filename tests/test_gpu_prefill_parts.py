@@ -3,7 +3,6 @@ along the keys (the workspace of nvk_varlen_prefill_parts_workspace_size), then
 merged.  The parts' result is checked against the oracle and against the same
 call without a workspace, at sizes on both sides of the rule, with tiles that
 keep one part beside cut ones, partly empty first tiles and ragged batches."""
-import numpy as np
 import pytest
 import torch
 

@@ -3,7 +3,6 @@ nvk_paged_verify (lengths read as they are, no cu_seqlens) against the oracle an
 against the varlen call over explicit cu_seqlens: rows up to the kernels' 16,
 contexts at chunk and page edges, shorter than the query block or empty, one and
 two chunks per wave, K through LDS, strided q."""
-import numpy as np
 import pytest
 import torch
 
