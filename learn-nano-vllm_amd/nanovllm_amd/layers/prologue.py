@@ -196,6 +196,16 @@ def _hooked(m: torch.nn.Module) -> bool:
                 or mod._global_backward_pre_hooks)
 
 
+def _caches_fit(attn, dtype: torch.dtype) -> bool:
+    """Whether the module's caches are paged keys and values as the one-call
+    prefill reads them.  Others take the two calls, whose checks refuse them
+    (or accept them: without slots, caches of another head count)."""
+    k, v = attn.k_cache, attn.v_cache
+    return (k.dim() == 4 and k.shape == v.shape and k.shape[2] == attn.num_kv_heads
+            and k.shape[3] == attn.head_dim and k.dtype == v.dtype == dtype
+            and k.is_contiguous() and v.is_contiguous())
+
+
 def _prefill_with_prologue(attn, context, positions, qkv, qw, kw, eps, cos_sin_cache, store):
     """A prefill step's prologue and attention in one library call
     (``nvk_varlen_prefill_prologue``): the results of ``qk_norm_rope_store``
@@ -217,8 +227,6 @@ def _prefill_with_prologue(attn, context, positions, qkv, qw, kw, eps, cos_sin_c
     out = torch.empty((T, hq, d), dtype=qkv.dtype, device=dev)
     if bt is not None:
         keys, k_new = attn.k_cache, None
-        if not (keys.is_contiguous() and attn.v_cache.is_contiguous()):
-            raise _lib.NvkError("paged k/v must be contiguous [num_blocks, block_size, Hkv, D] caches")
         bt = _int32(bt)
         if bt.dim() != 2 or bt.shape[0] != batch:
             raise _lib.NvkError("block_table must be [batch, max_blocks]")
@@ -265,7 +273,8 @@ def attention_with_prologue(attn, positions: torch.Tensor, qkv: torch.Tensor, q_
             context.slot_mapping, context.context_lens, context.block_tables,
             attn.scale).unsqueeze(1)
     if (context.is_prefill and context.max_seqlen_q > 0 and type(attn) is Attention
-            and (store or context.block_tables is None) and not _hooked(attn)):
+            and (context.block_tables is None or (store and _caches_fit(attn, qkv.dtype)))
+            and not _hooked(attn)):
         return _prefill_with_prologue(attn, context, positions, qkv, q_norm.weight, k_norm.weight,
                                       q_norm.eps, rotary_emb.cos_sin_cache, store)
     # k itself is read only by the dense (no block table) prefill
