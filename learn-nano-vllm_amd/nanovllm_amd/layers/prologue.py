@@ -187,13 +187,18 @@ def paged_decode_with_prologue(positions: torch.Tensor, qkv: torch.Tensor, num_h
     return out
 
 
-def _hooked(m: torch.nn.Module) -> bool:
-    """Whether calling the module runs more than its forward."""
+_FORWARD = Attention.forward
+
+
+def _calls_more(m: Attention) -> bool:
+    """Whether calling the module runs anything but ``Attention.forward``: hooks,
+    a forward replaced on the instance or on the class, a compiled call."""
     mod = torch.nn.modules.module
     return bool(m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
                 or m._backward_pre_hooks or mod._global_forward_hooks
                 or mod._global_forward_pre_hooks or mod._global_backward_hooks
-                or mod._global_backward_pre_hooks)
+                or mod._global_backward_pre_hooks or "forward" in m.__dict__
+                or Attention.forward is not _FORWARD or m._compiled_call_impl is not None)
 
 
 def _caches_fit(attn, dtype: torch.dtype) -> bool:
@@ -274,7 +279,7 @@ def attention_with_prologue(attn, positions: torch.Tensor, qkv: torch.Tensor, q_
             attn.scale).unsqueeze(1)
     if (context.is_prefill and context.max_seqlen_q > 0 and type(attn) is Attention
             and (context.block_tables is None or (store and _caches_fit(attn, qkv.dtype)))
-            and not _hooked(attn)):
+            and not _calls_more(attn)):
         return _prefill_with_prologue(attn, context, positions, qkv, q_norm.weight, k_norm.weight,
                                       q_norm.eps, rotary_emb.cos_sin_cache, store)
     # k itself is read only by the dense (no block table) prefill

@@ -89,3 +89,27 @@ def test_caches_of_another_head_count_are_read_as_they_are(calls):
     """Without slots nothing is stored and the caches' own head count holds."""
     attention_with_prologue(*_args(_zeros(4, PAGE, 4, D), _zeros(4, PAGE, 4, D), slots=False))
     assert calls == TWO
+
+
+@pytest.mark.parametrize("where", ["instance", "class"])
+def test_a_replaced_forward_runs(calls, monkeypatch, where):
+    """attention_with_prologue returns what the call of the module returns, also
+    where its forward was replaced (the way some libraries attach hooks)."""
+    args = _args()
+    attn, inner = args[0], Attention.forward
+    if where == "instance":
+        attn.forward = lambda *a, **kw: (inner(attn, *a, **kw), "seen")
+    else:
+        monkeypatch.setattr(Attention, "forward", lambda *a, **kw: (inner(*a, **kw), "seen"))
+    out, mark = attention_with_prologue(*args)
+    assert mark == "seen" and calls == TWO and out.shape == (T, HQ, D)
+
+
+def test_a_compiled_module_is_called(calls):
+    args = _args()
+    attn, called = args[0], []
+    attn.compile(backend="eager")
+    assert attn._compiled_call_impl is not None
+    attn._compiled_call_impl = lambda *a, **kw: called.append(1) or attn._call_impl(*a, **kw)
+    attention_with_prologue(*args)
+    assert called == [1] and calls == TWO
