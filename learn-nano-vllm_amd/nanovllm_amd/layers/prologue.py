@@ -229,6 +229,7 @@ def _prefill_with_prologue(attn, context, positions, qkv, qw, kw, eps, cos_sin_c
     if cu_k.numel() != batch + 1:
         raise _lib.NvkError("cu_seqlens_q and cu_seqlens_k disagree on the batch size")
     mq = int(context.max_seqlen_q)
+    scale = float(attn.scale) if attn.scale is not None else d ** -0.5
     out = torch.empty((T, hq, d), dtype=qkv.dtype, device=dev)
     if bt is not None:
         keys, k_new = attn.k_cache, None
@@ -252,7 +253,7 @@ def _prefill_with_prologue(attn, context, positions, qkv, qw, kw, eps, cos_sin_c
             attn.k_cache.data_ptr() if store else None, attn.v_cache.data_ptr() if store else None,
             _lib.ptr(slots), cache_slots, _lib.ptr(k_new), cu_q.data_ptr(), cu_k.data_ptr(), batch,
             mq, mk, _lib.ptr(bt), bt_stride, max_blocks, block_size, num_blocks, hq, hkv, d,
-            float(attn.scale), out.data_ptr(), out.stride(0), out.stride(1), _lib.ptr(ws),
+            scale, out.data_ptr(), out.stride(0), out.stride(1), _lib.ptr(ws),
             ws_bytes, _lib.ptr(order), order.numel() * 4 if order is not None else 0,
             _lib.dtype_code(qkv), _lib.stream_ptr(dev))
     _lib.check(code)

@@ -113,3 +113,8 @@ def test_a_compiled_module_is_called(calls):
     attn._compiled_call_impl = lambda *a, **kw: called.append(1) or attn._call_impl(*a, **kw)
     attention_with_prologue(*args)
     assert called == [1] and calls == TWO
+
+
+def test_no_scale_is_the_default_scale(calls):
+    out = attention_with_prologue(*_args(scale=None))
+    assert calls == ONE and out.shape == (T, HQ, D)
