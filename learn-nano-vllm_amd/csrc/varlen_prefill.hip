@@ -1368,7 +1368,8 @@ int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_he
   if (num_q_heads % num_kv_heads) return NVK_EINVAL;
   const int G = num_q_heads / num_kv_heads;
   if (G != 1 && G != 2 && G != 4 && G != 8) return NVK_EUNSUPPORTED;
-  if (batch == 0 || max_seqlen_q == 0) return NVK_OK;
+  if (batch == 0 || max_seqlen_q == 0)  // no query: k and v are still stored
+    return pro ? qk_prologue_launch(*pro, false, stream) : NVK_OK;
   if (!q || !k || !v || !cu_seqlens_q || !cu_seqlens_k || !out) return NVK_EINVAL;
   if (block_tables) {
     if (block_size <= 0 || max_blocks <= 0 || num_blocks < 0 || bt_stride < max_blocks)
@@ -1569,7 +1570,8 @@ extern "C" int nvk_varlen_prefill_prologue(
     size_t workspace_bytes, const int32_t* order, size_t order_bytes_, int32_t dtype,
     void* stream) {
   if (num_q_heads <= 0 || num_kv_heads <= 0 || head_dim <= 0) return NVK_EINVAL;
-  if (!qkv || (block_tables ? (!k_cache || !v_cache) : !k_new)) return NVK_EINVAL;
+  if (total_q != 0 && (!qkv || (block_tables ? (!k_cache || !v_cache) : !k_new)))
+    return NVK_EINVAL;
   const int64_t k_row = (int64_t)num_kv_heads * head_dim;
   const QkPrologue p = {qkv, qkv_row_stride, total_q, positions, q_norm_weight, k_norm_weight, eps,
                         cos_sin_cache, cos_sin_row_stride, max_position, num_q_heads, num_kv_heads,
@@ -1583,7 +1585,8 @@ extern "C" int nvk_varlen_prefill_prologue(
   if (out_stride_head < head_dim || out_stride_tok < (int64_t)num_q_heads * out_stride_head)
     return NVK_EINVAL;
   // dense: the step's own keys and the v part of qkv
-  const uint16_t* v = static_cast<const uint16_t*>(qkv) + (int64_t)num_q_heads * head_dim + k_row;
+  const uint16_t* v =
+      qkv ? static_cast<const uint16_t*>(qkv) + (int64_t)num_q_heads * head_dim + k_row : nullptr;
   return varlen_prefill_impl(
       out, out_stride_tok, out_stride_head, total_q, block_tables ? k_cache : k_new,
       block_tables ? v_cache : v, k_row, qkv_row_stride, head_dim, total_q, cu_seqlens_q,

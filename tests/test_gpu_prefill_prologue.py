@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from gpu_utils import say
-from nanovllm_amd import (Attention, attention_with_prologue, qk_norm_rope_store,
+from nanovllm_amd import (Attention, _lib, attention_with_prologue, qk_norm_rope_store,
                           rope_cos_sin_cache)
 from nanovllm_amd.utils.context import get_context, reset_context, set_context
 from nanovllm_amd.workloads import _Norm, _Rope
@@ -101,3 +101,37 @@ def test_empty_cache_and_hooks():
     finally:
         reset_context()
     assert torch.equal(bare, hooked) and seen == [hooked.shape]
+
+
+@pytest.mark.parametrize("no_query", ["no sequence", "no query bound"])
+def test_tokens_of_no_sequence_are_stored(no_query):
+    """As by the two calls: the prologue does not look at the sequences."""
+    qkv, w, pos, kc, vc, cs = _step(6, [40], [0], 16, 8, 64, torch.bfloat16, False)
+    slots = get_context().slot_mapping
+    k2, v2 = kc.clone(), vc.clone()
+    norms = _Norm(w[0], EPS), _Norm(w[1], EPS)
+    say(f"prefill with prologue, {no_query}")
+    cu = torch.zeros(1, dtype=torch.int32).cuda()
+    try:
+        if no_query == "no sequence":
+            attn = Attention(16, D, D ** -0.5, 8)
+            attn.k_cache, attn.v_cache = k2, v2
+            set_context(True, cu, cu, 7, 7, slots, None, None)
+            assert attention_with_prologue(attn, pos, qkv, *norms, _Rope(cs)).shape == (40, 16, D)
+        else:
+            k_new, out = torch.empty(40, 8, D, dtype=qkv.dtype).cuda(), torch.empty(
+                40, 16, D, dtype=qkv.dtype).cuda()
+            cu2 = torch.zeros(2, dtype=torch.int32).cuda()
+            cs2 = cs.view(cs.shape[0], -1)
+            _lib.check(_lib.load().nvk_varlen_prefill_prologue(
+                qkv.data_ptr(), qkv.stride(0), 40, pos.data_ptr(), w[0].data_ptr(),
+                w[1].data_ptr(), EPS, cs2.data_ptr(), cs2.stride(0), cs2.shape[0], k2.data_ptr(),
+                v2.data_ptr(), slots.data_ptr(), k2.shape[0] * k2.shape[1], k_new.data_ptr(),
+                cu2.data_ptr(), cu2.data_ptr(), 1, 0, 0, None, 0, 0, 0, 0, 16, 8, D, D ** -0.5,
+                out.data_ptr(), out.stride(0), out.stride(1), None, 0, None, 0,
+                _lib.dtype_code(qkv), _lib.stream_ptr(qkv.device)))
+        qk_norm_rope_store(pos, qkv, 16, 8, D, w[0], w[1], EPS, cs, kc, vc, slots)
+        torch.cuda.synchronize()
+    finally:
+        reset_context()
+    assert torch.equal(k2, kc) and torch.equal(v2, vc)

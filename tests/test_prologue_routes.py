@@ -118,3 +118,25 @@ def test_a_compiled_module_is_called(calls):
 def test_no_scale_is_the_default_scale(calls):
     out = attention_with_prologue(*_args(scale=None))
     assert calls == ONE and out.shape == (T, HQ, D)
+
+
+@pytest.mark.skipif(torch.cuda.is_available(),
+                    reason="passes fake device pointers; only runs where nothing can launch")
+def test_prefill_prologue_without_queries_runs_the_prologue():
+    """A step of no sequence (or no query bound) still stores its k and v, so the
+    prologue's own checks hold there; without tokens there is nothing to do."""
+    lib = _lib.load()
+    # qkv, stride, T, pos, qw, kw, eps, cos_sin, cs_stride, max_pos, k/v cache, slots,
+    # cache_slots, k_new, cu_q, cu_k, batch, max_q, max_k, tables, bt_stride, max_blocks, bs, nb,
+    # heads, D, scale, out, out strides, ws, ws_bytes, order, order_bytes, dtype, stream
+    a = [16, 32 * 128, 4, 16, 16, 16, -1.0, 16, 128, 4096, 16, 16, 16, 1 << 20, 16, 16, 16, 0, 7, 7,
+         None, 0, 0, 0, 0, 16, 8, 128, 0.088, 16, 16 * 128, 128, None, 0, None, 0, 0, None]
+    assert lib.nvk_varlen_prefill_prologue(*a) == -1             # eps < 0, batch 0
+    a[17], a[18] = 2, 0
+    assert lib.nvk_varlen_prefill_prologue(*a) == -1             # eps < 0, max_seqlen_q 0
+    empty = list(a)
+    empty[6] = 1e-6
+    for i in (0, 3, 10, 11, 12, 14, 29):
+        empty[i] = None
+    empty[2] = empty[17] = 0
+    assert lib.nvk_varlen_prefill_prologue(*empty) == 0          # no token, no sequence
