@@ -93,10 +93,12 @@ struct NvkElt<true> {  // f16
     return (float)__builtin_bit_cast(_Float16, (uint16_t)(w >> 16));
   }
   static NVK_DEVICE float round(float x) {
-    // x is a value rounded to f32: folding its product into v_fma_mixlo_f16
-    // would round once, and differently from one kernel to the next
-    asm("" : "+v"(x));
-    return (float)(_Float16)x;
+    // A product becomes v_fma_mixlo_f16 or v_mul_f16, rounded once.  The empty asm
+    // keeps two roundings from being paired (v_cvt_pk_f16_f32, which rounds the
+    // product to f32 first), so that every kernel gives the same bits.
+    _Float16 h = (_Float16)x;
+    asm("" : "+v"(h));
+    return (float)h;
   }
   static NVK_DEVICE nvk_f32x16 mfma32x32x16(vec8 a, vec8 b, nvk_f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);

@@ -8,8 +8,10 @@
 //   x1, x2 = halves of x; cos, sin = halves of cos_sin_cache[pos]
 //   y1 = x1*cos - x2*sin ; y2 = x2*cos + x1*sin ; T(cat(y1, y2))
 // Every f32 product and sum is rounded on its own (no fused multiply-add), as
-// the reference's separate tensor operations do; a product of two T values
-// is formed in f32 and rounded to T, as torch's elementwise kernels do.
+// the reference's separate tensor operations do, but for one: with T = f16
+// x * rsqrt(..) is rounded to f16 directly (v_fma_mixlo_f16), not to f32 first.
+// The two differ by an f16 ulp in about one of 2^14 values; the direct rounding
+// is the nearer one.  A product of two T values is exact in f32 and rounded to T.
 //
 // Lane mapping: a row group of 16 consecutive lanes owns the row, lane j
 // holds elements 8j .. 8j+7 (16 bytes).  The sum of squares is a 16-lane DPP

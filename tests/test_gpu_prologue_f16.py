@@ -121,3 +121,33 @@ def test_prologue_mixed_dtypes_rejected(cos_sin):
     with pytest.raises(_lib.NvkError, match="share one dtype"):
         qk_norm_rope_store(d(pos), d(qkv), 16, 8, D, d(qw), d(kw), EPS, d(cos_sin),
                            d(kc.to(torch.bfloat16)), d(vc.to(torch.bfloat16)), d(slots))
+
+
+def test_normed_product_is_rounded_once():
+    """x * rsqrt(mean(x^2) + eps) goes to f16 in one rounding.  The rows hold eight
+    integers of up to 10 bits: their sum of squares is exact in f32 and rsqrtf is within an
+    ulp of the exact value, mostly the nearest f32; with that one, the two ways of
+    rounding differ for the elements looked at, and nearly all of those show which."""
+    g = np.random.default_rng(5)
+    hq, t = 16, 16384
+    x = np.zeros((t, hq, D), np.float16)
+    x[:, :, ::16] = g.integers(-1023, 1024, (t, hq, 8))
+    x[:, :, 0] = np.where(x[:, :, 0] == 0, 1, x[:, :, 0])
+    ss = (x.astype(np.float64) ** 2).sum(-1, keepdims=True)
+    rstd = (1.0 / np.sqrt(ss / D)).astype(np.float32)
+    prod = x.astype(np.float64) * rstd                       # exact in f64
+    once, twice = prod.astype(np.float16), prod.astype(np.float32).astype(np.float16)
+    at = once != twice
+    assert at.sum() > 60
+    qkv = torch.zeros(t, (hq + 2) * D, dtype=F16)
+    qkv[:, :hq * D] = torch.from_numpy(x.reshape(t, -1))
+    qkv[:, hq * D:] = 1
+    one = torch.ones(D, dtype=F16).cuda()
+    turn = torch.cat([torch.ones(1, 1, D // 2), torch.zeros(1, 1, D // 2)], -1).cuda()  # angle 0
+    say("f16 prologue, rounding of the normed product")
+    q, _, _ = qk_norm_rope_store(torch.zeros(t, dtype=torch.int64).cuda(), qkv.cuda(), hq, 1, D,
+                                 one, one, 0.0, turn, None, None, None)
+    got = q.cpu().numpy()
+    share = (got[at] == once[at]).mean()
+    print(f"{at.sum()} elements, rounded once {share:.3f}, twice {(got[at] == twice[at]).mean():.3f}")
+    assert share > 0.75
