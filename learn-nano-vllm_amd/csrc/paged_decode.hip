@@ -912,6 +912,7 @@ int decode_short_query(const DecodeArgs& a, float scale, void* workspace, hipStr
   p.v_cache = a.v_cache;
   p.context_lens = a.context_lens;
   p.n_query = 1;
+  p.decode = true;
   p.batch = a.batch;
   p.block_tables = a.block_tables;
   p.bt_stride = a.bt_stride;

@@ -19,6 +19,7 @@ struct ShortQueryParams {
   // end of its context_lens[s] keys, cu_q / cu_k unused; else null
   const int32_t* context_lens = nullptr;
   int n_query = 1;
+  bool decode = false;  // a decode (uniform form, n_query 1): probabilities in two parts
   int batch;
   const int32_t* block_tables;
   int64_t bt_stride;

@@ -95,3 +95,31 @@ def test_one_and_two_chunks_per_wave(hq, hkv, ctx):
         out = paged_decode(c.q, c.k_cache, c.v_cache, c.context_lens, bt, case.scale)
         torch.cuda.synchronize()
         assert_attn_close(out, ref, f"{hq}/{hkv} {ctx}")
+
+
+@pytest.mark.parametrize("hq,hkv,b", [(16, 2, 24), (16, 4, 24), (8, 8, 40)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_no_less_exact_than_the_decode_kernel(hq, hkv, b, dtype):
+    """Pages of 16 keys stay on the decode kernel: over the same keys its error
+    against float64 bounds the MFMA kernels'."""
+    ctx = [200 + 61 * i for i in range(b)]
+    case = decode_case(seed=27, hq=hq, hkv=hkv, ctx=ctx, pool_blocks=sum(-(-c // 256) for c in ctx))
+    q, kc, vc = (t.to(dtype).cuda() for t in (case.q, case.k_cache, case.v_cache))
+    bt, lens = case.block_tables.cuda(), case.context_lens.cuda()
+    fine = (bt[..., None] * 16 + torch.arange(16, device="cuda", dtype=torch.int32)).flatten(1)
+    fine[(bt < 0).repeat_interleave(16, 1)] = -1
+    ref = torch.empty(b, hq, 128, dtype=torch.float64, device="cuda")
+    for i, n in enumerate(ctx):
+        pages = bt[i, :-(-n // 256)].long()
+        k, v = (c[pages].flatten(0, 1)[:n].double() for c in (kc, vc))
+        for h in range(hkv):
+            rows = slice(h * (hq // hkv), (h + 1) * (hq // hkv))
+            p = torch.softmax(q[i, rows].double() @ k[:, h].t().contiguous() * case.scale, -1)
+            ref[i, rows] = p @ v[:, h].contiguous()
+    say(f"decode {hq}/{hkv} heads, {b} sequences, {dtype}, error against float64")
+    here = paged_decode(q, kc, vc, lens, bt, case.scale)
+    there = paged_decode(q, kc.view(-1, 16, hkv, 128), vc.view(-1, 16, hkv, 128), lens,
+                         fine.contiguous(), case.scale)
+    err = [((o.double() - ref).norm() / ref.norm()).item() for o in (here, there)]
+    print(f"MFMA kernels {err[0]:.6f}, decode kernel {err[1]:.6f}")
+    assert err[0] <= err[1]
