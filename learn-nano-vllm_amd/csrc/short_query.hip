@@ -193,7 +193,9 @@ __device__ __forceinline__ float max_xor16(float x) {
 // to four running maxima per wave (each one's largest key rounds to nothing).
 // Relative error of a layer against 64 bits, 192 x U{256..4096} keys, 16/2 heads:
 // decode kernel 0.00355, one part here 0.00364, two 0.00335, at the same time (84.6 /
-// 84.5 us: the stream leaves the matrix cores idle).
+// 84.5 us: the stream leaves the matrix cores idle).  The remainders' products have
+// accumulators of their own, left out where they are not finite: an infinite value
+// times a remainder of 0, or of either sign, would turn the infinity into NaN.
 template <bool F16, bool KLDS, bool UNIFORM, bool SPLITP>
 __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs a) {
   using E = NvkElt<F16>;
@@ -257,7 +259,7 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
 
   // per-group state
   vec8 qf[HD / 32];
-  nvk_f32x4 acc_o[HD / 16];
+  nvk_f32x4 acc_o[HD / 16], acc_r[SPLITP ? HD / 16 : 1];
   float m_run = -INFINITY, l_part = 0.f;
   int q_row0 = 0, Lq = 0, nkeys = 0, diag = 0, tok = 0, head = 0;
   bool row_valid = false;
@@ -282,7 +284,10 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
       qf[ks] = __builtin_bit_cast(vec8, v);
     }
 #pragma unroll
-    for (int db = 0; db < HD / 16; ++db) acc_o[db] = nvk_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int db = 0; db < HD / 16; ++db) {
+      acc_o[db] = nvk_f32x4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (SPLITP) acc_r[db] = nvk_f32x4{0.f, 0.f, 0.f, 0.f};
+    }
     m_run = -INFINITY;
     l_part = 0.f;
   };
@@ -417,7 +422,10 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
     m_run = m_new;
     l_part *= alpha;
 #pragma unroll
-    for (int db = 0; db < HD / 16; ++db) acc_o[db] *= alpha;
+    for (int db = 0; db < HD / 16; ++db) {
+      acc_o[db] *= alpha;
+      if constexpr (SPLITP) acc_r[db] *= alpha;
+    }
     constexpr uint32_t kOnes = E::kOnes;  // the pair (1, 1)
     vec8 pf[kPairs], pr[kPairs];  // pr: the rounding's remainders (SPLITP)
 #pragma unroll
@@ -459,7 +467,7 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
         const nvk_i16x8 vv = {vlo[0], vlo[1], vlo[2], vlo[3], vhi[0], vhi[1], vhi[2], vhi[3]};
         acc_o[db] = E::mfma16x16x32(__builtin_bit_cast(vec8, vv), pf[p], acc_o[db]);
         if constexpr (SPLITP)
-          acc_o[db] = E::mfma16x16x32(__builtin_bit_cast(vec8, vv), pr[p], acc_o[db]);
+          acc_r[db] = E::mfma16x16x32(__builtin_bit_cast(vec8, vv), pr[p], acc_r[db]);
       }
     }
     // the V buffer is free again: the next chunk's V goes out
@@ -469,6 +477,13 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
     if (group_end || last) {
       const float l_tot = nvk_sum_xor32(sum_xor16(l_part));
       const bool whole = group_end && started_here;
+      if constexpr (SPLITP) {
+#pragma unroll
+        for (int db = 0; db < HD / 16; ++db)
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            acc_o[db][i] += __builtin_isfinite(acc_r[db][i]) ? acc_r[db][i] : 0.f;
+      }
       if (whole) {
         if (row_valid) {
           const float inv = l_tot > 0.f ? 1.f / l_tot : 0.f;

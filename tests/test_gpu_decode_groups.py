@@ -97,6 +97,45 @@ def test_one_and_two_chunks_per_wave(hq, hkv, ctx):
         assert_attn_close(out, ref, f"{hq}/{hkv} {ctx}")
 
 
+def _float64_decode(q, kc, vc, bt, ctx, scale):
+    """The plain decode in float64, on the caches' device."""
+    hkv, g, page = kc.shape[2], q.shape[1] // kc.shape[2], kc.shape[1]
+    ref = torch.empty(q.shape, dtype=torch.float64, device=q.device)
+    for i, n in enumerate(ctx):
+        pages = bt[i, :-(-n // page)].long()
+        k, v = (c[pages].flatten(0, 1)[:n].double() for c in (kc, vc))
+        for h in range(hkv):
+            rows = slice(h * g, (h + 1) * g)
+            p = torch.softmax(q[i, rows].double() @ k[:, h].t().contiguous() * scale, -1)
+            ref[i, rows] = p @ v[:, h].contiguous()
+    return ref
+
+
+INFINITE = [  # hq, hkv, contexts
+    (16, 2, [1, 20, 32]), (16, 4, [20]),            # groups that one wave finishes
+    (8, 8, [5 + i for i in range(28)] * 2),         # one head, from 33 sequences up
+]
+
+
+@pytest.mark.parametrize("hq,hkv,ctx", INFINITE)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_infinite_values_stay_infinite(hq, hkv, ctx, dtype):
+    """A value of +-inf gives +-inf in its dimension, not NaN: no probability here
+    rounds to 0, and nothing may multiply it by 0 on the side."""
+    case = decode_case(seed=19, hq=hq, hkv=hkv, ctx=ctx, pool_blocks=sum(-(-c // 256) for c in ctx))
+    q, kc, vc = (t.to(dtype).cuda() for t in (case.q, case.k_cache, case.v_cache))
+    bt, lens = case.block_tables.cuda(), case.context_lens.cuda()
+    for i, n in enumerate(ctx):     # the first key and the last
+        for pos, dim, x in ((0, 5, float("inf")), (n - 1, 100, float("-inf"))):
+            vc[bt[i, pos // 256].long(), pos % 256, :, dim] = x
+    say(f"infinite values, {hq}/{hkv} heads, {len(ctx)} sequences of {min(ctx)}-{max(ctx)}, {dtype}")
+    out = paged_decode(q, kc, vc, lens, bt, case.scale).double()
+    ref = _float64_decode(q, kc, vc, bt, ctx, case.scale)
+    torch.cuda.synchronize()
+    assert ref[..., 5].eq(float("inf")).all() and ref[..., 100].eq(float("-inf")).all()
+    torch.testing.assert_close(out, ref, atol=2e-2, rtol=1e-2)
+
+
 @pytest.mark.parametrize("hq,hkv,b", [(16, 2, 24), (16, 4, 24), (8, 8, 40)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_no_less_exact_than_the_decode_kernel(hq, hkv, b, dtype):
@@ -108,14 +147,7 @@ def test_no_less_exact_than_the_decode_kernel(hq, hkv, b, dtype):
     bt, lens = case.block_tables.cuda(), case.context_lens.cuda()
     fine = (bt[..., None] * 16 + torch.arange(16, device="cuda", dtype=torch.int32)).flatten(1)
     fine[(bt < 0).repeat_interleave(16, 1)] = -1
-    ref = torch.empty(b, hq, 128, dtype=torch.float64, device="cuda")
-    for i, n in enumerate(ctx):
-        pages = bt[i, :-(-n // 256)].long()
-        k, v = (c[pages].flatten(0, 1)[:n].double() for c in (kc, vc))
-        for h in range(hkv):
-            rows = slice(h * (hq // hkv), (h + 1) * (hq // hkv))
-            p = torch.softmax(q[i, rows].double() @ k[:, h].t().contiguous() * case.scale, -1)
-            ref[i, rows] = p @ v[:, h].contiguous()
+    ref = _float64_decode(q, kc, vc, bt, ctx, case.scale)
     say(f"decode {hq}/{hkv} heads, {b} sequences, {dtype}, error against float64")
     here = paged_decode(q, kc, vc, lens, bt, case.scale)
     there = paged_decode(q, kc.view(-1, 16, hkv, 128), vc.view(-1, 16, hkv, 128), lens,
