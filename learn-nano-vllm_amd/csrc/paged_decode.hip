@@ -666,7 +666,8 @@ __device__ __forceinline__ void fold_parts(const DecodeArgs& a, const float* rec
     for (int u = 0; u < kBatch; ++u) {
       const float wt = nvk_fast_exp2(mv[u] - mref);
       L += lv[u] * wt;
-      O += ov[u] * wt;
+      // past the last part: part p1 again, which 0 does not cancel if infinite
+      O += (base + u * S <= p2 ? ov[u] : 0.f) * wt;
     }
     M = mb;
   }

@@ -561,7 +561,9 @@ __device__ __forceinline__ void sq_merge_parts(const SqArgs& a, int row, int d0,
     for (int u = 0; u < kBatch; ++u) {
       const float wt = nvk_fast_exp2(mv[u] - mb);
       L += lv[u] * wt;
-      O += wt * ov[u];
+      // past the last part: part p1 again, which 0 does not cancel if infinite
+      const nvk_f32x4 o = base + u * S <= p2 ? ov[u] : nvk_f32x4{0.f, 0.f, 0.f, 0.f};
+      O += wt * o;
     }
     M = mb;
   }

@@ -114,6 +114,8 @@ def _float64_decode(q, kc, vc, bt, ctx, scale):
 INFINITE = [  # hq, hkv, contexts
     (16, 2, [1, 20, 32]), (16, 4, [20]),            # groups that one wave finishes
     (8, 8, [5 + i for i in range(28)] * 2),         # one head, from 33 sequences up
+    (16, 8, [20]), (16, 8, [64, 70]), (16, 2, [64, 200]),   # cut into 2, 3 and 7 parts
+    (16, 8, [2000]), (16, 2, [2000]), (8, 1, [3000]),       # the sliced merges
 ]
 
 
