@@ -806,7 +806,7 @@ int launch_decode(const DecodeArgs& a, bool aligned, hipStream_t stream) {
   const dim3 grid(a.n_waves / kWavesPerWG);
   // HD 128 with 4 or 8 heads per kv head and pages of whole chunks: the
   // short-query kernels' (an empty pool, num_blocks 0, takes the general form)
-  constexpr bool kWholePages = FUSED || HD != 128 || G <= kDecodeKernelGroup;
+  constexpr bool kWholePages = HD != 128 || G <= kDecodeKernelGroup;
   if constexpr (kWholePages)
     if (aligned)
       hipLaunchKernelGGL((paged_decode_kernel<HD, G, true, FUSED, F16>), grid, dim3(256), 0,
@@ -1139,13 +1139,13 @@ extern "C" int nvk_paged_decode_prologue(
   const bool aligned = (block_size % tc) == 0;
   a.f16 = dtype == NVK_DTYPE_F16;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  // Group sizes whose decode runs on the short-query kernels: the prologue
-  // kernel writes q into `out` (whose rows a wave overwrites only when it has
-  // finished the whole group it read them for; the rows of cut groups are
-  // written by the combine), then that decode.
+  // Group sizes whose decode runs on the short-query kernels (as in
+  // nvk_paged_decode, so that both give the same bits): the prologue kernel
+  // writes q into `out`, in whatever order its rows lie (a wave overwrites them
+  // only when it has finished the whole group it read them for; the rows of cut
+  // groups are written by the combine), then that decode.
   if (short_query_decode_applies(block_size, num_blocks, num_q_heads, num_kv_heads, head_dim,
-                                 batch) &&
-      out_stride_head >= head_dim && out_stride_tok >= (int64_t)num_q_heads * out_stride_head) {
+                                 batch)) {
     const QkPrologue p = {qkv, qkv_row_stride, batch, positions, q_norm_weight, k_norm_weight, eps,
                           cos_sin_cache, cos_sin_row_stride, max_position, num_q_heads,
                           num_kv_heads, head_dim, out, out_stride_tok, out_stride_head, nullptr, 0,

@@ -22,7 +22,9 @@ struct QkPrologue {
   const int32_t* slot_mapping;  // null: no store
   int64_t cache_slots;
   int32_t dtype;
-  // decode steps: tokens whose context length is 0 (graph padding) store nothing; null: unused
+  // decode steps: tokens whose context length is 0 (graph padding) store nothing,
+  // and q_out is the attention's output, its rows in any order and any number;
+  // null: no decode step
   const int32_t* context_lens = nullptr;
 };
 

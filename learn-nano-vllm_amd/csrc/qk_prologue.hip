@@ -207,8 +207,10 @@ int qk_prologue_launch(const QkPrologue& p, bool with_q, void* stream) {
   if (p.max_position <= 0 || p.cos_sin_stride < p.head_dim) return NVK_EINVAL;
   const int64_t R = (int64_t)p.num_q_heads + 2 * p.num_kv_heads;
   if (p.qkv_row_stride < R * p.head_dim) return NVK_EINVAL;
-  if (with_q && (p.q_out_stride_head < p.head_dim ||
-                 p.q_out_stride_tok < (int64_t)p.num_q_heads * p.q_out_stride_head))
+  const bool any_rows = p.context_lens != nullptr;  // a decode step's output
+  if (with_q && !any_rows &&
+      (p.q_out_stride_head < p.head_dim ||
+       p.q_out_stride_tok < (int64_t)p.num_q_heads * p.q_out_stride_head))
     return NVK_EINVAL;
   if (p.k_out && (p.k_out_stride_head < p.head_dim ||
                   p.k_out_stride_tok < (int64_t)p.num_kv_heads * p.k_out_stride_head))
@@ -225,7 +227,7 @@ int qk_prologue_launch(const QkPrologue& p, bool with_q, void* stream) {
       (p.k_out && ((p.k_out_stride_tok % 8) || (p.k_out_stride_head % 8))) ||
       (p.cos_sin_stride % 4))
     return NVK_EALIGN;
-  if (p.n_tokens > INT32_MAX || R > 65535) return NVK_EINVAL;
+  if (p.n_tokens > INT32_MAX || (R > 65535 && !any_rows)) return NVK_EINVAL;
   if (!with_q && !p.k_out && !store) return NVK_OK;
   const int rows = (int)R - (with_q ? 0 : p.num_q_heads);
   const int max_groups = p.n_tokens <= kSmallTokens ? kMaxRowGroups : kMaxGroups;

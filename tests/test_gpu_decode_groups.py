@@ -46,26 +46,33 @@ def test_decode_groups_match_oracle(hq, hkv, ctx, bs, dtype):
     assert out[..., 128:].isnan().all(), "nothing outside the rows is written"
 
 
-@pytest.mark.parametrize("strided", [False, True])
-def test_prologue_form_with_q_in_the_output_rows(strided):
-    hq, hkv, bs = 16, 2, 256
-    ctx = [1, 32, 33, 257, 0, 1700, 2900]
-    case = decode_case(seed=8, hq=hq, hkv=hkv, ctx=ctx, pool_blocks=30)
+@pytest.mark.parametrize("rows", ["contiguous", "padded", "head by head"])
+@pytest.mark.parametrize("hq,hkv,ctx", [
+    (16, 2, [1, 32, 33, 257, 0, 1700, 2900]), (16, 4, [1, 32, 33, 257, 0, 1700, 2900]),
+    (4, 4, [1, 32, 33, 257, 0, 1700, 2900] + [3 * i for i in range(30)]),   # one head: 33 and up
+])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_prologue_form_with_q_in_the_output_rows(rows, hq, hkv, ctx, dtype):
+    bs = 256
+    case = decode_case(seed=8, hq=hq, hkv=hkv, ctx=ctx, pool_blocks=60)
+    case.k_cache, case.v_cache = case.k_cache.to(dtype), case.v_cache.to(dtype)
     g = torch.Generator().manual_seed(9)
-    qkv = (torch.randn(len(ctx), (hq + 2 * hkv) * 128, generator=g) * 2).to(torch.bfloat16).cuda()
-    w = (1 + 0.2 * torch.randn(2, 128, generator=g)).to(torch.bfloat16).cuda()
+    qkv = (torch.randn(len(ctx), (hq + 2 * hkv) * 128, generator=g) * 2).to(dtype).cuda()
+    w = (1 + 0.2 * torch.randn(2, 128, generator=g)).to(dtype).cuda()
     cs = rope_cos_sin_cache(128, 4096, 1e6).cuda()
     lens, bt = case.context_lens.cuda(), case.block_tables.cuda()
     pos = (lens - 1).long().clamp(min=0)
     slots = (bt.gather(1, (pos // bs)[:, None]).squeeze(1) * bs + pos % bs).to(torch.int32)
     slots[lens == 0] = -1
     caches = [[case.k_cache.cuda(), case.v_cache.cuda()] for _ in range(2)]
-    say(f"prologue form, strided out {strided}")
+    say(f"prologue form {hq}/{hkv}, {len(ctx)} sequences, {rows} out, {dtype}")
     q, _, _ = qk_norm_rope_store(pos, qkv, hq, hkv, 128, w[0], w[1], 1e-6, cs, *caches[0], slots,
                                  return_k=False)
     ref = paged_decode(q, *caches[0], lens, bt, 128 ** -0.5)
-    out = torch.empty(len(ctx), hq, 136 if strided else 128, dtype=torch.bfloat16, device="cuda")
+    out = torch.empty(len(ctx), hq, 136 if rows == "padded" else 128, dtype=dtype, device="cuda")
     out = out[..., :128]
+    if rows == "head by head":
+        out = torch.empty(hq, len(ctx), 128, dtype=dtype, device="cuda").transpose(0, 1)
     slots[lens == 0] = 3      # a row without a context stores nothing, whatever its slot
     for _ in range(2):      # the second call finds the first one's outputs in out
         paged_decode_with_prologue(pos, qkv, hq, hkv, 128, w[0], w[1], 1e-6, cs, *caches[1], slots,
