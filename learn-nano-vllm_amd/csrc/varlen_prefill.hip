@@ -1337,15 +1337,32 @@ size_t order_bytes_for(int32_t batch, int32_t max_seqlen_q, int64_t max_keys, in
 // Whether the attention workgroups norm and rotate their own q rows, so that
 // q is neither written by the prologue kernel nor read back (8 KiB per token of
 // 16 heads), at ~800 VALU instructions and a round trip for the rotation rows
-// at each workgroup's start.  Measured per pass, q through out's rows / here
-// (eager calls, two layers): 28 prompts of 100-1024 tokens 263.5 / 255.8 us, 32
-// x 100-1024 after a shared 512 402.5 / 390.0, 4 x 4096 (one layer) 335.0 /
-// 329.1, 1 x 4096 230.0 / 223.3, 8 x 100-1024 after 512 145.8 / 143.9; 8
-// prompts of 100-1024 82.1 / 82.6.  Below one round of the workgroup slots the
-// start is exposed, and parts of one tile would repeat the work.
+// at each workgroup's start.  Parts of one tile would repeat the work, and below
+// one round of the 512 workgroup slots the start is exposed.  With little more
+// than one round it still is, unless a step's tiles differ much in length (the
+// short ones then fill the second round): the new tokens have to outweigh the
+// cached ones there.  With 8 heads per kv head the prologue kernel has hardly
+// any other rows, and only few long prompts lose.  Measured per pass (eager
+// calls, three layers), q through out's rows / here, 16/16, 16/8 and 16/2 heads:
+//   9 x 500 tokens        154.5 / 163.4, 121.3 / 125.9, 104.2 / 99.7 us
+//   9 x 500 after 512     222.2 / 230.3, 194.7 / 195.3, 179.9 / 169.4
+//   5 x 900 after 512     235.3 / 237.2, 196.5 / 208.6, 182.2 / 186.9
+//   64 x 70..100                    -,   121.6 / 126.4,  98.3 /  89.7
+//   11 x 500              190.9 / 194.4, 149.4 / 149.2, 126.3 / 117.1
+//   11 x 500 after 512    262.1 / 262.2, 224.3 / 218.9, 200.0 / 189.6
+//   12 x 505              201.5 / 199.7, 154.7 / 153.4, 128.7 / 122.7
+//   32 x 505              513.9 / 485.3, 378.6 / 341.0, 307.3 / 259.1
+//   6 x 750               169.2 / 162.9, 133.3 / 125.5, 114.3 / 100.7
+//   3 x 1500              218.9 / 204.2, 182.4 / 171.9, 162.8 / 145.4
+//   2 x 2200 after 512    297.7 / 284.2, 268.4 / 255.5, 248.6 / 231.2
+//   1 x 4500              412.1 / 397.9, 382.7 / 368.8, 360.3 / 338.0
 constexpr int64_t kNormQMinWgs = 512, kNormQMinTokens = 4096;
-bool prefill_norms_q(const SplitPlan& p, int64_t wgs, int64_t tokens) {
-  return p.n_splits == 1 && wgs >= kNormQMinWgs && tokens >= kNormQMinTokens;
+bool prefill_norms_q(const SplitPlan& p, int64_t wgs, int64_t tokens, int batch,
+                     int64_t max_seqlen_q, int64_t max_keys, int G) {
+  if (p.n_splits != 1 || wgs < kNormQMinWgs || tokens < kNormQMinTokens) return false;
+  const bool few_others = G == 8 && tokens <= 700 * (int64_t)batch;
+  const int64_t any_shape = G == 1 ? 6000 : few_others ? kNormQMinTokens : 5400;
+  return tokens >= any_shape || 2 * max_seqlen_q >= max_keys + 700;
 }
 
 int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_head,
@@ -1418,7 +1435,8 @@ int varlen_prefill_impl(const void* q, int64_t q_stride_tok, int64_t q_stride_he
     if ((uintptr_t)given_order % 4) return NVK_EALIGN;
   }
 
-  const bool norm_q = pro && !short_q && prefill_norms_q(sp, pairs * num_kv_heads, total_q);
+  const bool norm_q = pro && !short_q && prefill_norms_q(sp, pairs * num_kv_heads, total_q, batch,
+                                                        max_seqlen_q, max_keys, G);
   if (pro) {
     // Without norm_q, q goes through out's rows: a workgroup (or, in the
     // short-query kernels, a wave) overwrites only rows whose q it alone has

@@ -60,6 +60,14 @@ CASES = [  # lens_q, cached, hq, hkv, bs
     ([300], [4000], 16, 8, 256),              # parts
     ([6, 6, 3], [900, 50, 2000], 16, 8, 256),  # short-query kernels
     ([1], [0], 4, 2, 256),
+    # own q rows behind cached ones
+    ([700] * 9 + [1, 33], [256 * i + 7 for i in range(11)], 16, 8, 256),
+    ([700] * 9 + [1, 33], [100] * 11, 16, 8, 48),
+    ([700] * 9, [64] * 9, 16, 4, 64),
+    ([600] * 11, [128] * 11, 16, 16, 256),
+    # and ranked tiles
+    ([700] * 12, [0] * 12, 16, 8, 256),
+    ([700] * 12, [100 * i for i in range(12)], 16, 4, 64),
 ]
 
 
@@ -84,6 +92,49 @@ def test_one_call_equals_two(lens_q, cached, hq, hkv, bs, dtype):
         reset_context()
     assert torch.equal(one, two)
     assert torch.equal(k1, kc) and torch.equal(v1, vc)
+
+
+@pytest.mark.parametrize("lens_q,cached,hq,hkv,own,ranked", [
+    ([600] * 8 + [599], [512] * 9, 16, 8, True, False),        # with the spare token: 5400
+    ([600] * 8 + [598], [512] * 9, 16, 8, False, False),
+    ([600] * 9 + [599], [512] * 10, 16, 16, True, False),      # 6000
+    ([600] * 9 + [598], [512] * 10, 16, 16, False, False),
+    ([512] * 7 + [511], [512] * 8, 16, 2, True, False),        # 4096
+    ([512] * 7 + [510], [512] * 8, 16, 2, False, False),
+    ([700] * 6 + [699], [512] * 7, 16, 2, True, False), ([700] * 7, [512] * 7, 16, 2, False, False),
+    ([1024] * 4, [324] * 4, 16, 8, True, False), ([1024] * 4, [325] * 4, 16, 8, False, False),
+    ([700] * 12, [0] * 12, 16, 8, True, True), ([700] * 12, [64] * 12, 16, 4, True, True),
+])
+def test_which_steps_norm_their_own_q(lens_q, cached, hq, hkv, own, ranked):
+    """The edges of the rule, seen on a token that belongs to no sequence: its row of
+    out gets q from the prologue kernel, or nothing where the attention's
+    workgroups norm their own rows."""
+    paged = any(cached)
+    qkv, w, pos, kc, vc, cs = _step(7, lens_q + [1], cached + [0], hq, hkv, 256, torch.bfloat16,
+                                    paged)
+    c, lib, T, batch = get_context(), _lib.load(), sum(lens_q) + 1, len(lens_q)
+    reset_context()
+    mq, mk = max(lens_q), max(a + b for a, b in zip(lens_q, cached))
+    sizes = (batch, mq, mk, hq, hkv)
+    assert (lib.nvk_prefill_tile_order_size(*sizes, 256) > 0) == ranked
+    out = torch.full((T, hq, D), 77.0, dtype=qkv.dtype, device="cuda")
+    k_new = torch.empty(T, hkv, D, dtype=qkv.dtype, device="cuda")
+    ws_bytes = lib.nvk_varlen_prefill_parts_workspace_size(*sizes, D)
+    ws = torch.empty(ws_bytes + 256, dtype=torch.uint8, device="cuda")
+    cs2, bt = cs.view(cs.shape[0], -1), c.block_tables
+    say(f"own q rows of {batch} sequences, {T - 1} tokens, {hq}/{hkv} heads")
+    _lib.check(lib.nvk_varlen_prefill_prologue(
+        qkv.data_ptr(), qkv.stride(0), T, pos.data_ptr(), w[0].data_ptr(), w[1].data_ptr(), EPS,
+        cs2.data_ptr(), cs2.stride(0), cs2.shape[0], kc.data_ptr(), vc.data_ptr(),
+        c.slot_mapping.data_ptr(), kc.shape[0] * kc.shape[1], None if paged else k_new.data_ptr(),
+        c.cu_seqlens_q.data_ptr(), c.cu_seqlens_k.data_ptr(), batch, mq, mk,
+        bt.data_ptr() if paged else None, bt.stride(0) if paged else 0,
+        bt.shape[1] if paged else 0, 256 if paged else 0, kc.shape[0] if paged else 0, hq, hkv, D,
+        D ** -0.5, out.data_ptr(), out.stride(0), out.stride(1), ws.data_ptr(), ws_bytes, None, 0,
+        _lib.dtype_code(qkv), _lib.stream_ptr(qkv.device)))
+    torch.cuda.synchronize()
+    assert out[-1].eq(77).all().item() == own
+    assert not out[:-1].eq(77).any()
 
 
 def test_empty_cache_and_hooks():
