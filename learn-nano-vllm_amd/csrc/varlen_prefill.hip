@@ -997,8 +997,8 @@ __global__ __launch_bounds__(64 * kWaves, 8 / kWaves) void varlen_prefill_kernel
       }
     }
     if (half == 0) {
-      rec[kRecO + 2 * row] = m_ref;
-      rec[kRecO + 2 * row + 1] = l_tot;
+      rec[kRecO + 64 * wave + 2 * lane] = m_ref;
+      rec[kRecO + 64 * wave + 2 * lane + 1] = l_tot;
     }
     return;
   }

@@ -278,3 +278,22 @@ def test_work_counts():
     row = D * 2
     assert prologue_bytes(10, 8, 6, 16, 8, D, write_k=True) == (
         10 * 32 * row + 10 * 12 + 6 * D * 4 + 10 * 16 * row + 8 * 16 * row + 10 * 8 * row)
+
+
+def test_plain_prefill_kernels_keep_their_registers():
+    """The compiled attention kernels of a prefill whose q is normed already keep
+    everything in registers, but for the one that looks every key row up by
+    itself.  Read from the metadata that the compiler leaves beside each kernel."""
+    msgpack = pytest.importorskip("msgpack")
+    blob = open(_lib.LIB_PATH, "rb").read()
+    spills, at = {}, blob.find(b"amdhsa.kernels")
+    while at >= 0:
+        notes = msgpack.Unpacker(strict_map_key=False)
+        notes.feed(blob[at - 2:])           # the map's head and the key's length byte before it
+        for k in notes.unpack()["amdhsa.kernels"]:
+            name = re.search(r"varlen_prefill_kernelILi(\d)ELi(\d)ELb([01])ELb0E", k[".name"])
+            if name:
+                spills[name.groups()] = k[".vgpr_spill_count"]
+        at = blob.find(b"amdhsa.kernels", at + 1)
+    assert len(spills) == 4 * 3 * 2         # group size, key layout, element type
+    assert not {k: n for k, n in spills.items() if n and k[1] != "2"}
