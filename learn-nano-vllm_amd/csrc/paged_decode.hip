@@ -35,10 +35,10 @@
 // non-temporal (read once).  The page of a chunk comes through a scalar load
 // when a page holds whole chunks.
 //
-// Steps with 4 or more query heads per kv head (or one, from 33 sequences up)
-// run on the MFMA kernels of short_query.hip instead (short_query.h has the
-// rule and both sides' times): the dot products and the softmax bookkeeping
-// here cost VALU time per query head.
+// Steps with 4 or more query heads per kv head run on the MFMA kernels of
+// short_query.hip instead (short_query.h has the rule and both sides' times):
+// the dot products and the softmax bookkeeping here cost VALU time per query
+// head.
 //
 // Finishing: a group that ends inside a wave's range is normalised in
 // registers and written as bf16.  A group cut between waves leaves one
@@ -570,6 +570,11 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(DecodeArgs a) {
       }
     } else {
       load_chunk<HD, G, ALIGNED, FUSED>(a, cur, ctx, role, tpi, buf);
+      // With one head the compiler otherwise starts on K and issues V's loads after
+      // it (88 registers): a second round trip per chunk.  16/16 heads, without /
+      // with: 1 x 1000 keys 12.5 / 9.7 us, 16 x U{500..1000} 27.2 / 24.2, 32 x
+      // U{100..2048} 63.8 / 51.9, 192 x U{256..4096} 610 / 485; HD 64 322 / 256.
+      if constexpr (G == 1) __builtin_amdgcn_sched_barrier(0);
     }
     compute_chunk<HD, G, F16>(a, buf, cur.k * a.tc, ctx, tpi, role, st);
     const bool last = c + 1 == c1;

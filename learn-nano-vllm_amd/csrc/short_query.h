@@ -38,23 +38,19 @@ bool short_query_applies(bool paged, int block_size, int max_seqlen_q, int num_q
 
 // True when a decode of these sizes runs here rather than on the decode
 // kernel: paged keys in pages of a multiple of 32 keys, head_dim 128, and 4 or
-// more query heads per kv head, or one in steps of more than 32 sequences.
-// The decode kernel's dot products cost VALU time per query head (8 heads:
-// twice the stream's time), and with one head its waves stream 20 % slower
-// than these (up to 32 sequences its form with the prologue inside is the
-// faster one, 16/16 heads, 16 sequences: 31.0 us against 36.2 with the
-// separate prologue, and the plain form keeps the same bits).  Measured on
-// MI355X, graph replays over inputs past the Infinity Cache, decode kernel /
-// these:
+// more query heads per kv head.  The decode kernel's dot products cost VALU
+// time per query head (8 heads: twice the stream's time).  Measured on MI355X,
+// graph replays over inputs past the Infinity Cache, decode kernel / these:
 //   16/2 heads: 1 x 100 keys 15.0 / 8.9 us, 16 x U{100..2048} 22.5 / 14.3,
 //     64 x U{100..2048} 39.1 / 24.0, 192 x U{256..4096} 119.8 / 81.5;
 //   16/4: 11.8 / 9.2, 19.1 / 16.7, 37.9 / 36.6, 158.9 / 149.2 us;
-//   16/16, 64 and 192 sequences: 129.6 / 101.4, 707.2 / 546.6 us;
-//   16/8 (stays): 9.6 / 9.3, 20.0 / 22.8, 57.5 / 57.2, 284.9 / 281.8 us.
+//   16/8 (stays): 9.6 / 9.3, 20.0 / 22.8, 57.5 / 57.2, 284.9 / 281.8 us;
+//   16/16 (stays): 33 x U{100..300} 16.4 / 17.7, 48 x U{100..500} 27.8 / 27.6, 64
+//     x U{100..2048} 90.2 / 87.5, 192 x U{256..4096} 485 / 479 us, and with the
+//     prologue 18.4 / 21.6, 29.3 / 31.4, 91.5 / 91.0, 491 / 483 us.
 // With the prologue (nvk_paged_decode_prologue), 16/2: 1 x 100 18.5 / 11.6,
 // 32 x U{100..2048} 42.9 / 22.3 us; 16/4: 13.2 / 12.4, 29.0 / 27.1 us.
 constexpr int kDecodeKernelGroup = 2;
-constexpr int kDecodeKernelBatch = 32;
 bool short_query_decode_applies(int block_size, int num_blocks, int num_q_heads, int num_kv_heads,
                                 int head_dim, int batch);
 

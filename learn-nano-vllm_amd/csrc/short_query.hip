@@ -701,7 +701,7 @@ bool short_query_decode_applies(int block_size, int num_blocks, int num_q_heads,
   if (num_kv_heads <= 0 || num_q_heads % num_kv_heads || batch <= 0 || batch > kMaxBatch)
     return false;
   const int G = num_q_heads / num_kv_heads;
-  return G <= kR && (G > kDecodeKernelGroup || (G == 1 && batch > kDecodeKernelBatch));
+  return G <= kR && G > kDecodeKernelGroup;
 }
 
 size_t short_query_ws_bytes(int batch, int64_t max_keys, int num_q_heads, int num_kv_heads,
