@@ -62,18 +62,21 @@ constexpr int kLoads = 8;          // load instructions per tensor per chunk
 constexpr int kWavesPerWG = 4;
 constexpr int kMaxWGs = 512;       // 256 CUs x 2 workgroups (8 waves per CU)
 constexpr int kMaxBatch = 2048;    // sequences per call (LDS prefix table)
-// Chunks a wave streams at least.  One where every chunk of the step gets a
-// wave of its own and no group is cut into very many parts: the second chunk's
-// page id, K/V round trip and arithmetic follow the first's, ~2 us of a step
-// that takes ~10.  Two otherwise: uneven ranges of one and two chunks take as
-// long as two, with more parts to merge.  Measured on MI355X, two / one, 16/8
-// heads: 1 x 100 keys 9.4 / 8.1 us, 1 x 1000 11.9 / 10.0, 16 x U{100..300}
-// 12.6 / 10.6, 4 x U{100..2048} 13.7 / 13.1 (a 28-layer graph step of one
-// sequence 391 / 309 us); 16 x U{100..2048} (1.8 chunks a wave) 20.1 / 21.8;
-// 8/4 heads, 1 x 16000 (500 chunks per group) 16.9 / 19.2, 2 x U{4000..8000}
-// 15.1 / 16.0.
+// Chunks a wave streams at least.  One in steps of up to 1024 chunks (a wave per
+// SIMD) whose groups are not cut into very many parts: the second chunk's page
+// id, K/V round trip and arithmetic follow the first's, ~2 us of a step that
+// takes ~10.  Two otherwise: waves that share a SIMD, uneven ranges and more
+// parts to merge take as long.  Measured on MI355X, two / one, 16/8 heads: 1 x
+// 100 keys 9.4 / 8.1 us, 1 x 1000 11.9 / 10.0, 16 x U{100..300} 12.6 / 10.6 (a
+// 28-layer graph step of one sequence 391 / 309 us).  Over 270 shapes of 1 to 12
+// sequences, 8 to 128 chunks per group and 4/2 to 16/16 heads, both forms: up to
+// 1024 chunks one gains 4.5 to 21 %; 1152 to 2048 chunks +4 to -6 % (8/4 heads, 4
+// x 2560 keys, 1280 chunks, 12.7 / 13.1; 16/8, 2 x 4096 keys with the prologue,
+// 2048 chunks, 15.2 / 16.1).  8/4 heads, 1 x 16000 (500 chunks per group) 16.9 /
+// 19.2.
 constexpr int kMinChunks = 2;
-constexpr int kOneChunkGroup = 128;  // chunks per group, on average, up to which one is taken
+constexpr int64_t kOneChunkMax = 1024;
+constexpr int kOneChunkGroup = 128;  // chunks per group, on average
 #ifndef NVK_DECODE_SLICE_MIN_WAVES
 #define NVK_DECODE_SLICE_MIN_WAVES 32
 #endif
@@ -131,9 +134,9 @@ __device__ __forceinline__ int clamp_ctx(const DecodeArgs& a, int b) {
 
 // Waves that take part for T chunks of `groups` groups: at most P, and few
 // enough that each range holds kMinChunks chunks (bounds how finely a context
-// is split), or one per chunk (kOneChunkGroup).
+// is split), or one per chunk (kOneChunkMax, kOneChunkGroup).
 __device__ __forceinline__ int64_t active_waves(int64_t T, int64_t P, int64_t groups) {
-  if (T <= P && T <= kOneChunkGroup * groups) return T < 1 ? 1 : T;
+  if (T <= P && T <= kOneChunkMax && T <= kOneChunkGroup * groups) return T < 1 ? 1 : T;
   int64_t p = T / kMinChunks;
   if (p > P) p = P;
   return p < 1 ? 1 : p;
@@ -786,12 +789,14 @@ int decode_tc(int num_kv_heads, int head_dim) {
   return kLoads * (rpi / decode_hpi(num_kv_heads, head_dim));
 }
 
-// Waves of the persistent grid for these static sizes.
+// Waves of the persistent grid for these static sizes: the most that
+// active_waves can give.  The combine's form is chosen by them.
 int decode_waves(int batch, int num_kv_heads, int head_dim, int block_size, int max_blocks) {
   const int tc = decode_tc(num_kv_heads, head_dim);
   const int64_t max_chunks_seq = ((int64_t)block_size * max_blocks + tc - 1) / tc;
   const int64_t t_max = max_chunks_seq * batch * (num_kv_heads / decode_hpi(num_kv_heads, head_dim));
-  int64_t wgs = (t_max + kWavesPerWG - 1) / kWavesPerWG;
+  const int64_t one = t_max < kOneChunkMax ? t_max : kOneChunkMax, two = t_max / kMinChunks;
+  int64_t wgs = ((one > two ? one : two) + kWavesPerWG - 1) / kWavesPerWG;
   if (wgs > kMaxWGs) wgs = kMaxWGs;
   if (wgs < 1) wgs = 1;
   return (int)wgs * kWavesPerWG;

@@ -670,12 +670,14 @@ __global__ __launch_bounds__(64 * kSqSlices) void short_query_combine_sliced_ker
   sq_write_row<F16>(op, L, O);
 }
 
-// Waves of the grid: as many as the step's chunks can use, by its static bound
-// (uniform form: one chunk each, the varlen form's workspace holds two).
+// Waves of the grid: the most that active_waves can give, by the step's static
+// bound (the varlen form's workspace holds two chunks a wave only).  The
+// combine's form is chosen by them.
 int sq_waves(int batch, int64_t max_keys, int num_kv_heads, bool uniform_q) {
   const int64_t chunks = (max_keys + kCK - 1) / kCK;
   const int64_t t_max = chunks * batch * num_kv_heads;
-  int64_t wgs = (t_max / (uniform_q ? 1 : kMinChunks) + kWavesPerWG - 1) / kWavesPerWG;
+  const int64_t one = t_max < kOneChunkMax ? t_max : kOneChunkMax, two = t_max / kMinChunks;
+  int64_t wgs = ((uniform_q && one > two ? one : two) + kWavesPerWG - 1) / kWavesPerWG;
   if (wgs > kMaxWGs) wgs = kMaxWGs;
   if (wgs < 1) wgs = 1;
   return (int)wgs * kWavesPerWG;

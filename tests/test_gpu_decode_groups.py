@@ -84,7 +84,8 @@ def test_prologue_form_with_q_in_the_output_rows(rows, hq, hkv, ctx, dtype):
 @pytest.mark.parametrize("hq,hkv,ctx", [
     (16, 8, [1]), (16, 8, [1000]),                 # one chunk per wave
     (4, 2, [4096]), (4, 2, [4097]),                # 128 and 129 chunks per group
-    (16, 8, [2048] * 4), (16, 8, [2048] * 4 + [1]),    # 2048 chunks (all waves) and more
+    (16, 8, [2048] * 2), (16, 8, [2048] * 2 + [1]),    # 1024 chunks and more
+    (16, 8, [2048] * 4), (16, 8, [2048] * 4 + [1]),    # 2048 chunks (two for each wave) and more
     (16, 2, [3072] * 4), (16, 2, [3073] * 4),      # 768 chunks, and more, on the MFMA kernels
     (8, 1, [4096, 1]), (8, 1, [9000, 0, 1]),
 ])
