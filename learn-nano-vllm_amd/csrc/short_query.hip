@@ -121,6 +121,12 @@ __device__ __forceinline__ int seq_chunks(const SqArgs& a, int s) {
   return seq_queries<UNIFORM>(a, s) > 0 ? (seq_keys<UNIFORM>(a, s) + kCK - 1) / kCK : 0;
 }
 
+// Rows of a record.
+template <bool UNIFORM>
+__device__ __forceinline__ int rec_rows(const SqArgs& a) {
+  return UNIFORM ? a.rec_rows : kR;
+}
+
 // Exclusive prefix of chunks per sequence into s_cs[0..B]; returns the total.
 template <bool UNIFORM>
 __device__ int chunk_prefix(const SqArgs& a, int* s_cs, int* s_wsum) {
@@ -148,8 +154,9 @@ __device__ int chunk_prefix(const SqArgs& a, int* s_cs, int* s_wsum) {
   return total;
 }
 
+template <bool UNIFORM>
 __device__ __forceinline__ int64_t active_waves(int64_t T, int64_t P, int64_t groups) {
-  if (T <= P && T <= kOneChunkMax && T <= kOneChunkGroup * groups) return T < 1 ? 1 : T;
+  if (UNIFORM && T <= P && T <= kOneChunkMax && T <= kOneChunkGroup * groups) return T < 1 ? 1 : T;
   int64_t p = T / kMinChunks;
   if (p > P) p = P;
   return p < 1 ? 1 : p;
@@ -216,7 +223,7 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
     }
   }
   const int64_t T = (int64_t)Hkv * S;
-  const int64_t P = active_waves(T, a.n_waves, (int64_t)a.p.batch * Hkv);
+  const int64_t P = active_waves<UNIFORM>(T, a.n_waves, (int64_t)a.p.batch * Hkv);
   const int wave = uniform(tid >> 6);
   const int64_t w = (int64_t)blockIdx.x * kWavesPerWG + wave;
   if (w >= P || T == 0) return;
@@ -498,7 +505,8 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
           }
         }
       } else if (row_valid) {  // the combine reads the valid rows only
-        float* rec = a.rec + ((w * 2 + (started_here ? 0 : 1)) * a.rec_rows + r) * (int64_t)kRec;
+        float* rec =
+            a.rec + ((w * 2 + (started_here ? 0 : 1)) * rec_rows<UNIFORM>(a) + r) * (int64_t)kRec;
 #pragma unroll
         for (int db = 0; db < HD / 16; ++db) *reinterpret_cast<nvk_f32x4*>(rec + 16 * db + 4 * g) = acc_o[db];
         if (g == 0) {
@@ -531,12 +539,17 @@ __global__ __launch_bounds__(64 * kWavesPerWG, 2) void short_query_kernel(SqArgs
 // p1's head record, slot 0, then the continuation records, slot 1): slice s
 // of S folds parts p1+s, p1+s+S, ..., kBatch parts per round trip; returns
 // the unnormalised sum O, its L and the reference max M.
-template <int kBatch>
+// Past the last part a slot of the batch reads this: zeros, which a weight of 0
+// cancels (a part read again, with an infinite sum, it would not).
+__device__ float g_no_record[kR * kRec];
+template <int kBatch, bool UNIFORM>
 __device__ __forceinline__ void sq_merge_parts(const SqArgs& a, int row, int d0, int p1, int p2,
                                                int s, int S, float& M, float& L, nvk_f32x4& O) {
   M = -INFINITY;
   L = 0.f;
   O = nvk_f32x4{0.f, 0.f, 0.f, 0.f};
+  const float* none = g_no_record;
+  asm("" : "+s"(none));  // read like a record: no select per element in its place
   for (int base = p1 + s; base <= p2; base += kBatch * S) {
     float mv[kBatch], lv[kBatch];
     nvk_f32x4 ov[kBatch];
@@ -544,8 +557,10 @@ __device__ __forceinline__ void sq_merge_parts(const SqArgs& a, int row, int d0,
     for (int u = 0; u < kBatch; ++u) {
       const int p = base + u * S;
       const bool ok = p <= p2;
-      const int pr = ok ? p : p1;
-      const float* rec = a.rec + (((int64_t)pr * 2 + (pr == p1 ? 0 : 1)) * a.rec_rows + row) * kRec;
+      const float* rec =
+          (ok ? a.rec + (uint32_t)((p * 2 + (p == p1 ? 0 : 1)) * rec_rows<UNIFORM>(a) * kRec)
+              : none) +
+          row * kRec;
       mv[u] = ok ? rec[HD] : -INFINITY;
       lv[u] = rec[HD + 1];
       ov[u] = *reinterpret_cast<const nvk_f32x4*>(rec + d0);
@@ -561,9 +576,7 @@ __device__ __forceinline__ void sq_merge_parts(const SqArgs& a, int row, int d0,
     for (int u = 0; u < kBatch; ++u) {
       const float wt = nvk_fast_exp2(mv[u] - mb);
       L += lv[u] * wt;
-      // past the last part: part p1 again, which 0 does not cancel if infinite
-      const nvk_f32x4 o = base + u * S <= p2 ? ov[u] : nvk_f32x4{0.f, 0.f, 0.f, 0.f};
-      O += wt * o;
+      O += wt * ov[u];
     }
     M = mb;
   }
@@ -603,11 +616,11 @@ __global__ __launch_bounds__(512) void short_query_combine_kernel(SqArgs a) {
   nvk_f32x4 O;
   const int parts = p2 - p1 + 1;
   if (parts <= 4)
-    sq_merge_parts<4>(a, row, d0, p1, p2, 0, 1, M, L, O);
+    sq_merge_parts<4, UNIFORM>(a, row, d0, p1, p2, 0, 1, M, L, O);
   else if (parts <= 8)
-    sq_merge_parts<8>(a, row, d0, p1, p2, 0, 1, M, L, O);
+    sq_merge_parts<8, UNIFORM>(a, row, d0, p1, p2, 0, 1, M, L, O);
   else
-    sq_merge_parts<16>(a, row, d0, p1, p2, 0, 1, M, L, O);
+    sq_merge_parts<16, UNIFORM>(a, row, d0, p1, p2, 0, 1, M, L, O);
   sq_write_row<F16>(op, L, O);
 }
 
@@ -621,7 +634,7 @@ constexpr int kSqSlices = 16;
 template <bool F16, bool UNIFORM>
 __global__ __launch_bounds__(64 * kSqSlices) void short_query_combine_sliced_kernel(SqArgs a) {
   const int kvh = blockIdx.x / (kR / 2), s = blockIdx.y;
-  const int lane = threadIdx.x & 63, slice = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, slice = uniform(threadIdx.x >> 6);
   int row = 2 * (blockIdx.x % (kR / 2)) + (lane >> 5);
   const int d0 = 4 * (lane & 31);
   const int Lq = seq_queries<UNIFORM>(a, s);
@@ -643,11 +656,11 @@ __global__ __launch_bounds__(64 * kSqSlices) void short_query_combine_sliced_ker
   nvk_f32x4 O;
   const int per_slice = (p2 - p1 + kSqSlices) / kSqSlices;  // ceil(parts / kSqSlices)
   if (per_slice <= 4)
-    sq_merge_parts<4>(a, row, d0, p1, p2, slice, kSqSlices, M, L, O);
+    sq_merge_parts<4, UNIFORM>(a, row, d0, p1, p2, slice, kSqSlices, M, L, O);
   else if (per_slice <= 8)
-    sq_merge_parts<8>(a, row, d0, p1, p2, slice, kSqSlices, M, L, O);
+    sq_merge_parts<8, UNIFORM>(a, row, d0, p1, p2, slice, kSqSlices, M, L, O);
   else
-    sq_merge_parts<16>(a, row, d0, p1, p2, slice, kSqSlices, M, L, O);
+    sq_merge_parts<16, UNIFORM>(a, row, d0, p1, p2, slice, kSqSlices, M, L, O);
   __shared__ float sm[kSqSlices][64], sl[kSqSlices][64];
   __shared__ nvk_f32x4 so[kSqSlices][64];
   sm[slice][lane] = M;
