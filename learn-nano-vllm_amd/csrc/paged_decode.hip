@@ -62,21 +62,22 @@ constexpr int kLoads = 8;          // load instructions per tensor per chunk
 constexpr int kWavesPerWG = 4;
 constexpr int kMaxWGs = 512;       // 256 CUs x 2 workgroups (8 waves per CU)
 constexpr int kMaxBatch = 2048;    // sequences per call (LDS prefix table)
-// Chunks a wave streams at least.  One in steps of up to 1024 chunks (a wave per
-// SIMD) whose groups are not cut into very many parts: the second chunk's page
-// id, K/V round trip and arithmetic follow the first's, ~2 us of a step that
-// takes ~10.  Two otherwise: waves that share a SIMD, uneven ranges and more
-// parts to merge take as long.  Measured on MI355X, two / one, 16/8 heads: 1 x
-// 100 keys 9.4 / 8.1 us, 1 x 1000 11.9 / 10.0, 16 x U{100..300} 12.6 / 10.6 (a
-// 28-layer graph step of one sequence 391 / 309 us).  Over 270 shapes of 1 to 12
-// sequences, 8 to 128 chunks per group and 4/2 to 16/16 heads, both forms: up to
-// 1024 chunks one gains 4.5 to 21 %; 1152 to 2048 chunks +4 to -6 % (8/4 heads, 4
-// x 2560 keys, 1280 chunks, 12.7 / 13.1; 16/8, 2 x 4096 keys with the prologue,
-// 2048 chunks, 15.2 / 16.1).  8/4 heads, 1 x 16000 (500 chunks per group) 16.9 /
-// 19.2.
+// Chunks a wave streams at least.  One in steps of about a wave per SIMD (1024)
+// whose groups are not cut into very many parts: the second chunk's page id, K/V
+// round trip and arithmetic follow the first's, ~2 us of a step that takes ~10.
+// Two otherwise: waves that share a SIMD, uneven ranges and more parts to merge
+// take as long.  Measured on MI355X, two / one, 16/8 heads: 1 x 100 keys 9.4 / 8.1
+// us, 1 x 1000 11.9 / 10.0, 16 x U{100..300} 12.6 / 10.6 (a 28-layer graph step of
+// one sequence 391 / 309 us, of three, 1048 chunks, 401 / 387).  Over 172 shapes of
+// 1 to 12 sequences, 8 to 128 chunks per group and 4/2 to 16/16 heads, with and
+// without the prologue: up to 1024 chunks one gains 4.5 to 21 %; 1152 chunks, 48
+// per group, 2.5 to 9 %, 96 per group -2 to -7 %; 1536 chunks, 16 to 32 per group,
+// -1 to -3 %, 2048 chunks -1 to -6 % (16/8, 2 x 4096 keys with the prologue 15.2 /
+// 16.1 us).  8/4 heads, 1 x 16000 keys (500 chunks per group) 16.9 / 19.2.
 constexpr int kMinChunks = 2;
-constexpr int64_t kOneChunkMax = 1024;
-constexpr int kOneChunkGroup = 128;  // chunks per group, on average
+constexpr int64_t kOneChunkMax = 1280;                  // chunks of the step where a group
+constexpr int64_t kOneChunkLong = 1024;                 // has up to kOneChunkFew on average,
+constexpr int kOneChunkFew = 64, kOneChunkGroup = 128;  // and up to kOneChunkGroup
 #ifndef NVK_DECODE_SLICE_MIN_WAVES
 #define NVK_DECODE_SLICE_MIN_WAVES 32
 #endif
@@ -134,9 +135,11 @@ __device__ __forceinline__ int clamp_ctx(const DecodeArgs& a, int b) {
 
 // Waves that take part for T chunks of `groups` groups: at most P, and few
 // enough that each range holds kMinChunks chunks (bounds how finely a context
-// is split), or one per chunk (kOneChunkMax, kOneChunkGroup).
+// is split), or one per chunk (kOneChunkMax and the others).
 __device__ __forceinline__ int64_t active_waves(int64_t T, int64_t P, int64_t groups) {
-  if (T <= P && T <= kOneChunkMax && T <= kOneChunkGroup * groups) return T < 1 ? 1 : T;
+  if (T <= P && (T <= kOneChunkFew * groups ? T <= kOneChunkMax
+                                            : T <= kOneChunkLong && T <= kOneChunkGroup * groups))
+    return T < 1 ? 1 : T;
   int64_t p = T / kMinChunks;
   if (p > P) p = P;
   return p < 1 ? 1 : p;
