@@ -14,8 +14,9 @@ normed and rotated, the rotated k and the raw v rows go straight into the
 caches.  In a decode step ``paged_decode_with_prologue`` goes one step
 further: the decode kernel itself norms and rotates q and the new k, stores
 the new k and v and attends (``nvk_paged_decode_prologue``), one launch
-fewer and q never written.  ``attention_with_prologue`` is the matching
-replacement for the body of ``Qwen3Attention.forward`` up to
+fewer and q never written (4 or 8 query heads per kv head: the prologue and the
+decode in one call, q in the output's rows).  ``attention_with_prologue`` is the
+matching replacement for the body of ``Qwen3Attention.forward`` up to
 ``self.attn(q, k, v)``: it takes the decode-step form for batches of up to
 ``FUSED_DECODE_MAX_BATCH`` sequences, and in prefill steps one call that runs
 prologue and attention (``nvk_varlen_prefill_prologue``).
@@ -136,10 +137,11 @@ def paged_decode_with_prologue(positions: torch.Tensor, qkv: torch.Tensor, num_h
                                v_cache: torch.Tensor, slot_mapping: torch.Tensor,
                                context_lens: torch.Tensor, block_tables: torch.Tensor,
                                scale: float, out: torch.Tensor | None = None) -> torch.Tensor:
-    """A decode step's prologue and attention in one decode kernel: the same
-    results, bit for bit, as ``qk_norm_rope_store(...)`` (storing the new k and
-    v at ``slot_mapping``) followed by ``paged_decode(q, k_cache, v_cache,
-    context_lens, block_tables, scale)``.  Row b of qkv is sequence b's new
+    """A decode step's prologue and attention in one call (with one or two query
+    heads per kv head in one decode kernel): the same results, bit for bit, as
+    ``qk_norm_rope_store(...)`` (storing the new k and v at ``slot_mapping``)
+    followed by ``paged_decode(q, k_cache, v_cache, context_lens, block_tables,
+    scale)``.  Row b of qkv is sequence b's new
     token; ``slot_mapping[b]`` must be the cache row of key
     ``context_lens[b] - 1`` (as model_runner.prepare_decode builds them).
     Returns [B, Hq, D] (or fills ``out``)."""
@@ -206,8 +208,9 @@ def _caches_fit(attn, dtype: torch.dtype) -> bool:
     prefill reads them.  Others take the two calls, whose checks refuse them
     (or accept them: without slots, caches of another head count)."""
     k, v = attn.k_cache, attn.v_cache
-    return (k.dim() == 4 and k.shape == v.shape and k.shape[2] == attn.num_kv_heads
-            and k.shape[3] == attn.head_dim and k.dtype == v.dtype == dtype
+    shape = k.shape
+    return (len(shape) == 4 and shape == v.shape and shape[2] == attn.num_kv_heads
+            and shape[3] == attn.head_dim and k.dtype == v.dtype == dtype
             and k.is_contiguous() and v.is_contiguous())
 
 
