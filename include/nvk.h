@@ -219,10 +219,11 @@ int nvk_paged_decode_noalloc(const void* q, int64_t q_stride_tok, int64_t q_stri
  *   and the attention kernel runs them longest first; without the workspace
  *   they run in grid order, with the same output bits.  Two calls in flight
  *   at once need two workspaces.  With a workspace of
- *   nvk_varlen_prefill_parts_workspace_size() bytes (up to 36 MB; never less
- *   than the former) longer query ranges whose tiles fill at most half of the
- *   GPU, e.g. one prompt's chunk after a long prefix, are split as well where
- *   that is faster.
+ *   nvk_varlen_prefill_parts_workspace_size() bytes (never less than the
+ *   former) longer query ranges whose tiles fill at most half of the GPU, e.g.
+ *   one prompt's chunk after a long prefix, are split as well where that is
+ *   faster: at most 512 partial results, 34.6 MB.  Ranges of at most half a query
+ *   tile (64 / G tokens) may leave up to 2046, 138.3 MB, by either size.
  * scale must be > 0.  dtype: NVK_DTYPE_BF16 or NVK_DTYPE_F16 (q, k / v and
  * out alike; f32 accumulation either way).  head_dim: 128.  G: 1, 2, 4 or 8.
  */
@@ -395,10 +396,11 @@ int nvk_qk_norm_rope_store(const void* qkv, int64_t qkv_row_stride, int64_t n_to
                            int64_t cache_slots, int32_t dtype, void* stream);
 
 /*
- * Decode step with the attention prologue applied inside the decode kernel:
- * nvk_qk_norm_rope_store followed by nvk_paged_decode for one new token per
- * sequence (qwen3.py:79-86 then attention.py:62-63 and 72-74 in a decode
- * step), without materialising q and with one launch fewer.
+ * Decode step with the attention prologue: nvk_qk_norm_rope_store followed by
+ * nvk_paged_decode for one new token per sequence (qwen3.py:79-86 then
+ * attention.py:62-63 and 72-74 in a decode step), in one call and without
+ * memory for q.  The decode kernel applies the prologue itself, with one launch
+ * fewer than the two calls (4 or 8 query heads per kv head: see below).
  * Row b of qkv is sequence b's new token (row stride qkv_row_stride, layout
  * as in nvk_qk_norm_rope_store).  q is normed and rotated at positions[b] in
  * the kernel; the new token's k (normed, rotated) and v are stored at cache
@@ -406,16 +408,17 @@ int nvk_qk_norm_rope_store(const void* qkv, int64_t qkv_row_stride, int64_t n_to
  * registers for key context_lens[b] - 1, which must be that cache row (as
  * model_runner.prepare_decode builds it: slot = the row of position
  * len - 1, context_lens = len); a sequence of context length 0 (a graph
- * padding row) stores nothing.  With 4 or 8 query heads per kv head (and, from
- * 33 sequences up, with one) the prologue runs as a kernel of its own, q passing
- * through out's rows, and key context_lens[b] - 1 is read back from the cache.
+ * padding row) stores nothing.  With 4 or 8 query heads per kv head, in pages of
+ * a multiple of 32 keys, the prologue runs as a kernel of its own, q passing
+ * through out's rows in whatever order they lie, and key context_lens[b] - 1 is
+ * read back from the cache.
  * Output, caches, block tables, context
  * lengths, workspace (nvk_paged_decode_workspace_size) and empty contexts as
  * in nvk_paged_decode; norm weights, eps, cos_sin_cache and positions as in
  * nvk_qk_norm_rope_store.  The result equals the two calls' bit for bit.
  * dtype: NVK_DTYPE_BF16 or NVK_DTYPE_F16 (qkv, weights, caches and out
  * alike).  head_dim: 128.  Two kernels are enqueued (decode with prologue,
- * combine).
+ * combine), or three (prologue, decode, combine).
  */
 int nvk_paged_decode_prologue(
     const void* qkv, int64_t qkv_row_stride, const int64_t* positions, const void* q_norm_weight,

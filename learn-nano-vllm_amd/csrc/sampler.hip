@@ -314,7 +314,7 @@ __global__ __launch_bounds__(kPartThreads) void sample_draw_kernel(SampleArgs a)
   const int first = c * kChunk + tid * 8;
   if (sizeof(T) == 2 && a.vec_ok && (int64_t)(c + 1) * kChunk <= a.vocab) {
     // a whole chunk of bf16: the kIters 16-byte loads all leave before the first
-    // wait.  Read once: non-temporal (512 rows 32.2 -> 29.3 us, 64 rows 9.8 ->
+    // wait.  Read once: non-temporal (512 rows 30.6 -> 28.1 us, 64 rows 9.8 ->
     // 8.9 against cached loads).
     const uint16_t* p = static_cast<const uint16_t*>(a.logits) + (int64_t)row * a.row_stride + first;
     nvk_u32x4 w[kIters];

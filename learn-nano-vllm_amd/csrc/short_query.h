@@ -31,8 +31,8 @@ struct ShortQueryParams {
   bool f16;  // elements are f16 (else bf16)
 };
 
-// True when the short-query kernels cover a launch of these sizes: paged keys
-// with 64-aligned pages, max_seqlen_q * G <= 16 rows, head_dim 128.
+// True when the short-query kernels cover a launch of these sizes: keys in pages
+// of a multiple of 32 keys, max_seqlen_q * G <= 16 rows, head_dim 128.
 bool short_query_applies(bool paged, int block_size, int max_seqlen_q, int num_q_heads,
                          int num_kv_heads, int head_dim, int batch);
 
@@ -49,7 +49,11 @@ bool short_query_applies(bool paged, int block_size, int max_seqlen_q, int num_q
 //     x U{100..2048} 90.2 / 87.5, 192 x U{256..4096} 485 / 479 us, and with the
 //     prologue 18.4 / 21.6, 29.3 / 31.4, 91.5 / 91.0, 491 / 483 us.
 // With the prologue (nvk_paged_decode_prologue), 16/2: 1 x 100 18.5 / 11.6,
-// 32 x U{100..2048} 42.9 / 22.3 us; 16/4: 13.2 / 12.4, 29.0 / 27.1 us.
+// 32 x U{100..2048} 42.9 / 22.3 us; 16/4: 13.2 / 12.4, 29.0 / 27.1 us, 64 x
+// U{100..2048} 37.9 / 35.6.  One or two long sequences of 4 heads are the exception
+// there (16/4, 1 x 12000 keys 18.9 / 20.0 us, 2 x U{3000..4000} 14.9-16.4 / 16.1;
+// without the prologue 18.1 / 16.9, 15.2 / 13.2): the host knows no lengths, and
+// both forms take one kernel, so that they give the same bits.
 constexpr int kDecodeKernelGroup = 2;
 bool short_query_decode_applies(int block_size, int num_blocks, int num_q_heads, int num_kv_heads,
                                 int head_dim, int batch);

@@ -1286,7 +1286,7 @@ size_t prefill_workspace_bytes(bool parts, int32_t batch, int32_t max_seqlen_q,
     split = n > split ? n : split;
   }
   // short query ranges over paged keys take the short-query kernels (pages of
-  // a multiple of 64 keys; the size does not depend on the page size)
+  // a multiple of 32 keys; the size does not depend on the page size)
   const size_t sq = short_query_applies(true, 64, max_seqlen_q, num_q_heads, num_kv_heads,
                                         head_dim, batch)
                         ? short_query_ws_bytes(batch, max_seqlen_k, num_q_heads, num_kv_heads)

@@ -15,23 +15,26 @@ pytestmark = pytest.mark.gpu
 EDGES = [1, 0, 31, 32, 33, 255, 256, 257, 0, 1500, 4097]
 
 
-@pytest.mark.parametrize("hq,hkv,ctx,bs", [
-    (16, 4, EDGES, 256),
-    (16, 2, EDGES, 32),
-    (8, 1, [9000], 256),                          # one group over many waves: sliced combine
-    (16, 2, [0, 0, 0], 256),                      # nothing to read
-    (16, 2, [300 + 7 * i for i in range(150)], 64),   # K through LDS
-    (4, 4, [1 + 37 * i for i in range(33)], 256),     # one head: the decode kernel
-    (4, 1, EDGES, 48),                            # pages of 48 keys: too
+@pytest.mark.parametrize("hq,hkv,ctx,bs,width", [
+    (16, 4, EDGES, 256, 0),
+    (16, 2, EDGES, 32, 0),
+    (8, 1, [9000], 256, 0),                       # one group over many waves: sliced combine
+    (16, 2, [0, 0, 0], 256, 0),                   # nothing to read
+    (16, 2, [300 + 7 * i for i in range(150)], 64, 0),
+    # tables that could name 32 chunks of 32 keys for each of 1024 waves: K through LDS
+    (16, 2, [300 + 7 * i for i in range(150)], 64, 56),
+    (8, 1, [0, 33, 1] + [97 * i for i in range(61)], 256, 64),
+    (4, 4, [1 + 37 * i for i in range(33)], 256, 0),     # one head: the decode kernel
+    (4, 1, EDGES, 48, 0),                         # pages of 48 keys: too
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_decode_groups_match_oracle(hq, hkv, ctx, bs, dtype):
+def test_decode_groups_match_oracle(hq, hkv, ctx, bs, width, dtype):
     pages = sum(-(-c // bs) for c in ctx)
     case = decode_case(seed=7, hq=hq, hkv=hkv, ctx=ctx, block_size=bs, pool_blocks=pages + 2,
-                       width=max(1, max(-(-c // bs) for c in ctx)))
+                       width=max(1, width, max(-(-c // bs) for c in ctx)))
     q, kc, vc = (t.to(dtype) for t in (case.q, case.k_cache, case.v_cache))
     ref = oracle_decode(q, kc, vc, case.block_tables, case.context_lens, bs, case.scale)
-    say(f"decode {hq}/{hkv} heads, {len(ctx)} sequences, page {bs}, {dtype}")
+    say(f"decode {hq}/{hkv} heads, {len(ctx)} sequences, page {bs}, width {width}, {dtype}")
     b = len(ctx)
     wide = torch.zeros(b, hq, 160, dtype=dtype, device="cuda")
     wide[..., 16:144] = q.cuda()
@@ -46,14 +49,17 @@ def test_decode_groups_match_oracle(hq, hkv, ctx, bs, dtype):
 
 
 @pytest.mark.parametrize("rows", ["contiguous", "padded", "head by head"])
-@pytest.mark.parametrize("hq,hkv,ctx", [
-    (16, 2, [1, 32, 33, 257, 0, 1700, 2900]), (16, 4, [1, 32, 33, 257, 0, 1700, 2900]),
-    (4, 4, [1, 32, 33, 257, 0, 1700, 2900] + [3 * i for i in range(30)]),   # inside the decode kernel
+@pytest.mark.parametrize("hq,hkv,ctx,width", [
+    (16, 2, [1, 32, 33, 257, 0, 1700, 2900], 12), (16, 4, [1, 32, 33, 257, 0, 1700, 2900], 12),
+    (16, 2, [1, 32, 33, 257, 0, 1700, 2900], 293),          # K through LDS
+    (8, 1, [64 * i + 31 * (i % 3) for i in range(65)], 17),  # several groups to a wave
+    (4, 4, [1, 32, 33, 257, 0, 1700, 2900] + [3 * i for i in range(30)], 12),   # the decode kernel
 ])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
-def test_prologue_form_with_q_in_the_output_rows(rows, hq, hkv, ctx, dtype):
+def test_prologue_form_with_q_in_the_output_rows(rows, hq, hkv, ctx, width, dtype):
     bs = 256
-    case = decode_case(seed=8, hq=hq, hkv=hkv, ctx=ctx, pool_blocks=60)
+    case = decode_case(seed=8, hq=hq, hkv=hkv, ctx=ctx, width=width,
+                       pool_blocks=sum(-(-c // bs) for c in ctx) + 1)
     case.k_cache, case.v_cache = case.k_cache.to(dtype), case.v_cache.to(dtype)
     g = torch.Generator().manual_seed(9)
     qkv = (torch.randn(len(ctx), (hq + 2 * hkv) * 128, generator=g) * 2).to(dtype).cuda()
@@ -84,7 +90,8 @@ def test_prologue_form_with_q_in_the_output_rows(rows, hq, hkv, ctx, dtype):
 @pytest.mark.parametrize("hq,hkv,ctx", [
     (16, 8, [1]), (16, 8, [1000]),                 # one chunk per wave
     (4, 2, [4096]), (4, 2, [4097]),                # 128 and 129 chunks per group
-    (16, 8, [2048] * 2), (16, 8, [2048] * 2 + [1]),    # 1024 chunks and more
+    (16, 8, [2048] * 2), (16, 8, [2080] * 2),          # 64 chunks per group, and more, of 1024 up
+    (16, 8, [1280] * 4), (16, 8, [1280] * 4 + [1]),    # 1280 chunks, and more
     (16, 8, [2048] * 4), (16, 8, [2048] * 4 + [1]),    # 2048 chunks (two for each wave) and more
     (16, 2, [3072] * 4), (16, 2, [3073] * 4),      # 768 chunks, and more, on the MFMA kernels
     (8, 1, [4096, 1]), (8, 1, [9000, 0, 1]),

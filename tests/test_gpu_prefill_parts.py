@@ -57,3 +57,8 @@ def test_rule_keeps_whole_tiles_where_parts_cost_more():
                  (1, 65, 1500, 1, 1, 128)]:
         need = size(*args)
         assert 0 < need <= 512 * 128 * 132 * 4 and need % (128 * 132 * 4) == 0
+    # ranges of at most half a tile keep their own plan: up to 16 parts, 1024 workgroups and more
+    plain = _lib.load().nvk_varlen_prefill_workspace_size
+    for args, records in [((64, 20, 2048, 16, 8, 128), 1024), ((127, 20, 2048, 16, 8, 128), 2032),
+                          ((1023, 8, 2048, 8, 1, 128), 2046), ((1024, 8, 2048, 8, 1, 128), 0)]:
+        assert size(*args) == plain(*args) == records * 128 * 132 * 4

@@ -297,3 +297,14 @@ def test_plain_prefill_kernels_keep_their_registers():
         at = blob.find(b"amdhsa.kernels", at + 1)
     assert len(spills) == 4 * 3 * 2         # group size, key layout, element type
     assert not {k: n for k, n in spills.items() if n and k[1] != "2"}
+
+
+def test_the_decode_workspace_holds_either_kernel():
+    """Decodes of 4 and 8 heads per kv head run on the short-query kernels in the
+    decode's workspace."""
+    lib = _lib.load()
+    for hq, hkv in [(16, 4), (16, 2), (8, 1), (32, 8), (64, 8)]:
+        for batch in (1, 2, 3, 5, 12, 33, 64, 200, 777, 2048):
+            for bs, pages in [(32, 1), (32, 7), (64, 12), (256, 1), (256, 16), (256, 160)]:
+                short = lib.nvk_paged_verify_workspace_size(batch, 1, hq, hkv, 128, bs, pages)
+                assert 0 < short <= lib.nvk_paged_decode_workspace_size(batch, hq, hkv, 128, bs, pages)
