@@ -62,26 +62,27 @@ constexpr int kLoads = 8;          // load instructions per tensor per chunk
 constexpr int kWavesPerWG = 4;
 constexpr int kMaxWGs = 512;       // 256 CUs x 2 workgroups (8 waves per CU)
 constexpr int kMaxBatch = 2048;    // sequences per call (LDS prefix table)
-// Chunks a wave streams at least.  One in steps of about a wave per SIMD (1024)
-// whose groups are not cut into very many parts: the second chunk's page id, K/V
-// round trip and arithmetic follow the first's, ~2 us of a step that takes ~10.
-// Two otherwise: waves that share a SIMD, uneven ranges and more parts to merge
-// take as long.  Measured on MI355X, two / one, 16/8 heads: 1 x 100 keys 9.4 / 8.1
-// us, 1 x 1000 11.9 / 10.0, 16 x U{100..300} 12.6 / 10.6 (a 28-layer graph step of
-// one sequence 391 / 309 us, of three, 1048 chunks, 401 / 387).  Over 172 shapes of
-// 1 to 12 sequences, 8 to 128 chunks per group and 4/2 to 16/16 heads, with and
-// without the prologue: up to 1024 chunks one gains 4.5 to 21 %; 1152 chunks, 48
-// per group, 2.5 to 9 %, 96 per group -2 to -7 %; 1536 chunks, 16 to 32 per group,
-// -1 to -3 %, 2048 chunks -1 to -6 % (16/8, 2 x 4096 keys with the prologue 15.2 /
-// 16.1 us).  8/4 heads, 1 x 16000 keys (500 chunks per group) 16.9 / 19.2.
+// Chunks a wave streams at least: one in steps of up to kOneChunkMax chunks (a
+// wave per SIMD), the second chunk's page id, K/V round trip and arithmetic
+// following the first's, ~2 us of a step that takes ~10; else two, since waves
+// that share a SIMD and uneven ranges take as long and leave more parts to merge.
+// The exceptions are groups of 33 to 64 chunks on average, where one chunk per
+// wave stays ahead in as many waves as there are, if the sliced combine folds the
+// parts, and groups of more than 128, whose parts cost more than they give.
+// Measured on MI355X, two / one, 16/8 heads: 1 x 100 keys 9.4 / 8.1 us, 1 x 1000
+// 11.9 / 10.0, 16 x U{100..300} 12.6 / 10.6; a 28-layer graph step of one sequence
+// 391 / 309 us, of three (1048 chunks, 44 per group) 401 / 387.  Over 400 shapes of
+// 1 to 20 sequences and 4/2 to 16/16 heads, with and without the prologue, one
+// gains: up to 1024 chunks 4.5 to 21 %; 1025 to 2048, 33 to 64 per group -1 to 6 %,
+// 17 to 32 -1 to -8 % (6 x 704 keys, 1056 chunks, 13.1 / 14.1), 65 to 128 -1 to -7 %
+// (2 x 4096 with the prologue 15.2 / 16.1); with the plain combine 48 groups of 33
+// take 17.1 for 15.1.  8/4 heads, 1 x 16000 keys (500 per group) 16.9 / 19.2.
 constexpr int kMinChunks = 2;
-constexpr int64_t kOneChunkMax = 1280;                  // chunks of the step where a group
-constexpr int64_t kOneChunkLong = 1024;                 // has up to kOneChunkFew on average,
-constexpr int kOneChunkFew = 64, kOneChunkGroup = 128;  // and up to kOneChunkGroup
+constexpr int64_t kOneChunkMax = 1024;
 #ifndef NVK_DECODE_SLICE_MIN_WAVES
 #define NVK_DECODE_SLICE_MIN_WAVES 32
 #endif
-constexpr int kSliceMinWaves = NVK_DECODE_SLICE_MIN_WAVES;
+constexpr int kSliceMinWaves = NVK_DECODE_SLICE_MIN_WAVES;  // waves per group: sliced combine
 
 typedef __attribute__((address_space(4))) const int32_t nvk_const_i32;
 typedef __attribute__((address_space(4))) const int64_t nvk_const_i64;
@@ -135,11 +136,11 @@ __device__ __forceinline__ int clamp_ctx(const DecodeArgs& a, int b) {
 
 // Waves that take part for T chunks of `groups` groups: at most P, and few
 // enough that each range holds kMinChunks chunks (bounds how finely a context
-// is split), or one per chunk (kOneChunkMax and the others).
+// is split), or one per chunk (see kOneChunkMax).
 __device__ __forceinline__ int64_t active_waves(int64_t T, int64_t P, int64_t groups) {
-  if (T <= P && (T <= kOneChunkFew * groups ? T <= kOneChunkMax
-                                            : T <= kOneChunkLong && T <= kOneChunkGroup * groups))
-    return T < 1 ? 1 : T;
+  const bool sliced = P >= kSliceMinWaves * groups;
+  const bool more = sliced && T > 32 * groups && T <= 64 * groups;
+  if (T <= P && (T <= kOneChunkMax || more) && T <= 128 * groups) return T < 1 ? 1 : T;
   int64_t p = T / kMinChunks;
   if (p > P) p = P;
   return p < 1 ? 1 : p;
@@ -792,13 +793,15 @@ int decode_tc(int num_kv_heads, int head_dim) {
   return kLoads * (rpi / decode_hpi(num_kv_heads, head_dim));
 }
 
-// Waves of the persistent grid for these static sizes: the most that
-// active_waves can give.  The combine's form is chosen by them.
+// Waves of the persistent grid for these static sizes: two chunks each, or one
+// where active_waves may give one (tables that name more than 32 chunks per
+// group, in grids that hold them all).  The combine's form is chosen by them.
 int decode_waves(int batch, int num_kv_heads, int head_dim, int block_size, int max_blocks) {
   const int tc = decode_tc(num_kv_heads, head_dim);
   const int64_t max_chunks_seq = ((int64_t)block_size * max_blocks + tc - 1) / tc;
   const int64_t t_max = max_chunks_seq * batch * (num_kv_heads / decode_hpi(num_kv_heads, head_dim));
-  const int64_t one = t_max < kOneChunkMax ? t_max : kOneChunkMax, two = t_max / kMinChunks;
+  const bool all = max_chunks_seq > 32 && t_max <= kMaxWGs * kWavesPerWG;
+  const int64_t one = all || t_max < kOneChunkMax ? t_max : kOneChunkMax, two = t_max / kMinChunks;
   int64_t wgs = ((one > two ? one : two) + kWavesPerWG - 1) / kWavesPerWG;
   if (wgs > kMaxWGs) wgs = kMaxWGs;
   if (wgs < 1) wgs = 1;

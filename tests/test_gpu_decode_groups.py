@@ -90,8 +90,9 @@ def test_prologue_form_with_q_in_the_output_rows(rows, hq, hkv, ctx, width, dtyp
 @pytest.mark.parametrize("hq,hkv,ctx", [
     (16, 8, [1]), (16, 8, [1000]),                 # one chunk per wave
     (4, 2, [4096]), (4, 2, [4097]),                # 128 and 129 chunks per group
-    (16, 8, [2048] * 2), (16, 8, [2080] * 2),          # 64 chunks per group, and more, of 1024 up
-    (16, 8, [1280] * 4), (16, 8, [1280] * 4 + [1]),    # 1280 chunks, and more
+    (16, 8, [2048] * 2), (16, 8, [2080] * 2),          # 1024 chunks, and 65 per group
+    (16, 8, [2048] * 3), (16, 8, [1024] * 5),          # more chunks, 64 and 32 per group
+    (16, 8, [1056] * 6), (16, 8, [1056] * 7 + [2500]),   # 33 per group: sliced merge, plain merge
     (16, 8, [2048] * 4), (16, 8, [2048] * 4 + [1]),    # 2048 chunks (two for each wave) and more
     (16, 2, [3072] * 4), (16, 2, [3073] * 4),      # 768 chunks, and more, on the MFMA kernels
     (8, 1, [4096, 1]), (8, 1, [9000, 0, 1]),
