@@ -64,21 +64,22 @@ constexpr int kMaxWGs = 512;       // 256 CUs x 2 workgroups (8 waves per CU)
 constexpr int kMaxBatch = 2048;    // sequences per call (LDS prefix table)
 // Chunks a wave streams at least: one in steps of up to kOneChunkMax chunks (a
 // wave per SIMD), the second chunk's page id, K/V round trip and arithmetic
-// following the first's, ~2 us of a step that takes ~10; else two, since waves
-// that share a SIMD and uneven ranges take as long and leave more parts to merge.
-// The exceptions are groups of 33 to 64 chunks on average, where one chunk per
-// wave stays ahead in as many waves as there are, if the sliced combine folds the
-// parts, and groups of more than 128, whose parts cost more than they give.
-// Measured on MI355X, two / one, 16/8 heads: 1 x 100 keys 9.4 / 8.1 us, 1 x 1000
-// 11.9 / 10.0, 16 x U{100..300} 12.6 / 10.6; a 28-layer graph step of one sequence
-// 391 / 309 us, of three (1048 chunks, 44 per group) 401 / 387.  Over 400 shapes of
-// 1 to 20 sequences and 4/2 to 16/16 heads, with and without the prologue, one
-// gains: up to 1024 chunks 4.5 to 21 %; 1025 to 2048, 33 to 64 per group -1 to 6 %,
-// 17 to 32 -1 to -8 % (6 x 704 keys, 1056 chunks, 13.1 / 14.1), 65 to 128 -1 to -7 %
-// (2 x 4096 with the prologue 15.2 / 16.1); with the plain combine 48 groups of 33
-// take 17.1 for 15.1.  8/4 heads, 1 x 16000 keys (500 per group) 16.9 / 19.2.
+// following the first's, ~2 us of a step that takes ~10.  Beyond, up to the 2048
+// waves of the grid, waves share a SIMD and there is more to merge, and one or two
+// depends on the chunks per group (one_chunk).  Measured on MI355X, two / one,
+// 16/8 heads: 1 x 100 keys 9.4 / 8.1 us, 1 x 1000 11.9 / 10.0, 16 x U{100..300}
+// 12.6 / 10.6; a 28-layer graph step of one sequence 391 / 309 us, of three (1048
+// chunks, 44 per group) 401 / 387.  Over 800 shapes of 1 to 600 sequences and 4/2
+// to 16/16 heads, one gains: up to 1024 chunks 4.5 to 29 %; 1025 to 2048 chunks of
+// whole pages, by chunks per group, without (with) the prologue:
+//   1 to 3: 1 to 15 % (-1 to 12; -3 to -9 where every context has two); 4: 3 to 10
+//   (-2 to 4) %; 5 to 8: 5 to -4 (1 to -5) %; 9 to 32: 5 to -8 (7 to -10) %, mostly
+//   losses; 33 to 64: 14 to -1 (9 to -2) %; 65 to 128: -1 to -5 (-1 to -6) %.
+// HD 64 0 to 21 %, but -3 to -6 % where all contexts have 2 or 8 chunks, and up to
+// -7 % at 18; pages that do not hold whole chunks, whose rows look up their pages
+// one by one, 16 to 43 %.  8/4 heads, 1 x 16000 keys (500 per group) 16.9 / 19.2 us.
 constexpr int kMinChunks = 2;
-constexpr int64_t kOneChunkMax = 1024;
+constexpr int kOneChunkMax = 1024;
 #ifndef NVK_DECODE_SLICE_MIN_WAVES
 #define NVK_DECODE_SLICE_MIN_WAVES 32
 #endif
@@ -134,13 +135,20 @@ __device__ __forceinline__ int clamp_ctx(const DecodeArgs& a, int b) {
   return ctx;
 }
 
+// Whether each of T chunks gets a wave of its own (see kOneChunkMax).
+template <int HD, bool ALIGNED, bool FUSED>
+__device__ __forceinline__ bool one_chunk(int64_t T, int P, int groups) {
+  const int g = groups < P ? groups : P;  // T <= P: more make no difference
+  if (T > P || T > 128 * g) return false;
+  if (T <= kOneChunkMax || !ALIGNED || HD == 64) return true;
+  return T <= (FUSED ? 4 : 8) * g || (T > 32 * g && T <= 64 * g);
+}
 // Waves that take part for T chunks of `groups` groups: at most P, and few
 // enough that each range holds kMinChunks chunks (bounds how finely a context
-// is split), or one per chunk (see kOneChunkMax).
-__device__ __forceinline__ int64_t active_waves(int64_t T, int64_t P, int64_t groups) {
-  const bool sliced = P >= kSliceMinWaves * groups;
-  const bool more = sliced && T > 32 * groups && T <= 64 * groups;
-  if (T <= P && (T <= kOneChunkMax || more) && T <= 128 * groups) return T < 1 ? 1 : T;
+// is split), or one per chunk.
+template <int HD, bool ALIGNED, bool FUSED>
+__device__ __forceinline__ int64_t active_waves(int64_t T, int P, int groups) {
+  if (one_chunk<HD, ALIGNED, FUSED>(T, P, groups)) return T < 1 ? 1 : T;
   int64_t p = T / kMinChunks;
   if (p > P) p = P;
   return p < 1 ? 1 : p;
@@ -526,7 +534,8 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(DecodeArgs a) {
   role.tt = g / hpi;
   const int n_blk = a.num_kv_heads / hpi;
 
-  const int S = chunk_prefix(a, s_cs, s_ctx, s_wsum);
+  // uniform: the rule and the range come out of scalar arithmetic (0.1 us a call)
+  const int S = uniform(chunk_prefix(a, s_cs, s_ctx, s_wsum));
   if (blockIdx.x == 0) {  // empty contexts: no wave visits them
     for (int e = tid; e < a.batch * n_blk; e += 256) {
       const int b = e / n_blk;
@@ -534,7 +543,7 @@ __global__ __launch_bounds__(256) void paged_decode_kernel(DecodeArgs a) {
     }
   }
   const int64_t T = (int64_t)n_blk * S;
-  const int64_t P = active_waves(T, a.n_waves, (int64_t)a.batch * n_blk);
+  const int64_t P = active_waves<HD, ALIGNED, FUSED>(T, a.n_waves, a.batch * n_blk);
   // the wave index is wave-uniform; say so, so that the range bookkeeping and
   // the page-table reads stay scalar
   const int64_t w = (int64_t)blockIdx.x * kWavesPerWG + uniform(tid >> 6);
@@ -793,16 +802,13 @@ int decode_tc(int num_kv_heads, int head_dim) {
   return kLoads * (rpi / decode_hpi(num_kv_heads, head_dim));
 }
 
-// Waves of the persistent grid for these static sizes: two chunks each, or one
-// where active_waves may give one (tables that name more than 32 chunks per
-// group, in grids that hold them all).  The combine's form is chosen by them.
+// Waves of the persistent grid for these static sizes: one per chunk that the
+// tables can name, up to the grid's largest.
 int decode_waves(int batch, int num_kv_heads, int head_dim, int block_size, int max_blocks) {
   const int tc = decode_tc(num_kv_heads, head_dim);
   const int64_t max_chunks_seq = ((int64_t)block_size * max_blocks + tc - 1) / tc;
   const int64_t t_max = max_chunks_seq * batch * (num_kv_heads / decode_hpi(num_kv_heads, head_dim));
-  const bool all = max_chunks_seq > 32 && t_max <= kMaxWGs * kWavesPerWG;
-  const int64_t one = all || t_max < kOneChunkMax ? t_max : kOneChunkMax, two = t_max / kMinChunks;
-  int64_t wgs = ((one > two ? one : two) + kWavesPerWG - 1) / kWavesPerWG;
+  int64_t wgs = (t_max + kWavesPerWG - 1) / kWavesPerWG;
   if (wgs > kMaxWGs) wgs = kMaxWGs;
   if (wgs < 1) wgs = 1;
   return (int)wgs * kWavesPerWG;
@@ -835,7 +841,7 @@ int launch_decode(const DecodeArgs& a, bool aligned, hipStream_t stream) {
   // Steps with at least NVK_DECODE_SLICE_MIN_WAVES waves per group cut
   // their groups into many parts: the sliced combine folds them.
   const int64_t groups = (int64_t)a.batch * (a.num_kv_heads / a.hpi);
-  if (a.n_waves >= (int64_t)kSliceMinWaves * groups)
+  if (a.n_waves >= kSliceMinWaves * groups)
     hipLaunchKernelGGL((paged_decode_combine_sliced_kernel<HD, G, F16>),
                        dim3(a.num_kv_heads * (G * HD / 64), a.batch), dim3(64 * kSlices), 0,
                        stream, a);

@@ -92,7 +92,8 @@ def test_prologue_form_with_q_in_the_output_rows(rows, hq, hkv, ctx, width, dtyp
     (4, 2, [4096]), (4, 2, [4097]),                # 128 and 129 chunks per group
     (16, 8, [2048] * 2), (16, 8, [2080] * 2),          # 1024 chunks, and 65 per group
     (16, 8, [2048] * 3), (16, 8, [1024] * 5),          # more chunks, 64 and 32 per group
-    (16, 8, [1056] * 6), (16, 8, [1056] * 7 + [2500]),   # 33 per group: sliced merge, plain merge
+    (16, 8, [97] * 48), (16, 8, [129] * 32),       # 4 and 5 per group
+    (16, 8, [225] * 24), (16, 8, [257] * 16), (16, 8, [1056] * 6),  # 8, 9 and 33
     (16, 8, [2048] * 4), (16, 8, [2048] * 4 + [1]),    # 2048 chunks (two for each wave) and more
     (16, 2, [3072] * 4), (16, 2, [3073] * 4),      # 768 chunks, and more, on the MFMA kernels
     (8, 1, [4096, 1]), (8, 1, [9000, 0, 1]),
